@@ -144,6 +144,19 @@ int rr_ssd_bwd_noalloc(const float* dy, const float* dfinal, const void* u, cons
                        const float* h0, const float* ckpt, void* du, void* ddelta, void* dB,
                        void* dC, float* dA_neg, int64_t dA_stride_n, float* dh0, void* stream);
 
+/* Forward without checkpoints, for calls that no backward follows (a prompt
+ * run once before decoding): arguments as rr_ssd_fwd, except that only the
+ * final state `fin` [B,H,Dh,N] is written, in the layout of h0 (replaces the
+ * same kernel, ssd.py:54-135; the reference has no such variant).  seg takes
+ * part in the shape rules only.  rr_ssd_final_workspace_bytes returns the
+ * workspace it needs, or -1 for calls that rr_ssd_fwd is to run. */
+int64_t rr_ssd_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
+                                     int64_t A_stride_n, int dtype);
+int rr_ssd_final_fwd(const void* u, const void* delta, const void* Bm, const void* Cm,
+                     const float* A_neg, int64_t A_stride_n, int dtype, int64_t B, int64_t L, int64_t H,
+                     int64_t Dh, int64_t N, int64_t seg, const float* h0, float* y, float* fin,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------ GLA --
  * q/k/v [B,L,H,Dh], gates [B,L,H] (dtype).  y [B,L,H,Dh] fp32.
  * ckpt [B,H,nC,Dh(j),Dh(i)] fp32: state S[i,j] stored with i fastest, so
@@ -170,6 +183,13 @@ int rr_gla_bwd(const float* dy, const float* dfinal, const void* q, const void* 
                int64_t H, int64_t Dh, int64_t seg, const float* h0, const float* ckpt,
                void* dq, void* dk, void* dv, void* dgates, float* dh0, void* workspace,
                size_t workspace_bytes, void* stream);
+
+/* The GLA forward without checkpoints (see rr_ssd_final_fwd): fin
+ * [B,H,Dh(i),Dh(j)], the layout of h0. */
+int64_t rr_gla_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t seg, int dtype);
+int rr_gla_final_fwd(const void* q, const void* k, const void* v, const void* gates, int dtype,
+                     int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t seg, const float* h0,
+                     float* y, float* fin, void* workspace, size_t workspace_bytes, void* stream);
 
 /* --------------------------------------------------------------- RG-LRU --
  * a, x [B,L,D] (dtype).  y [B,L,D] fp32.  ckpt [B,nC,D] fp32.

@@ -1,0 +1,617 @@
+// final_fwd.hip — SSD (one decay rate per head) and GLA forward for calls that
+// need y and the final state only (no gradient, so no checkpoints): bf16
+// inputs of any length L >= 1.
+//
+// Per (batch, head) the recurrence and its 32-step chunk form are those of
+// rr_chunked.h,
+//     Y     = (M o C B^T o w_s) U + diag(gam) C h_in^T
+//     h_end = gam_31 h_in + (diag(m31 o w) U)^T B,
+// with the last chunk's missing steps taken as identity steps (zero rows, no
+// decay).  A workgroup owns a head and walks its chunks; each wave owns 16 DB
+// rows d of the state for all n and never exchanges anything with the others:
+// the state lives in accumulators as h^T[n][d] (rows n), which are, element
+// for element, the B operand of C h^T, and (C B^T)^T's accumulators (rows s)
+// are the A operand of W U, so neither passes through LDS.  The k index of
+// those products runs in the accumulators' order pi(g, e) = 4 g + e (e < 4),
+// 16 + 4 g + e - 4 (e >= 4); B and C are staged in LDS with their n index in
+// that order, and read back as row fragments (16 bytes) or transposed.
+//
+// fp32 factors (the state, W, the weighted U) are split into three bf16 terms,
+// hi + mid + lo = all 24 bits, each multiplied with an exact bf16 operand, and
+// the small terms are summed first: the error against float64 stays that of
+// fp32 arithmetic (1e-7; the two-term split of the training kernels has
+// 2.5e-6).
+//
+// Heads alone may not fill the GPU: the chunks are then cut into S segments.
+// A first launch forms every segment's map (its state from a zero start and
+// its decay), and the walk of segment j starts from h0 carried through the
+// maps of segments 0 .. j - 1.
+//
+// What bounds it: the instructions of a chunk (per wave about 700 VALU, a
+// third of them the three-term splits, beside 66 MFMAs at N = 128) on two
+// waves per SIMD, not memory: B4 L1000 H80 Dh64 N128 takes 132 us, 2.3 TB/s of
+// the 0.31 GB it cannot do without (6.1 ms on the VALU engine, which forms and
+// stores a state every 8 steps there); B8 L4096 H80 895 us where the training
+// forward with its 2.7 GB of checkpoints takes 1227.
+#include "rr_chunked.h"
+
+namespace {
+
+using rr::f32x4_t;
+using rr::u16x4_t;
+using rr::u16x8_t;
+
+constexpr int Q = 32;
+
+struct FinalArgs {
+  const uint16_t* u;      // [B,L,H,DH] (GLA: v)
+  const uint16_t* step;   // [B,L,H] delta (GLA: gates)
+  const uint16_t* Bm;     // [B,L,H,N] (GLA: k)
+  const uint16_t* Cm;     // [B,L,H,N] (GLA: q)
+  const float* A;         // [H] (SSD)
+  const float* h0;        // [B,H,DH,N] as d, n (GLA [B,H,N,DH] as n, d), or null
+  float* y;               // [B,L,H,DH]
+  float* fin;             // layout of h0
+  float4* segE;           // [B*H][S-1] segment states in fragment order
+  float* segP;            // [B*H][S-1] segment decays
+  int L, H, nC, S, cps;   // chunks, segments, chunks per segment
+};
+
+// fp32 -> bf16 hi + mid + lo of eight values
+__device__ __forceinline__ void split3(const float (&x)[8], u16x8_t& hi, u16x8_t& mid, u16x8_t& lo) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    h[i] = rr::bf_pack2(x[2 * i], x[2 * i + 1]);
+    const float a = x[2 * i] - __uint_as_float(h[i] << 16), b = x[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u);
+    m[i] = rr::bf_pack2(a, b);
+    l[i] = rr::bf_pack2(a - __uint_as_float(m[i] << 16), b - __uint_as_float(m[i] & 0xffff0000u));
+  }
+  hi = __builtin_bit_cast(u16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
+  mid = __builtin_bit_cast(u16x8_t, make_uint4(m[0], m[1], m[2], m[3]));
+  lo = __builtin_bit_cast(u16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// Workgroup barrier ordering LDS only: loads and stores to memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// LDS images of one chunk.  16-byte units of a row are permuted by row (xor)
+// so that both the row fragments (16 rows, one unit) and the transposing reads
+// (4 rows x 4 units) of a 16-lane group hit distinct banks.
+template <int NSP>
+__device__ __forceinline__ int swz_n(int row) {
+  return NSP == 128 ? ((row & 3) << 2) | ((row >> 2) & 3)
+         : NSP == 64 ? (((row >> 1) & 1) << 2) | ((row >> 2) & 3)
+                     : (row >> 2) & 3;
+}
+template <int DH>
+__device__ __forceinline__ int swz_d(int row) {
+  return DH == 128 ? 2 * (row & 7) : DH == 64 ? 2 * ((row >> 1) & 3) : 2 * ((row >> 2) & 1);
+}
+
+template <int DH, int NS, int DB>
+struct alignas(16) FinalSm {
+  static constexpr int NSP = NS < 32 ? 32 : NS, NW = DH / (16 * DB);
+  uint16_t B[2][Q * NSP], C[2][Q * NSP], U[2][Q * DH];
+  float sc[2][NW][4][Q];   // per wave: gam, m31 w, cd (GLA: gates), w
+};
+
+// The 12 decays M[t][s] of a lane: t = 16 tb + l15; m0[e]: tb 0, s = 4 g + e;
+// m1[e]: tb 1, s = 4 g + e; m1[4 + e]: tb 1, s = 16 + 4 g + e; zero for s > t.
+template <bool GLA>
+__device__ __forceinline__ void decays(const float* st, float a, int l15, int g, float (&m0)[4], float (&m1)[8]) {
+  const float4 s0 = *reinterpret_cast<const float4*>(&st[4 * g]);
+  const float4 s1 = *reinterpret_cast<const float4*>(&st[16 + 4 * g]);
+  const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  if constexpr (!GLA) {
+    const float c0 = st[l15], c1 = st[16 + l15];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      m0[e] = rr::chunked::masked_exp(4 * g + e <= l15, a * (c0 - sv[e]));
+      m1[e] = __expf(a * (c1 - sv[e]));
+      m1[4 + e] = rr::chunked::masked_exp(4 * g + e <= l15, a * (c1 - sv[4 + e]));
+    }
+  } else {
+    // products of the gates of steps s + 1 .. t, by quads of steps: the rest
+    // of s's quad, whole quads between, t's quad up to t (any sign, zeros exact)
+    float qd[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 q = *reinterpret_cast<const float4*>(&st[4 * j]);
+      qd[j] = (q.x * q.y) * (q.z * q.w);
+    }
+    const int qt = l15 >> 2, pt = l15 & 3;   // t's quad within its 16 steps, position in it
+    const float4 t0 = *reinterpret_cast<const float4*>(&st[4 * qt]);
+    const float4 t1 = *reinterpret_cast<const float4*>(&st[16 + 4 * qt]);
+    auto upto = [&](const float4& q) {
+      const float p1 = q.x * q.y, p2 = p1 * q.z, p3 = p2 * q.w;
+      return pt == 0 ? q.x : pt == 1 ? p1 : pt == 2 ? p2 : p3;
+    };
+    const float h0 = upto(t0), h1 = upto(t1);
+    // whole quads strictly between g and qt (both in 0 .. 3: quads 1 and 2)
+    const bool b1 = g < 1 && qt > 1, b2 = g < 2 && qt > 2;
+    const float mid0 = (b1 ? qd[1] : 1.f) * (b2 ? qd[2] : 1.f);
+    const float mid1 = (b1 ? qd[5] : 1.f) * (b2 ? qd[6] : 1.f);
+    float midx = (g < 1 ? qd[1] : 1.f) * (g < 2 ? qd[2] : 1.f) * (g < 3 ? qd[3] : 1.f);
+    midx *= (qt > 0 ? qd[4] : 1.f) * (qt > 1 ? qd[5] : 1.f) * (qt > 2 ? qd[6] : 1.f);
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      const float* q = sv + 4 * hb;
+      const float r2 = q[3], r1 = q[2] * r2, r0 = q[1] * r1;   // rest of the quad after s
+      const float rest[4] = {r0, r1, r2, 1.f};
+      // t in s's own quad: product of positions e + 1 .. pt
+      const float yz = q[1] * q[2];
+      const float in0 = pt == 0 ? 1.f : pt == 1 ? q[1] : pt == 2 ? yz : yz * q[3];
+      const float in1 = pt == 1 ? 1.f : pt == 2 ? q[2] : q[2] * q[3];
+      const float in2 = pt == 2 ? 1.f : q[3];
+      const float inq[4] = {in0, in1, in2, 1.f};
+      const float far = (hb ? mid1 : mid0) * (hb ? h1 : h0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = qt == g ? inq[e] : rest[e] * far;
+        const float keep = 4 * g + e <= l15 ? v : 0.f;
+        if (hb) m1[4 + e] = keep;
+        else {
+          m0[e] = keep;
+          m1[e] = rest[e] * midx * h1;
+        }
+      }
+    }
+  }
+}
+
+// AGG: only the segment's state from a zero start and its decay (segE, segP).
+template <int DH, int NS, bool GLA, int DB, bool AGG>
+__global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) {
+  using S = FinalSm<DH, NS, DB>;
+  constexpr int NSP = S::NSP, NW = S::NW, T = 64 * NW, NK = NSP / 32, NBN = NSP / 16;
+  constexpr int BV = (Q * NS / 8 + T - 1) / T, UV = (Q * DH / 8 + T - 1) / T;
+  __shared__ S sm;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, g = lane >> 4;
+  const int bh = blockIdx.x, seg = blockIdx.y, h = bh % p.H, b = bh / p.H;
+  const int c0 = seg * p.cps, c1 = min(c0 + p.cps, p.nC);
+  const float a = GLA ? 0.f : p.A[h];
+  const int64_t rows = (int64_t)b * p.L;
+  const uint32_t rsN = (uint32_t)p.H * NS, rsD = (uint32_t)p.H * DH;
+
+  if constexpr (NS < 32) {   // n 16 .. 31 of both images stay zero
+    for (int i = tid; i < 2 * Q * NSP / 2; i += T) {
+      reinterpret_cast<uint32_t*>(&sm.B[0][0])[i] = 0;
+      reinterpret_cast<uint32_t*>(&sm.C[0][0])[i] = 0;
+    }
+    lds_barrier();
+  }
+
+  u16x8_t bv[BV], cv[BV], uv[UV];
+  float xv;
+  // chunk c's pieces into registers: unconditional loads, offsets past the
+  // sequence clamped to its last piece (those rows become zero, or the neutral
+  // step, when staged)
+  auto load = [&](int c) {
+    const int t0 = min(c, p.nC - 1) * Q, last = p.L - 1 - t0;
+    const uint32_t lastN = (uint32_t)min(last, Q) * rsN + NS - 8, lastD = (uint32_t)min(last, Q) * rsD + DH - 8;
+    const uint16_t* Bp = p.Bm + ((rows + t0) * p.H + h) * NS;
+    const uint16_t* Cp = p.Cm + ((rows + t0) * p.H + h) * NS;
+    const uint16_t* Up = p.u + ((rows + t0) * p.H + h) * DH;
+#pragma unroll
+    for (int v = 0; v < BV; ++v) {
+      const int i = min(tid + T * v, Q * NS / 8 - 1);
+      const uint32_t o = min((uint32_t)(i / (NS / 8)) * rsN + 8 * (i % (NS / 8)), lastN);
+      bv[v] = rr::ld32<u16x8_t>(Bp, o);
+      if constexpr (!AGG) cv[v] = rr::ld32<u16x8_t>(Cp, o);
+    }
+#pragma unroll
+    for (int v = 0; v < UV; ++v) {
+      const int i = min(tid + T * v, Q * DH / 8 - 1);
+      uv[v] = rr::ld32<u16x8_t>(Up, min((uint32_t)(i / (DH / 8)) * rsD + 8 * (i % (DH / 8)), lastD));
+    }
+    xv = rr::bf_val(p.step[(rows + t0 + min(lane & (Q - 1), last)) * p.H + h]);
+  };
+  auto stage_rows = [&](int V, int buf, auto full) {   // full: all 32 steps present
+#pragma unroll
+    for (int v = 0; v < BV; ++v) {
+      const int i = tid + T * v, t = i / (NS / 8), m = i % (NS / 8);
+      if (Q * NS / 8 % T != 0 && i >= Q * NS / 8) break;
+      const bool in = decltype(full)::value || t < V;
+      const int f = swz_n<NSP>(t), un = 4 * (m >> 2) + 2 * (m & 1), hf = 4 * ((m >> 1) & 1);
+      const uint4 x = __builtin_bit_cast(uint4, bv[v]);
+      uint16_t* d = &sm.B[buf][t * NSP + hf];
+      *reinterpret_cast<uint2*>(d + 8 * (un ^ f)) = in ? make_uint2(x.x, x.y) : make_uint2(0, 0);
+      *reinterpret_cast<uint2*>(d + 8 * ((un + 1) ^ f)) = in ? make_uint2(x.z, x.w) : make_uint2(0, 0);
+      if constexpr (!AGG) {
+        const uint4 z = __builtin_bit_cast(uint4, cv[v]);
+        d = &sm.C[buf][t * NSP + hf];
+        *reinterpret_cast<uint2*>(d + 8 * (un ^ f)) = in ? make_uint2(z.x, z.y) : make_uint2(0, 0);
+        *reinterpret_cast<uint2*>(d + 8 * ((un + 1) ^ f)) = in ? make_uint2(z.z, z.w) : make_uint2(0, 0);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < UV; ++v) {
+      const int i = tid + T * v, t = i / (DH / 8), m = i % (DH / 8);
+      if (Q * DH / 8 % T != 0 && i >= Q * DH / 8) break;
+      *reinterpret_cast<u16x8_t*>(&sm.U[buf][t * DH + 8 * (m ^ swz_d<DH>(t))]) =
+          decltype(full)::value || t < V ? uv[v] : u16x8_t{};
+    }
+  };
+  auto stage = [&](int c, int buf) {
+    const int V = p.L - c * Q;   // steps present
+    if (V >= Q) stage_rows(V, buf, std::true_type{});
+    else stage_rows(V, buf, std::false_type{});
+    const bool live = lane < V;
+    const float x = live ? xv : (GLA ? 1.f : 0.f);
+    const rr::chunked::StepScalars sc = rr::chunked::step_scalars<GLA>(lane < Q ? x : (GLA ? 1.f : 0.f), a, lane);
+    if (lane < Q) {
+      sm.sc[buf][w][0][lane] = sc.gam;
+      sm.sc[buf][w][1][lane] = sc.m31 * sc.w;
+      sm.sc[buf][w][2][lane] = GLA ? x : sc.cd;
+      sm.sc[buf][w][3][lane] = sc.w;
+    }
+  };
+
+  f32x4_t hs[DB][NBN];   // h^T[16 nb + 4 g + r][d = 16 (w DB + i) + l15]
+  float decay = 1.f;     // AGG: the segment's decay
+#pragma unroll
+  for (int i = 0; i < DB; ++i)
+#pragma unroll
+    for (int nb = 0; nb < NBN; ++nb) hs[i][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  load(c0);
+  if constexpr (!AGG) {
+    if (p.h0 != nullptr) {
+      const float* hp = p.h0 + (int64_t)bh * DH * NS;
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NS / 16; ++nb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            hs[i][nb][r] = hp[rr::chunked::state_off<GLA, DH, NS>(16 * (w * DB + i) + l15, 16 * nb + 4 * g + r)];
+    }
+    const float4* E = p.segE + (int64_t)bh * (p.S - 1) * (DB * NBN * T) + tid;
+    for (int j = 0; j < seg; ++j) {
+      const float P = p.segP[bh * (p.S - 1) + j];
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NBN; ++nb) {
+          const float4 e = E[(j * DB * NBN + i * NBN + nb) * T];
+          hs[i][nb] = f32x4_t{P * hs[i][nb][0] + e.x, P * hs[i][nb][1] + e.y, P * hs[i][nb][2] + e.z,
+                              P * hs[i][nb][3] + e.w};
+        }
+    }
+  }
+  stage(c0, 0);
+  load(c0 + 1);
+  lds_barrier();
+
+  for (int c = c0; c < c1; ++c) {
+    const int buf = (c - c0) & 1;
+    if (c + 1 < c1) {
+      stage(c + 1, buf ^ 1);
+      load(c + 2);
+    }
+    const uint16_t *Bs = sm.B[buf], *Cs = sm.C[buf], *Us = sm.U[buf];
+    const float(*sc)[Q] = sm.sc[buf][w];
+    const float tot = sc[0][Q - 1];
+    // U as B operand: U[pi(g, e)][d]
+    u16x8_t uf[DB];
+    {
+      const int r0 = 4 * g + (l15 >> 2), q = l15 & 3;
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        const uint16_t* up = Us + r0 * DH + 8 * ((2 * (w * DB + i) + (q >> 1)) ^ swz_d<DH>(r0)) + 4 * (q & 1);
+        const u16x4_t lo = rr::tr_read4(up), hi = rr::tr_read4(up + 16 * DH);
+        uf[i] = u16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    }
+    if constexpr (!AGG) {
+      u16x8_t cf[2][NK];   // C[16 tb + l15][32 kk + pi]
+      f32x4_t d00 = {0.f, 0.f, 0.f, 0.f}, d01 = d00, d11 = d00;   // (C B^T)^T blocks [s][t]
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) {
+        const int off = l15 * NSP + 8 * ((4 * kk + g) ^ swz_n<NSP>(l15));
+        const u16x8_t b0 = rr::frag(Bs + off), b1 = rr::frag(Bs + off + 16 * NSP);
+        cf[0][kk] = rr::frag(Cs + off);
+        cf[1][kk] = rr::frag(Cs + off + 16 * NSP);
+        d00 = rr::mfma16(b0, cf[0][kk], d00);
+        d01 = rr::mfma16(b0, cf[1][kk], d01);
+        d11 = rr::mfma16(b1, cf[1][kk], d11);
+      }
+      float w0[8], w1[8];   // W[l15][pi], W[16 + l15][pi]
+      {
+        float m0[4], m1[8];
+        decays<GLA>(sc[2], a, l15, g, m0, m1);
+        const float4 x0 = *reinterpret_cast<const float4*>(&sc[3][4 * g]);
+        const float4 x1 = *reinterpret_cast<const float4*>(&sc[3][16 + 4 * g]);
+        const float wl[4] = {x0.x, x0.y, x0.z, x0.w}, wh[4] = {x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool low = 4 * g + e <= l15;   // a select, so that a non-finite B row stays out of earlier steps
+          w0[e] = low ? m0[e] * (d00[e] * wl[e]) : 0.f;
+          w0[4 + e] = 0.f;
+          w1[e] = m1[e] * (d01[e] * wl[e]);
+          w1[4 + e] = low ? m1[4 + e] * (d11[e] * wh[e]) : 0.f;
+        }
+      }
+      u16x8_t wf[2][3];
+      split3(w0, wf[0][0], wf[0][1], wf[0][2]);
+      split3(w1, wf[1][0], wf[1][1], wf[1][2]);
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        f32x4_t ab[2], as[2];   // C h^T: hi terms, mid + lo terms
+        ab[0] = ab[1] = as[0] = as[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+          const float x[8] = {hs[i][2 * kk][0],     hs[i][2 * kk][1],     hs[i][2 * kk][2],     hs[i][2 * kk][3],
+                              hs[i][2 * kk + 1][0], hs[i][2 * kk + 1][1], hs[i][2 * kk + 1][2], hs[i][2 * kk + 1][3]};
+          u16x8_t hh, hm, hl;
+          split3(x, hh, hm, hl);
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb) {
+            as[tb] = rr::mfma16(cf[tb][kk], hl, as[tb]);
+            ab[tb] = rr::mfma16(cf[tb][kk], hh, ab[tb]);
+            as[tb] = rr::mfma16(cf[tb][kk], hm, as[tb]);
+          }
+        }
+        // a non-finite u must not reach the steps before it through W's zeros:
+        // such elements leave the product and are added step by step below
+        u16x8_t ui = uf[i];
+        bool odd = false;
+        {
+          uint4 x = __builtin_bit_cast(uint4, ui);
+          auto over = [](uint32_t v) { return ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u; };
+          odd = (over(x.x) | over(x.y) | over(x.z) | over(x.w)) != 0;
+        }
+        const bool any_odd = __any(odd);
+        if (any_odd) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ui[e] = (ui[e] & 0x7f80) == 0x7f80 ? 0 : ui[e];
+        }
+        f32x4_t o[2];
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+          f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          z = rr::mfma16(wf[tb][2], ui, z);
+          z = rr::mfma16(wf[tb][1], ui, z);
+          const float4 gm = *reinterpret_cast<const float4*>(&sc[0][16 * tb + 4 * g]);
+          z = f32x4_t{gm.x * (ab[tb][0] + as[tb][0]) + z[0], gm.y * (ab[tb][1] + as[tb][1]) + z[1],
+                      gm.z * (ab[tb][2] + as[tb][2]) + z[2], gm.w * (ab[tb][3] + as[tb][3]) + z[3]};
+          o[tb] = rr::mfma16(wf[tb][0], ui, z);
+        }
+        if (any_odd) {
+          for (int s = 0; s < Q; ++s) {
+            const int src = 16 * ((s >> 2) & 3), e = (s & 3) + 4 * (s >> 4);
+            float us = 0.f, ws0 = 0.f, ws1 = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              us = k == e ? rr::bf_val(uf[i][k]) : us;
+              ws0 = k == e ? rr::bf_val(wf[0][0][k]) + rr::bf_val(wf[0][1][k]) : ws0;
+              ws1 = k == e ? rr::bf_val(wf[1][0][k]) + rr::bf_val(wf[1][1][k]) : ws1;
+            }
+            us = __shfl(us, src + l15);
+            const bool add = !(fabsf(us) < __builtin_inff());   // the elements left out above
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float v0 = __shfl(ws0, src + 4 * g + r), v1 = __shfl(ws1, src + 4 * g + r);
+              if (add && s <= 4 * g + r) o[0][r] += v0 * us;
+              if (add && s <= 16 + 4 * g + r) o[1][r] += v1 * us;
+            }
+          }
+        }
+        const int V = p.L - c * Q;
+        float* yp = p.y + ((rows + (int64_t)c * Q) * p.H + h) * DH + 16 * (w * DB + i);
+        auto put = [&](int tb, int r) {
+          const uint32_t off = (uint32_t)(16 * tb + 4 * g + r) * rsD + l15;
+          *reinterpret_cast<float*>(reinterpret_cast<char*>(yp) + off * 4u) = o[tb][r];
+        };
+        if (V >= Q) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) put(j >> 2, j & 3);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (16 * (j >> 2) + 4 * g + (j & 3) < V) put(j >> 2, j & 3);
+        }
+      }
+    }
+    // h^T <- gam_31 h^T + B^T (m31 w o U): B^T transposed reads are the exact A operand
+    u16x8_t us[DB][3];
+    {
+      const float4 x0 = *reinterpret_cast<const float4*>(&sc[1][4 * g]);
+      const float4 x1 = *reinterpret_cast<const float4*>(&sc[1][16 + 4 * g]);
+      const float mw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = mw[e] * rr::bf_val(uf[i][e]);
+        split3(x, us[i][0], us[i][1], us[i][2]);
+      }
+    }
+    {
+      const int r0 = 4 * g + (l15 >> 2), f = swz_n<NSP>(r0);
+#pragma unroll
+      for (int nb = 0; nb < NBN; ++nb) {
+        const uint16_t* bp = Bs + r0 * NSP + 8 * ((4 * (nb >> 1) + (l15 & 3)) ^ f) + 4 * (nb & 1);
+        const u16x4_t lo = rr::tr_read4(bp), hi = rr::tr_read4(bp + 16 * NSP);
+        const u16x8_t bt = u16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+        for (int i = 0; i < DB; ++i) {
+          f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          z = rr::mfma16(bt, us[i][2], z);
+          z = rr::mfma16(bt, us[i][1], z);
+          z = rr::mfma16(bt, us[i][0], z);
+          hs[i][nb] = f32x4_t{tot * hs[i][nb][0] + z[0], tot * hs[i][nb][1] + z[1], tot * hs[i][nb][2] + z[2],
+                              tot * hs[i][nb][3] + z[3]};
+        }
+      }
+    }
+    if constexpr (AGG) decay *= tot;
+    lds_barrier();
+  }
+
+  if constexpr (AGG) {
+    float4* E = p.segE + ((int64_t)bh * (p.S - 1) + seg) * (DB * NBN * T) + tid;
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NBN; ++nb)
+        E[(i * NBN + nb) * T] = make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
+    if (tid == 0) p.segP[bh * (p.S - 1) + seg] = decay;
+  } else if (seg == p.S - 1) {
+    float* fp = p.fin + (int64_t)bh * DH * NS;
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NS / 16; ++nb) {
+        const int d = 16 * (w * DB + i) + l15, n = 16 * nb + 4 * g;
+        if constexpr (GLA) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) fp[(n + r) * DH + d] = hs[i][nb][r];
+        } else {
+          *reinterpret_cast<float4*>(fp + d * NS + n) =
+              make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
+        }
+      }
+  }
+}
+
+// ------------------------------------------------------------------ host
+bool covered(int64_t Dh, int64_t N, bool gla) {
+  if (gla) return Dh == N && (Dh == 32 || Dh == 64 || Dh == 128);
+  return (Dh == 32 || Dh == 64 || Dh == 128) && (N == 16 || N == 32 || N == 64 || N == 128);
+}
+
+// Segments: enough workgroups for two waves per SIMD, at least four chunks each.
+void segments(int64_t BH, int64_t nC, int64_t Dh, int& S, int& cps) {
+  const int64_t waves = BH * (Dh / 16), want = std::max<int64_t>(1, 2048 / std::max<int64_t>(waves, 1));
+  int64_t s = std::min(std::min<int64_t>(want, nC / 4), (int64_t)32);
+  s = std::max<int64_t>(s, 1);
+  cps = (int)((nC + s - 1) / s);
+  S = (int)((nC + cps - 1) / cps);
+}
+
+size_t ws_bytes(int64_t BH, int64_t Dh, int64_t N, int S) {
+  if (S <= 1) return 0;
+  const size_t state = (size_t)Dh * (size_t)std::max<int64_t>(N, 32) * 4;
+  return (size_t)BH * (S - 1) * (state + 4) + 256;
+}
+
+template <int DH, int NS, bool GLA>
+int launch(const FinalArgs& p, int64_t BH, hipStream_t s) {
+  constexpr int T = 4 * DH;
+  if (p.S > 1) {
+    hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, true>), dim3((unsigned)BH, p.S - 1), dim3(T), 0, s, p);
+    if (int rc = rr::check_launch("final-state forward (segment maps)")) return rc;
+  }
+  hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, false>), dim3((unsigned)BH, p.S), dim3(T), 0, s, p);
+  return rr::check_launch("final-state forward");
+}
+
+template <bool GLA>
+int run(FinalArgs& p, int64_t B, int64_t H, int64_t Dh, int64_t N, void* ws, size_t wsb, hipStream_t s) {
+  const int64_t BH = B * H;
+  segments(BH, p.nC, Dh, p.S, p.cps);
+  const size_t need = ws_bytes(BH, Dh, N, p.S);
+  if (need > 0) {
+    if (ws == nullptr || wsb < need) return rr::fail(RR_EWORKSPACE, "final-state forward: workspace too small");
+    p.segE = static_cast<float4*>(ws);
+    p.segP = reinterpret_cast<float*>(static_cast<char*>(ws) + (size_t)BH * (p.S - 1) * Dh * std::max<int64_t>(N, 32) * 4);
+  }
+#define RR_CASE(D, NN) \
+  if (Dh == D && N == NN) return launch<D, NN, GLA>(p, BH, s)
+  if constexpr (GLA) {
+    RR_CASE(32, 32);
+    RR_CASE(64, 64);
+    RR_CASE(128, 128);
+  } else {
+    RR_CASE(32, 16); RR_CASE(32, 32); RR_CASE(32, 64); RR_CASE(32, 128);
+    RR_CASE(64, 16); RR_CASE(64, 32); RR_CASE(64, 64); RR_CASE(64, 128);
+    RR_CASE(128, 16); RR_CASE(128, 32); RR_CASE(128, 64); RR_CASE(128, 128);
+  }
+#undef RR_CASE
+  return rr::fail(RR_EUNSUPPORTED, "final-state forward: sizes not covered");
+}
+
+bool sizes_ok(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N) {
+  if (B <= 0 || L <= 0 || H <= 0 || Dh <= 0 || N <= 0) return false;
+  // 1-D grid of heads; 32-bit byte offsets within a chunk; int step counts
+  return B <= 0x7fffffff && H <= 0x7fffffff && B * H < (int64_t(1) << 31) && L < (int64_t(1) << 30) &&
+         H * std::max(Dh, N) * Q * 4 < (int64_t(1) << 31);
+}
+
+// Which calls run here.  Where seg leaves a checkpoint interval T below 32 the
+// other forward is the VALU engine: every covered size (bf16 prompts of odd
+// length: 2.8x at B1 L40 H8, 43x at B4 L1000 H80 Dh64 N128).  At T = 32 it is
+// the training forward with its checkpoints, which has more parallelism for
+// short prompts (resident / direct kernels, one workgroup per chunk) and less
+// work per chunk at N = 16: this kernel from 17 chunks with N >= 64 (24 with
+// N = 32), where it measured 1.08x (GLA B8 L768 H80 Dh64, 166 -> 154 us) to
+// 2.5x (SSD B4 L2048 H24 Dh64 N128, 193 -> 76 us); below that 0.6x to 1.1x
+// (SSD B3 L512 H12 Dh64 N16 9.7 -> 15.1 us), at N = 16 0.83x to 1.22x.
+int64_t query(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg, int dtype, bool gla) {
+  if (dtype != RR_BF16 || !sizes_ok(B, L, H, Dh, N) || !covered(Dh, N, gla)) return -1;
+  const int64_t nC = (L + Q - 1) / Q;
+  if (rr::chunk_len(L, seg) == Q && !(N >= 64 ? nC > 16 : N == 32 && nC >= 24)) return -1;
+  int S, cps;
+  segments(B * H, nC, Dh, S, cps);
+  return (int64_t)ws_bytes(B * H, Dh, N, S);
+}
+
+}  // namespace
+
+extern "C" int64_t rr_ssd_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
+                                                int64_t A_stride_n, int dtype) {
+  if (rr::chunk_len(L, seg) == 0 || A_stride_n != 0) return -1;
+  return query(B, L, H, Dh, N, seg, dtype, false);
+}
+
+extern "C" int rr_ssd_final_fwd(const void* u, const void* delta, const void* Bm, const void* Cm, const float* A_neg,
+                                int64_t A_stride_n, int dtype, int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N,
+                                int64_t seg, const float* h0, float* y, float* fin, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  if (int rc = rr::check_segment_shape(L, seg, Dh, "Dh")) return rc;
+  if (!u || !delta || !Bm || !Cm || !A_neg || !y || !fin)
+    return rr::fail(RR_EINVAL, "ssd_final_fwd: null pointer argument");
+  if (rr_ssd_final_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype) < 0)
+    return rr::fail(RR_EUNSUPPORTED, "ssd_final_fwd: call not covered (rr_ssd_final_workspace_bytes is -1)");
+  FinalArgs p{};
+  p.u = static_cast<const uint16_t*>(u);
+  p.step = static_cast<const uint16_t*>(delta);
+  p.Bm = static_cast<const uint16_t*>(Bm);
+  p.Cm = static_cast<const uint16_t*>(Cm);
+  p.A = A_neg;
+  p.h0 = h0;
+  p.y = y;
+  p.fin = fin;
+  p.L = (int)L; p.H = (int)H; p.nC = (int)((L + Q - 1) / Q);
+  return run<false>(p, B, H, Dh, N, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t rr_gla_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t seg, int dtype) {
+  if (rr::chunk_len(L, seg) == 0) return -1;
+  return query(B, L, H, Dh, Dh, seg, dtype, true);
+}
+
+extern "C" int rr_gla_final_fwd(const void* q, const void* k, const void* v, const void* gates, int dtype, int64_t B,
+                                int64_t L, int64_t H, int64_t Dh, int64_t seg, const float* h0, float* y, float* fin,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = rr::check_segment_shape(L, seg, Dh, "Dh")) return rc;
+  if (!q || !k || !v || !gates || !y || !fin) return rr::fail(RR_EINVAL, "gla_final_fwd: null pointer argument");
+  if (rr_gla_final_workspace_bytes(B, L, H, Dh, seg, dtype) < 0)
+    return rr::fail(RR_EUNSUPPORTED, "gla_final_fwd: call not covered (rr_gla_final_workspace_bytes is -1)");
+  FinalArgs p{};
+  p.u = static_cast<const uint16_t*>(v);
+  p.step = static_cast<const uint16_t*>(gates);
+  p.Bm = static_cast<const uint16_t*>(k);
+  p.Cm = static_cast<const uint16_t*>(q);
+  p.h0 = h0;
+  p.y = y;
+  p.fin = fin;
+  p.L = (int)L; p.H = (int)H; p.nC = (int)((L + Q - 1) / Q);
+  return run<true>(p, B, H, Dh, Dh, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}

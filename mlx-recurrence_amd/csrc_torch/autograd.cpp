@@ -122,6 +122,15 @@ int64_t numel(at::IntArrayRef sizes) {
   return n;
 }
 
+// Whether a call of these inputs records a backward (what Function::apply
+// itself decides by); without one the forward keeps no checkpoints.
+bool records(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
 // ------------------------------------------------------------------ SSD
 // A_neg as passed by the caller: [H] (one rate per head), [H, N] with stride 0
 // along N (a broadcast per-head rate) or a dense [H, N].  The kernels take
@@ -130,7 +139,7 @@ int64_t numel(at::IntArrayRef sizes) {
 struct SSDFn : public torch::autograd::Function<SSDFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& u, const Tensor& delta, const Tensor& Bm,
                                const Tensor& Cm, const Tensor& A_neg, const c10::optional<Tensor>& h0opt,
-                               int64_t seg) {
+                               int64_t seg, bool grad) {
     const Tensor h0 = h0opt.has_value() ? *h0opt : Tensor();
     require_device({&u, &delta, &Bm, &Cm, &A_neg, &h0});
     const at::DeviceGuard guard(u.device());
@@ -147,9 +156,19 @@ struct SSDFn : public torch::autograd::Function<SSDFn> {
       A_ = prep(A_neg, at::kFloat);
     }
     const Tensor h0_ = h0.defined() ? prep(h0, at::kFloat) : Tensor();
+    const auto f32 = u_.options().dtype(at::kFloat);
+    const int64_t fwsb = grad ? -1 : rr_ssd_final_workspace_bytes(Bsz, L, H, Dh, N, seg, a_sn, dtype_code(dt));
+    if (fwsb >= 0) {   // y and the final state only
+      ctx->set_materialize_grads(false);
+      Tensor y = at::empty({Bsz, L, H, Dh}, f32), fin = at::empty({Bsz, H, Dh, N}, f32);
+      const Tensor ws = workspace((size_t)fwsb, u_.options());
+      check(rr_ssd_final_fwd(P(u_), P(d_), P(B_), P(C_), PF(A_), a_sn, dtype_code(dt), Bsz, L, H, Dh, N, seg, PF(h0_),
+                             MF(y), MF(fin), P(ws), (size_t)fwsb, stream_of(u_)),
+            "rr_ssd_final_fwd");
+      return {y, fin};
+    }
     const int64_t nC = L / rr_chunk_len(L, seg);
     const size_t wsb = rr_ssd_workspace_bytes(Bsz, L, H, Dh, N, seg, a_sn, dtype_code(dt), 0);
-    const auto f32 = u_.options().dtype(at::kFloat);
     Tensor y = at::empty({Bsz, L, H, Dh}, f32), ckpt = at::empty({Bsz, H, nC, Dh, N}, f32);
     const Tensor ws = workspace(wsb, u_.options());
     check(rr_ssd_fwd(P(u_), P(d_), P(B_), P(C_), PF(A_), a_sn, dtype_code(dt), Bsz, L, H, Dh, N, seg, PF(h0_),
@@ -194,20 +213,21 @@ struct SSDFn : public torch::autograd::Function<SSDFn> {
                      PF(h0_), PF(ckpt), P(du), P(dd), P(dB), P(dC), MF(dA), heads ? 0 : 1, MF(dh0), P(ws), wsb,
                      stream_of(u_)),
           "rr_ssd_bwd");
-    return {du, dd, dB, dC, dA, dh0, Tensor()};
+    return {du, dd, dB, dC, dA, dh0, Tensor(), Tensor()};
   }
 };
 
 std::tuple<Tensor, Tensor> ssd_scan(const Tensor& u, const Tensor& delta, const Tensor& Bm, const Tensor& Cm,
                                     const Tensor& A_neg, const c10::optional<Tensor>& h0, int64_t seg) {
-  const variable_list out = SSDFn::apply(u, delta, Bm, Cm, A_neg, h0, seg);
+  const variable_list out = SSDFn::apply(u, delta, Bm, Cm, A_neg, h0, seg,
+                   records({&u, &delta, &Bm, &Cm, &A_neg}) || (h0.has_value() && records({&*h0})));
   return {out[0], out[1]};
 }
 
 // ------------------------------------------------------------------ GLA
 struct GLAFn : public torch::autograd::Function<GLAFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
-                               const Tensor& gates, const c10::optional<Tensor>& h0opt, int64_t seg) {
+                               const Tensor& gates, const c10::optional<Tensor>& h0opt, int64_t seg, bool grad) {
     const Tensor h0 = h0opt.has_value() ? *h0opt : Tensor();
     require_device({&q, &k, &v, &gates, &h0});
     const at::DeviceGuard guard(q.device());
@@ -215,9 +235,19 @@ struct GLAFn : public torch::autograd::Function<GLAFn> {
     const Tensor q_ = prep(q, dt), k_ = prep(k, dt), v_ = prep(v, dt), g_ = prep(gates, dt);
     const int64_t B = q_.size(0), L = q_.size(1), H = q_.size(2), Dh = q_.size(3);
     const Tensor h0_ = h0.defined() ? prep(h0, at::kFloat) : Tensor();
+    const auto f32 = q_.options().dtype(at::kFloat);
+    const int64_t fwsb = grad ? -1 : rr_gla_final_workspace_bytes(B, L, H, Dh, seg, dtype_code(dt));
+    if (fwsb >= 0) {   // y and the final state only
+      ctx->set_materialize_grads(false);
+      Tensor y = at::empty({B, L, H, Dh}, f32), fin = at::empty({B, H, Dh, Dh}, f32);
+      const Tensor ws = workspace((size_t)fwsb, q_.options());
+      check(rr_gla_final_fwd(P(q_), P(k_), P(v_), P(g_), dtype_code(dt), B, L, H, Dh, seg, PF(h0_), MF(y), MF(fin), P(ws),
+                             (size_t)fwsb, stream_of(q_)),
+            "rr_gla_final_fwd");
+      return {y, fin};
+    }
     const int64_t nC = L / rr_chunk_len(L, seg);
     const size_t wsb = rr_gla_workspace_bytes(B, L, H, Dh, seg, dtype_code(dt), 0);
-    const auto f32 = q_.options().dtype(at::kFloat);
     Tensor y = at::empty({B, L, H, Dh}, f32), ckpt = at::empty({B, H, nC, Dh, Dh}, f32);
     const Tensor ws = workspace(wsb, q_.options());
     check(rr_gla_fwd(P(q_), P(k_), P(v_), P(g_), dtype_code(dt), B, L, H, Dh, seg, PF(h0_), MF(y), MF(ckpt),
@@ -257,13 +287,14 @@ struct GLAFn : public torch::autograd::Function<GLAFn> {
     check(rr_gla_bwd(PF(dy), PF(dfinal), P(q_), P(k_), P(v_), P(g_), dtc, B, L, H, Dh, seg, PF(h0_), PF(ckpt), P(dq),
                      P(dk), P(dv), P(dg), MF(dh0), P(ws), wsb, stream_of(q_)),
           "rr_gla_bwd");
-    return {dq, dk, dv, dg, dh0, Tensor()};
+    return {dq, dk, dv, dg, dh0, Tensor(), Tensor()};
   }
 };
 
 std::tuple<Tensor, Tensor> gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& gates,
                                     const c10::optional<Tensor>& h0, int64_t seg) {
-  const variable_list out = GLAFn::apply(q, k, v, gates, h0, seg);
+  const variable_list out = GLAFn::apply(q, k, v, gates, h0, seg,
+                                          records({&q, &k, &v, &gates}) || (h0.has_value() && records({&*h0})));
   return {out[0], out[1]};
 }
 

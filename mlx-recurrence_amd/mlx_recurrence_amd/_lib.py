@@ -49,6 +49,10 @@ _SIGS = {
                    + [_c_ptr] * 2 + [_c_size, _c_ptr]),
     "rr_ssd_bwd_noalloc": (_c_int, [_c_ptr] * 7 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 7 + [_c_i64]
                            + [_c_ptr] * 2),
+    "rr_ssd_final_workspace_bytes": (_c_i64, [_c_i64] * 7 + [_c_int]),
+    "rr_ssd_final_fwd": (_c_int, [_c_ptr] * 5 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 4 + [_c_size, _c_ptr]),
+    "rr_gla_final_workspace_bytes": (_c_i64, [_c_i64] * 5 + [_c_int]),
+    "rr_gla_final_fwd": (_c_int, [_c_ptr] * 4 + [_c_int] + [_c_i64] * 5 + [_c_ptr] * 4 + [_c_size, _c_ptr]),
     "rr_gla_workspace_bytes": (_c_size, [_c_i64] * 5 + [_c_int, _c_int]),
     "rr_gla_fwd": (_c_int, [_c_ptr] * 4 + [_c_int] + [_c_i64] * 5 + [_c_ptr] * 4 + [_c_size, _c_ptr]),
     "rr_gla_bwd": (_c_int, [_c_ptr] * 6 + [_c_int] + [_c_i64] * 5 + [_c_ptr] * 8 + [_c_size, _c_ptr]),
@@ -298,7 +302,38 @@ def ssd_bwd_noalloc(dy, dfinal, u, delta, Bm, Cm, A, a_stride_n, h0, ckpt, seg, 
     _check(rc, "rr_ssd_bwd_noalloc")
 
 
+def records(*tensors) -> bool:
+    """Whether a call of these inputs records a backward."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def ssd_final_workspace(B, L, H, Dh, N, seg, a_stride_n, dtype) -> int:
+    """Workspace bytes of ssd_final_fwd, or -1 where ssd_fwd is to run the call."""
+    return _ws_bytes("rr_ssd_final_workspace_bytes", (B, L, H, Dh, N, seg, a_stride_n, DTYPE_CODE[dtype]))
+
+
+def ssd_final_fwd(u, delta, Bm, Cm, A, a_stride_n, h0, seg, y, fin, ws):
+    B, L, H, Dh = u.shape
+    rc = load().rr_ssd_final_fwd(
+        ptr(u), ptr(delta), ptr(Bm), ptr(Cm), ptr(A), a_stride_n, DTYPE_CODE[u.dtype],
+        B, L, H, Dh, Bm.shape[-1], seg, ptr(h0), ptr(y), ptr(fin), ptr(ws),
+        0 if ws is None else ws.numel(), stream_of(u))
+    _check(rc, "rr_ssd_final_fwd")
+
+
 # ---------------------------------------------------------------- GLA
+def gla_final_workspace(B, L, H, Dh, seg, dtype) -> int:
+    return _ws_bytes("rr_gla_final_workspace_bytes", (B, L, H, Dh, seg, DTYPE_CODE[dtype]))
+
+
+def gla_final_fwd(q, k, v, g, h0, seg, y, fin, ws):
+    B, L, H, Dh = q.shape
+    rc = load().rr_gla_final_fwd(
+        ptr(q), ptr(k), ptr(v), ptr(g), DTYPE_CODE[q.dtype], B, L, H, Dh, seg,
+        ptr(h0), ptr(y), ptr(fin), ptr(ws), 0 if ws is None else ws.numel(), stream_of(q))
+    _check(rc, "rr_gla_final_fwd")
+
+
 def gla_workspace(B, L, H, Dh, seg, dtype, pass_, device) -> torch.Tensor | None:
     n = _ws_bytes("rr_gla_workspace_bytes", (B, L, H, Dh, seg, DTYPE_CODE[dtype], pass_))
     return _alloc_ws(n, device)

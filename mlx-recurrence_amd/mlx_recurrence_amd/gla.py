@@ -37,14 +37,21 @@ def _validate(q, k, v, gates):
 
 class _GLAScan(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, gates, h0, seg):
+    def forward(ctx, q, k, v, gates, h0, seg, grad=True):
         dev = _lib.require_device(q, k, v, gates, h0)
         dt = _lib.common_dtype(q, k, v, gates)
         q_, k_, v_, g_ = (_lib.prep(t, dt) for t in (q, k, v, gates))
         B, L, H, Dh = q_.shape
         h0_ = None if h0 is None else _lib.prep(h0, torch.float32)
-        nC = L // _lib.chunk_len(L, seg)
         y = torch.empty((B, L, H, Dh), dtype=torch.float32, device=dev)
+        fwsb = -1 if grad else _lib.gla_final_workspace(B, L, H, Dh, seg, dt)
+        if fwsb >= 0:   # y and the final state only
+            ctx.set_materialize_grads(False)
+            fin = torch.empty((B, H, Dh, Dh), dtype=torch.float32, device=dev)
+            with _lib.device_guard(dev):
+                _lib.gla_final_fwd(q_, k_, v_, g_, h0_, seg, y, fin, _lib._alloc_ws(fwsb, dev))
+            return y, fin
+        nC = L // _lib.chunk_len(L, seg)
         ckpt = torch.empty((B, H, nC, Dh, Dh), dtype=torch.float32, device=dev)
         with _lib.device_guard(dev):
             ws = _lib.gla_workspace(B, L, H, Dh, seg, dt, 0, dev)
@@ -67,7 +74,7 @@ class _GLAScan(torch.autograd.Function):
         with _lib.device_guard(dev):
             ws = _lib.gla_workspace(B, L, H, Dh, ctx.seg, q_.dtype, 1, dev)
             _lib.gla_bwd(dy, dfinal, q_, k_, v_, g_, h0_, ckpt, ctx.seg, dq, dk, dv, dg, dh0, ws)
-        return dq, dk, dv, dg, dh0, None
+        return dq, dk, dv, dg, dh0, None, None
 
 
 def _run(q, k, v, gates, seg, initial_state):
@@ -80,7 +87,7 @@ def _run(q, k, v, gates, seg, initial_state):
     ext = _lib.autograd_ext()
     if ext is not None:   # the same forward / backward as one C++ autograd node
         return ext.gla_scan(q, k, v, gates, initial_state, seg)
-    return _GLAScan.apply(q, k, v, gates, initial_state, seg)
+    return _GLAScan.apply(q, k, v, gates, initial_state, seg, _lib.records(q, k, v, gates, initial_state))
 
 
 def gla_scan(q, k, v, gates, seg=DEFAULT_SEG, *, initial_state=None):

@@ -59,7 +59,7 @@ def _decay_rates(A_neg):
 
 class _SSDScan(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, u, delta, Bm, Cm, A_neg, h0, seg):
+    def forward(ctx, u, delta, Bm, Cm, A_neg, h0, seg, grad=True):
         dev = _lib.require_device(u, delta, Bm, Cm, A_neg, h0)
         dt = _lib.common_dtype(u, delta, Bm, Cm)
         u_, d_, B_, C_ = (_lib.prep(t, dt) for t in (u, delta, Bm, Cm))
@@ -67,8 +67,15 @@ class _SSDScan(torch.autograd.Function):
         Bsz, L, H, Dh = u_.shape
         N = B_.shape[-1]
         h0_ = None if h0 is None else _lib.prep(h0, torch.float32)
-        nC = L // _lib.chunk_len(L, seg)
         y = torch.empty((Bsz, L, H, Dh), dtype=torch.float32, device=dev)
+        fwsb = -1 if grad else _lib.ssd_final_workspace(Bsz, L, H, Dh, N, seg, a_sn, dt)
+        if fwsb >= 0:   # y and the final state only
+            ctx.set_materialize_grads(False)
+            fin = torch.empty((Bsz, H, Dh, N), dtype=torch.float32, device=dev)
+            with _lib.device_guard(dev):
+                _lib.ssd_final_fwd(u_, d_, B_, C_, A_, a_sn, h0_, seg, y, fin, _lib._alloc_ws(fwsb, dev))
+            return y, fin
+        nC = L // _lib.chunk_len(L, seg)
         ckpt = torch.empty((Bsz, H, nC, Dh, N), dtype=torch.float32, device=dev)
         with _lib.device_guard(dev):
             ws = _lib.ssd_workspace(Bsz, L, H, Dh, N, seg, a_sn, dt, 0, dev)
@@ -95,7 +102,7 @@ class _SSDScan(torch.autograd.Function):
         with _lib.device_guard(dev):
             ws = _lib.ssd_workspace(Bsz, L, H, Dh, N, ctx.seg, ctx.a_sn, u_.dtype, 1, dev)
             _lib.ssd_bwd(dy, dfinal, u_, d_, B_, C_, A_, ctx.a_sn, h0_, ckpt, ctx.seg, du, dd, dB, dC, dA, dh0, ws)
-        return du, dd, dB, dC, dA, dh0, None
+        return du, dd, dB, dC, dA, dh0, None, None
 
 
 def _run(u, delta, B, C, A_neg, seg, initial_state):
@@ -108,7 +115,8 @@ def _run(u, delta, B, C, A_neg, seg, initial_state):
     ext = _lib.autograd_ext()
     if ext is not None:   # the same forward / backward as one C++ autograd node
         return ext.ssd_scan(u, delta, B, C, A_neg, initial_state, seg)
-    return _SSDScan.apply(u, delta, B, C, A_neg, initial_state, seg)
+    return _SSDScan.apply(u, delta, B, C, A_neg, initial_state, seg,
+                          _lib.records(u, delta, B, C, A_neg, initial_state))
 
 
 def ssd_scan(u, delta, B, C, A_neg, seg=DEFAULT_SEG, *, initial_state=None):

@@ -1,0 +1,115 @@
+"""The forward that keeps no checkpoints (final_fwd.hip: calls without a
+gradient, bf16, one decay rate per head for SSD) against the float64 oracle and
+against the general path, at the edges of its chunks and segments (MI355X only).
+
+Bar: it works to fp32 accuracy (three-term bf16 splits, fp32 accumulation), so
+outputs are held to the fp32 bar, 1e-5 of the largest value."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import mlx_recurrence_amd as mr
+from mlx_recurrence_amd import _lib
+from oracle import recurrence_oracle as orc
+from tests.gpu_util import TOL, check, rounded, to_dev
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def _ssd(B, L, H, Dh, N, seed):
+    rng = np.random.default_rng(seed)
+    return [to_dev(rng.standard_normal((B, L, H, Dh)), BF16),
+            to_dev(np.abs(rng.standard_normal((B, L, H))) * 0.1 + 0.01, BF16),
+            to_dev(rng.standard_normal((B, L, H, N)), BF16), to_dev(rng.standard_normal((B, L, H, N)), BF16),
+            to_dev(-np.exp(rng.uniform(0, np.log(16), H)), F32)], to_dev(rng.standard_normal((B, H, Dh, N)), F32)
+
+
+def _gla(B, L, H, Dh, seed):
+    rng = np.random.default_rng(seed)
+    g = 1 / (1 + np.exp(-(rng.standard_normal((B, L, H)) + 2)))
+    g[:, L // 2] *= -1          # either sign
+    g[:, L // 3] = 0            # a reset
+    return ([to_dev(rng.standard_normal((B, L, H, Dh)) / np.sqrt(Dh), BF16) for _ in range(3)] + [to_dev(g, BF16)],
+            to_dev(rng.standard_normal((B, H, Dh, Dh)), F32))
+
+
+# (B, L, H, Dh, N, seg): one step, a chunk less one, a chunk plus one, odd tails,
+# every Dh and N, several segments (1000 and 2040 steps of few heads), T = 32
+SSD = [(1, 1, 2, 32, 16, 1), (2, 31, 1, 64, 128, 31), (1, 33, 3, 128, 32, 11), (2, 40, 5, 32, 64, 8),
+       (1, 100, 3, 64, 64, 4), (2, 1000, 3, 64, 16, 8), (1, 2040, 2, 32, 128, 8), (1, 520, 2, 128, 128, 8),
+       (1, 72, 2, 128, 16, 24), (1, 77, 2, 32, 32, 7), (3, 544, 2, 64, 128, 32), (1, 768, 1, 64, 32, 32)]
+GLA = [(1, 1, 2, 64, 1), (2, 31, 1, 32, 31), (1, 33, 3, 128, 11), (1, 1000, 2, 64, 8), (2, 520, 1, 128, 8),
+       (1, 100, 3, 32, 20), (1, 544, 2, 64, 32)]
+
+
+@pytest.mark.parametrize("h0", [False, True])
+@pytest.mark.parametrize("B,L,H,Dh,N,seg", SSD)
+def test_ssd_final(B, L, H, Dh, N, seg, h0):
+    print(f"[case] ssd final B={B} L={L} H={H} Dh={Dh} N={N} seg={seg} h0={h0}", flush=True)
+    assert _lib.ssd_final_workspace(B, L, H, Dh, N, seg, 0, BF16) >= 0
+    ins, st = _ssd(B, L, H, Dh, N, L + Dh)
+    y, fs = mr.ssd_scan_with_state(*ins, seg=seg, initial_state=st if h0 else None)
+    ref = [rounded(t) for t in ins]
+    ref[4] = np.repeat(ref[4][:, None], N, axis=1)
+    y_o, fs_o = orc.ssd_forward(*ref, rounded(st) if h0 else None)
+    rep = {}
+    assert y.shape == (B, L, H, Dh) and fs.shape == (B, H, Dh, N)
+    check("y", y, y_o, TOL[F32], rep)
+    check("final", fs, fs_o, TOL[F32], rep)
+    print(rep, flush=True)
+
+
+@pytest.mark.parametrize("h0", [False, True])
+@pytest.mark.parametrize("B,L,H,Dh,seg", GLA)
+def test_gla_final(B, L, H, Dh, seg, h0):
+    print(f"[case] gla final B={B} L={L} H={H} Dh={Dh} seg={seg} h0={h0}", flush=True)
+    assert _lib.gla_final_workspace(B, L, H, Dh, seg, BF16) >= 0
+    ins, st = _gla(B, L, H, Dh, L + Dh)
+    y, fs = mr.gla_scan_with_state(*ins, seg=seg, initial_state=st if h0 else None)
+    y_o, fs_o = orc.gla_forward(*[rounded(t) for t in ins], rounded(st) if h0 else None)
+    rep = {}
+    check("y", y, y_o, TOL[F32], rep)
+    check("final", fs, fs_o, TOL[F32], rep)
+    print(rep, flush=True)
+
+
+def test_forms_agree_with_the_recording_path():
+    """Every form the call accepts (strided and misaligned inputs, the three
+    forms of A_neg, mixed dtypes) gives what the path with checkpoints gives;
+    calls it does not cover go there."""
+    B, L, H, Dh, N, seg = 2, 72, 3, 64, 32, 8
+    ins, st = _ssd(B, L, H, Dh, N, 5)
+    u, d, Bm, Cm, A = ins
+    pad = torch.empty(u.numel() + 1, dtype=BF16, device=u.device)[1:]
+    odd = pad.copy_(u.flatten()).view_as(u)                                   # 2-byte aligned
+    strided = u.transpose(1, 2).contiguous().transpose(1, 2)
+    stt = st.transpose(-1, -2).contiguous().transpose(-1, -2)
+    forms = [(u, d, Bm, Cm, A), (odd, d, Bm, Cm, A), (strided, d, Bm, Cm, A[:, None].expand(H, N)),
+             (u, d, Bm.float(), Cm, A), (u, d, Bm, Cm, A[:, None].expand(H, N).contiguous())]
+    for k, f in enumerate(forms):
+        print(f"[case] form {k}", flush=True)
+        y, fs = mr.ssd_scan_with_state(*f, seg=seg, initial_state=stt)
+        yr, fr = mr.ssd_scan_with_state(f[0].detach().requires_grad_(True), *f[1:], seg=seg, initial_state=stt)
+        for got, want in ((y, yr), (fs, fr)):
+            assert got.dtype == want.dtype and got.shape == want.shape and not got.requires_grad
+            assert (got - want).abs().max() <= 1e-5 * want.abs().max(), k
+    assert _lib.ssd_final_workspace(B, L, H, Dh, N, seg, 1, BF16) == -1     # dense A
+    assert _lib.ssd_final_workspace(B, L, H, Dh, N, seg, 0, F32) == -1
+    assert _lib.ssd_final_workspace(B, L, H, 96, N, seg, 0, BF16) == -1
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_non_finite_input_stays_causal(bad):
+    """A non-finite u, B or C at one step leaves every earlier step as it was."""
+    B, L, H, Dh, N, s = 1, 72, 2, 64, 128, 41
+    ins, st = _ssd(B, L, H, Dh, N, 9)
+    clean, _ = mr.ssd_scan_with_state(*ins, seg=8, initial_state=st)
+    for k in (0, 2, 3):
+        xs = [t.clone() for t in ins]
+        xs[k][0, s, 1, 5] = bad
+        y, _ = mr.ssd_scan_with_state(*xs, seg=8, initial_state=st)
+        assert torch.equal(y[:, :s], clean[:, :s]) and torch.equal(y[:, :, 0], clean[:, :, 0]), k
+        assert not torch.isfinite(y[0, s, 1]).all(), k
