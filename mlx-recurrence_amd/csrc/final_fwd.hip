@@ -1,6 +1,7 @@
-// final_fwd.hip — SSD (one decay rate per head) and GLA forward for calls that
-// need y and the final state only (no gradient, so no checkpoints): bf16
-// inputs of any length L >= 1.
+// final_fwd.hip — SSD (one decay rate per head) and GLA forward, bf16 inputs, a
+// head's chunks walked in order by one workgroup: for calls that need y and
+// the final state only (no gradient, so no checkpoints; any length L >= 1),
+// and, writing the state after every chunk, for the training forward.
 //
 // Per (batch, head) the recurrence and its 32-step chunk form are those of
 // rr_chunked.h,
@@ -27,12 +28,18 @@
 // its decay), and the walk of segment j starts from h0 carried through the
 // maps of segments 0 .. j - 1.
 //
-// What bounds it: the instructions of a chunk (per wave about 700 VALU, a
-// third of them the three-term splits, beside 66 MFMAs at N = 128) on two
-// waves per SIMD, not memory: B4 L1000 H80 Dh64 N128 takes 132 us, 2.3 TB/s of
-// the 0.31 GB it cannot do without (6.1 ms on the VALU engine, which forms and
-// stores a state every 8 steps there); B8 L4096 H80 895 us where the training
-// forward with its 2.7 GB of checkpoints takes 1227.
+// W is formed once per chunk: its three nonzero 16x16 blocks are dealt to the
+// waves, which also take turns at the step scalars, a chunk ahead, so a chunk
+// has two barriers (LDS only: loads and stores stay in flight across them).
+//
+// What bounds it: without checkpoints the instructions of a chunk (per wave
+// about 500 VALU, a third of them the state's three-term split, beside 50
+// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 107 us,
+// 2.9 TB/s of the 0.31 GB it cannot do without (6.1 ms on the VALU engine,
+// which forms and stores a state every 8 steps there; 132 us with W and the
+// scalars formed by every wave for itself).  Three waves per SIMD (168 VGPRs)
+// spill 18 and take 178 us.  With checkpoints the traffic: B8 L4096 H80 Dh64
+// N128 1224 us, 4.4 TB/s; B8 L2048 H12 GLA Dh128 448 -> 215 us.
 #include "rr_chunked.h"
 
 namespace {
@@ -51,7 +58,7 @@ struct FinalArgs {
   const float* A;         // [H] (SSD)
   const float* h0;        // [B,H,DH,N] as d, n (GLA [B,H,N,DH] as n, d), or null
   float* y;               // [B,L,H,DH]
-  float* fin;             // layout of h0
+  float* fin;             // final state, layout of h0 (kCkpt: the checkpoints [B*H][nC][DH][N])
   float4* segE;           // [B*H][S-1] segment states in fragment order
   float* segP;            // [B*H][S-1] segment decays
   int L, H, nC, S, cps;   // chunks, segments, chunks per segment
@@ -97,78 +104,69 @@ template <int DH, int NS, int DB>
 struct alignas(16) FinalSm {
   static constexpr int NSP = NS < 32 ? 32 : NS, NW = DH / (16 * DB);
   uint16_t B[2][Q * NSP], C[2][Q * NSP], U[2][Q * DH];
-  float sc[2][NW][4][Q];   // per wave: gam, m31 w, cd (GLA: gates), w
+  uint2 W[2][3][3][64];    // a chunk's W: [16x16 block][hi, mid, lo][lane], see w_block
+  float sc[3][4][Q];       // a chunk's step scalars: gam, m31 w, cd (GLA: gates), w
 };
 
-// The 12 decays M[t][s] of a lane: t = 16 tb + l15; m0[e]: tb 0, s = 4 g + e;
-// m1[e]: tb 1, s = 4 g + e; m1[4 + e]: tb 1, s = 16 + 4 g + e; zero for s > t.
+// The four decays M[t][s] a lane holds of 16x16 block blk of (C B^T)^T:
+// blk 0: s = 4 g + e, t = l15; blk 1: s = 4 g + e, t = 16 + l15; blk 2: both
+// plus 16.  Zero for s > t.
 template <bool GLA>
-__device__ __forceinline__ void decays(const float* st, float a, int l15, int g, float (&m0)[4], float (&m1)[8]) {
-  const float4 s0 = *reinterpret_cast<const float4*>(&st[4 * g]);
-  const float4 s1 = *reinterpret_cast<const float4*>(&st[16 + 4 * g]);
-  const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+__device__ __forceinline__ void decays(const float* st, float a, int blk, int l15, int g, float (&m)[4]) {
+  const int s0 = blk == 2 ? 16 : 0, t0 = blk > 0 ? 16 : 0;
+  const float4 sq = *reinterpret_cast<const float4*>(&st[s0 + 4 * g]);
+  const float sv[4] = {sq.x, sq.y, sq.z, sq.w};
   if constexpr (!GLA) {
-    const float c0 = st[l15], c1 = st[16 + l15];
+    const float ct = st[t0 + l15];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      m0[e] = rr::chunked::masked_exp(4 * g + e <= l15, a * (c0 - sv[e]));
-      m1[e] = __expf(a * (c1 - sv[e]));
-      m1[4 + e] = rr::chunked::masked_exp(4 * g + e <= l15, a * (c1 - sv[4 + e]));
-    }
+    for (int e = 0; e < 4; ++e) m[e] = rr::chunked::masked_exp(blk == 1 || 4 * g + e <= l15, a * (ct - sv[e]));
   } else {
     // products of the gates of steps s + 1 .. t, by quads of steps: the rest
     // of s's quad, whole quads between, t's quad up to t (any sign, zeros exact)
-    float qd[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float4 q = *reinterpret_cast<const float4*>(&st[4 * j]);
-      qd[j] = (q.x * q.y) * (q.z * q.w);
-    }
     const int qt = l15 >> 2, pt = l15 & 3;   // t's quad within its 16 steps, position in it
-    const float4 t0 = *reinterpret_cast<const float4*>(&st[4 * qt]);
-    const float4 t1 = *reinterpret_cast<const float4*>(&st[16 + 4 * qt]);
-    auto upto = [&](const float4& q) {
-      const float p1 = q.x * q.y, p2 = p1 * q.z, p3 = p2 * q.w;
-      return pt == 0 ? q.x : pt == 1 ? p1 : pt == 2 ? p2 : p3;
+    const float4 tq = *reinterpret_cast<const float4*>(&st[t0 + 4 * qt]);
+    const float p1 = tq.x * tq.y, p2 = p1 * tq.z, p3 = p2 * tq.w;
+    float far = pt == 0 ? tq.x : pt == 1 ? p1 : pt == 2 ? p2 : p3;
+    auto quad = [&](int j) {
+      const float4 q = *reinterpret_cast<const float4*>(&st[4 * j]);
+      return (q.x * q.y) * (q.z * q.w);
     };
-    const float h0 = upto(t0), h1 = upto(t1);
-    // whole quads strictly between g and qt (both in 0 .. 3: quads 1 and 2)
-    const bool b1 = g < 1 && qt > 1, b2 = g < 2 && qt > 2;
-    const float mid0 = (b1 ? qd[1] : 1.f) * (b2 ? qd[2] : 1.f);
-    const float mid1 = (b1 ? qd[5] : 1.f) * (b2 ? qd[6] : 1.f);
-    float midx = (g < 1 ? qd[1] : 1.f) * (g < 2 ? qd[2] : 1.f) * (g < 3 ? qd[3] : 1.f);
-    midx *= (qt > 0 ? qd[4] : 1.f) * (qt > 1 ? qd[5] : 1.f) * (qt > 2 ? qd[6] : 1.f);
+    const float r2 = sv[3], r1 = sv[2] * r2, r0 = sv[1] * r1;   // rest of s's quad after s
+    const float rest[4] = {r0, r1, r2, 1.f};
+    if (blk == 1) {   // quads g + 1 .. 3 and 4 .. 3 + qt
+      const float q1 = quad(1), q2 = quad(2), q3 = quad(3), q4 = quad(4), q5 = quad(5), q6 = quad(6);
+      far *= (g < 1 ? q1 : 1.f) * (g < 2 ? q2 : 1.f) * (g < 3 ? q3 : 1.f);
+      far *= (qt > 0 ? q4 : 1.f) * (qt > 1 ? q5 : 1.f) * (qt > 2 ? q6 : 1.f);
 #pragma unroll
-    for (int hb = 0; hb < 2; ++hb) {
-      const float* q = sv + 4 * hb;
-      const float r2 = q[3], r1 = q[2] * r2, r0 = q[1] * r1;   // rest of the quad after s
-      const float rest[4] = {r0, r1, r2, 1.f};
+      for (int e = 0; e < 4; ++e) m[e] = rest[e] * far;
+    } else {
+      // whole quads strictly between g and qt (both in 0 .. 3: quads 1 and 2)
+      const float q1 = quad(s0 / 4 + 1), q2 = quad(s0 / 4 + 2);
+      far *= (g < 1 && qt > 1 ? q1 : 1.f) * (g < 2 && qt > 2 ? q2 : 1.f);
       // t in s's own quad: product of positions e + 1 .. pt
-      const float yz = q[1] * q[2];
-      const float in0 = pt == 0 ? 1.f : pt == 1 ? q[1] : pt == 2 ? yz : yz * q[3];
-      const float in1 = pt == 1 ? 1.f : pt == 2 ? q[2] : q[2] * q[3];
-      const float in2 = pt == 2 ? 1.f : q[3];
+      const float yz = sv[1] * sv[2];
+      const float in0 = pt == 0 ? 1.f : pt == 1 ? sv[1] : pt == 2 ? yz : yz * sv[3];
+      const float in1 = pt == 1 ? 1.f : pt == 2 ? sv[2] : sv[2] * sv[3];
+      const float in2 = pt == 2 ? 1.f : sv[3];
       const float inq[4] = {in0, in1, in2, 1.f};
-      const float far = (hb ? mid1 : mid0) * (hb ? h1 : h0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float v = qt == g ? inq[e] : rest[e] * far;
-        const float keep = 4 * g + e <= l15 ? v : 0.f;
-        if (hb) m1[4 + e] = keep;
-        else {
-          m0[e] = keep;
-          m1[e] = rest[e] * midx * h1;
-        }
+        m[e] = 4 * g + e <= l15 ? v : 0.f;
       }
     }
   }
 }
 
-// AGG: only the segment's state from a zero start and its decay (segE, segP).
-template <int DH, int NS, bool GLA, int DB, bool AGG>
+// OUT: kMap only the segment's state from a zero start and its decay (segE,
+// segP); kFinal y and the final state; kCkpt y and the state after every chunk
+// (L a multiple of 32).
+enum Out { kMap = 0, kFinal = 1, kCkpt = 2 };
+template <int DH, int NS, bool GLA, int DB, int OUT>
 __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) {
   using S = FinalSm<DH, NS, DB>;
   constexpr int NSP = S::NSP, NW = S::NW, T = 64 * NW, NK = NSP / 32, NBN = NSP / 16;
+  constexpr bool AGG = OUT == kMap;
   constexpr int BV = (Q * NS / 8 + T - 1) / T, UV = (Q * DH / 8 + T - 1) / T;
   __shared__ S sm;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -188,7 +186,7 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
   }
 
   u16x8_t bv[BV], cv[BV], uv[UV];
-  float xv;
+  float xv;   // this lane's step input of the chunk whose scalars come next
   // chunk c's pieces into registers: unconditional loads, offsets past the
   // sequence clamped to its last piece (those rows become zero, or the neutral
   // step, when staged)
@@ -210,7 +208,55 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
       const int i = min(tid + T * v, Q * DH / 8 - 1);
       uv[v] = rr::ld32<u16x8_t>(Up, min((uint32_t)(i / (DH / 8)) * rsD + 8 * (i % (DH / 8)), lastD));
     }
-    xv = rr::bf_val(p.step[(rows + t0 + min(lane & (Q - 1), last)) * p.H + h]);
+  };
+  auto load_step = [&](int c) {
+    const int t0 = min(c, p.nC - 1) * Q;
+    xv = rr::bf_val(p.step[(rows + t0 + min(lane & (Q - 1), p.L - 1 - t0)) * p.H + h]);
+  };
+  // step scalars of chunk c (one wave)
+  auto scalars = [&](int c) {
+    const bool live = lane < Q && lane < p.L - c * Q;
+    const float x = live ? xv : (GLA ? 1.f : 0.f);
+    const rr::chunked::StepScalars st = rr::chunked::step_scalars<GLA>(x, a, lane);
+    float(*sc)[Q] = sm.sc[c % 3];
+    if (lane < Q) {
+      sc[0][lane] = st.gam;
+      sc[1][lane] = st.m31 * st.w;
+      sc[2][lane] = GLA ? x : st.cd;
+      sc[3][lane] = st.w;
+    }
+  };
+  // W[t][s] = M[t][s] (C B^T)[t][s] w_s of chunk c from its staged B and C, by
+  // 16x16 blocks (three: the upper right one is zero) dealt to the waves; the
+  // accumulators of (C B^T)^T are W's A operand, kept as lane fragments
+  auto w_blocks = [&](int c, int buf) {
+    const float(*sc)[Q] = sm.sc[c % 3];
+    for (int blk = w; blk < 3; blk += NW) {
+      const int ro = (blk == 2 ? 16 * NSP : 0), co = (blk > 0 ? 16 * NSP : 0);
+      f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) {
+        const int off = l15 * NSP + 8 * ((4 * kk + g) ^ swz_n<NSP>(l15));
+        d = rr::mfma16(rr::frag(&sm.B[buf][off + ro]), rr::frag(&sm.C[buf][off + co]), d);
+      }
+      float m[4];
+      decays<GLA>(sc[2], a, blk, l15, g, m);
+      const float4 x = *reinterpret_cast<const float4*>(&sc[3][(blk == 2 ? 16 : 0) + 4 * g]);
+      const float wl[4] = {x.x, x.y, x.z, x.w};
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {   // a select, so that a non-finite B row stays out of earlier steps
+        v[e] = blk == 1 || 4 * g + e <= l15 ? m[e] * (d[e] * wl[e]) : 0.f;
+        v[4 + e] = 0.f;
+      }
+      u16x8_t f[3];
+      split3(v, f[0], f[1], f[2]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const uint4 u4 = __builtin_bit_cast(uint4, f[k]);
+        sm.W[buf][blk][k][lane] = make_uint2(u4.x, u4.y);
+      }
+    }
   };
   auto stage_rows = [&](int V, int buf, auto full) {   // full: all 32 steps present
 #pragma unroll
@@ -242,15 +288,6 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
     const int V = p.L - c * Q;   // steps present
     if (V >= Q) stage_rows(V, buf, std::true_type{});
     else stage_rows(V, buf, std::false_type{});
-    const bool live = lane < V;
-    const float x = live ? xv : (GLA ? 1.f : 0.f);
-    const rr::chunked::StepScalars sc = rr::chunked::step_scalars<GLA>(lane < Q ? x : (GLA ? 1.f : 0.f), a, lane);
-    if (lane < Q) {
-      sm.sc[buf][w][0][lane] = sc.gam;
-      sm.sc[buf][w][1][lane] = sc.m31 * sc.w;
-      sm.sc[buf][w][2][lane] = GLA ? x : sc.cd;
-      sm.sc[buf][w][3][lane] = sc.w;
-    }
   };
 
   f32x4_t hs[DB][NBN];   // h^T[16 nb + 4 g + r][d = 16 (w DB + i) + l15]
@@ -272,6 +309,7 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
             hs[i][nb][r] = hp[rr::chunked::state_off<GLA, DH, NS>(16 * (w * DB + i) + l15, 16 * nb + 4 * g + r)];
     }
     const float4* E = p.segE + (int64_t)bh * (p.S - 1) * (DB * NBN * T) + tid;
+#pragma unroll 2
     for (int j = 0; j < seg; ++j) {
       const float P = p.segP[bh * (p.S - 1) + j];
 #pragma unroll
@@ -284,9 +322,17 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
         }
     }
   }
+  load_step(c0);
   stage(c0, 0);
   load(c0 + 1);
+  if (w == NW - 1) {
+    scalars(c0);
+    load_step(c0 + 1);
+    scalars(min(c0 + 1, p.nC - 1));
+  }
+  load_step(c0 + 2);
   lds_barrier();
+  if constexpr (!AGG) w_blocks(c0, 0);
 
   for (int c = c0; c < c1; ++c) {
     const int buf = (c - c0) & 1;
@@ -294,8 +340,14 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
       stage(c + 1, buf ^ 1);
       load(c + 2);
     }
+    lds_barrier();   // this chunk's W, the next one's rows
+    if constexpr (!AGG) {
+      if (c + 1 < c1) w_blocks(c + 1, buf ^ 1);
+    }
+    if (w == NW - 1 && c + 2 < c1) scalars(c + 2);
+    load_step(c + 3);
     const uint16_t *Bs = sm.B[buf], *Cs = sm.C[buf], *Us = sm.U[buf];
-    const float(*sc)[Q] = sm.sc[buf][w];
+    const float(*sc)[Q] = sm.sc[c % 3];
     const float tot = sc[0][Q - 1];
     // U as B operand: U[pi(g, e)][d]
     u16x8_t uf[DB];
@@ -310,36 +362,19 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
     }
     if constexpr (!AGG) {
       u16x8_t cf[2][NK];   // C[16 tb + l15][32 kk + pi]
-      f32x4_t d00 = {0.f, 0.f, 0.f, 0.f}, d01 = d00, d11 = d00;   // (C B^T)^T blocks [s][t]
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk) {
         const int off = l15 * NSP + 8 * ((4 * kk + g) ^ swz_n<NSP>(l15));
-        const u16x8_t b0 = rr::frag(Bs + off), b1 = rr::frag(Bs + off + 16 * NSP);
         cf[0][kk] = rr::frag(Cs + off);
         cf[1][kk] = rr::frag(Cs + off + 16 * NSP);
-        d00 = rr::mfma16(b0, cf[0][kk], d00);
-        d01 = rr::mfma16(b0, cf[1][kk], d01);
-        d11 = rr::mfma16(b1, cf[1][kk], d11);
       }
-      float w0[8], w1[8];   // W[l15][pi], W[16 + l15][pi]
-      {
-        float m0[4], m1[8];
-        decays<GLA>(sc[2], a, l15, g, m0, m1);
-        const float4 x0 = *reinterpret_cast<const float4*>(&sc[3][4 * g]);
-        const float4 x1 = *reinterpret_cast<const float4*>(&sc[3][16 + 4 * g]);
-        const float wl[4] = {x0.x, x0.y, x0.z, x0.w}, wh[4] = {x1.x, x1.y, x1.z, x1.w};
+      u16x8_t wf[2][3];   // W[16 tb + l15][pi]
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool low = 4 * g + e <= l15;   // a select, so that a non-finite B row stays out of earlier steps
-          w0[e] = low ? m0[e] * (d00[e] * wl[e]) : 0.f;
-          w0[4 + e] = 0.f;
-          w1[e] = m1[e] * (d01[e] * wl[e]);
-          w1[4 + e] = low ? m1[4 + e] * (d11[e] * wh[e]) : 0.f;
-        }
+      for (int k = 0; k < 3; ++k) {
+        const uint2 x0 = sm.W[buf][0][k][lane], x1 = sm.W[buf][1][k][lane], x2 = sm.W[buf][2][k][lane];
+        wf[0][k] = __builtin_bit_cast(u16x8_t, make_uint4(x0.x, x0.y, 0, 0));
+        wf[1][k] = __builtin_bit_cast(u16x8_t, make_uint4(x1.x, x1.y, x2.x, x2.y));
       }
-      u16x8_t wf[2][3];
-      split3(w0, wf[0][0], wf[0][1], wf[0][2]);
-      split3(w1, wf[1][0], wf[1][1], wf[1][2]);
 #pragma unroll
       for (int i = 0; i < DB; ++i) {
         f32x4_t ab[2], as[2];   // C h^T: hi terms, mid + lo terms
@@ -451,6 +486,15 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
       }
     }
     if constexpr (AGG) decay *= tot;
+    if constexpr (OUT == kCkpt) {
+      float* ck = p.fin + ((int64_t)bh * p.nC + c) * DH * NS;
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NS / 16; ++nb)
+          *reinterpret_cast<float4*>(ck + (16 * (w * DB + i) + l15) * NS + 16 * nb + 4 * g) =
+              make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
+    }
     lds_barrier();
   }
 
@@ -462,7 +506,7 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
       for (int nb = 0; nb < NBN; ++nb)
         E[(i * NBN + nb) * T] = make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
     if (tid == 0) p.segP[bh * (p.S - 1) + seg] = decay;
-  } else if (seg == p.S - 1) {
+  } else if (OUT == kFinal && seg == p.S - 1) {
     float* fp = p.fin + (int64_t)bh * DH * NS;
 #pragma unroll
     for (int i = 0; i < DB; ++i)
@@ -486,11 +530,14 @@ bool covered(int64_t Dh, int64_t N, bool gla) {
   return (Dh == 32 || Dh == 64 || Dh == 128) && (N == 16 || N == 32 || N == 64 || N == 128);
 }
 
-// Segments: enough workgroups for two waves per SIMD, at least four chunks each.
+// Segments: enough workgroups for two waves per SIMD, at least two chunks each,
+// and at most sqrt(8 nC): each segment before a walk costs it the reading of a
+// map, each chunk of a segment its map and its output (SSD 8 heads, 32 chunks,
+// Dh 64 N 128: 23.0 us with 8 segments, 22.8 with 10, 18.7 with 16).
 void segments(int64_t BH, int64_t nC, int64_t Dh, int& S, int& cps) {
   const int64_t waves = BH * (Dh / 16), want = std::max<int64_t>(1, 2048 / std::max<int64_t>(waves, 1));
-  int64_t s = std::min(std::min<int64_t>(want, nC / 4), (int64_t)32);
-  s = std::max<int64_t>(s, 1);
+  int64_t s = std::max<int64_t>(1, std::min(want, nC / 2));
+  while (s * s > 8 * nC) --s;
   cps = (int)((nC + s - 1) / s);
   S = (int)((nC + cps - 1) / cps);
 }
@@ -501,18 +548,18 @@ size_t ws_bytes(int64_t BH, int64_t Dh, int64_t N, int S) {
   return (size_t)BH * (S - 1) * (state + 4) + 256;
 }
 
-template <int DH, int NS, bool GLA>
+template <int DH, int NS, bool GLA, int OUT>
 int launch(const FinalArgs& p, int64_t BH, hipStream_t s) {
   constexpr int T = 4 * DH;
   if (p.S > 1) {
-    hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, true>), dim3((unsigned)BH, p.S - 1), dim3(T), 0, s, p);
+    hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, kMap>), dim3((unsigned)BH, p.S - 1), dim3(T), 0, s, p);
     if (int rc = rr::check_launch("final-state forward (segment maps)")) return rc;
   }
-  hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, false>), dim3((unsigned)BH, p.S), dim3(T), 0, s, p);
+  hipLaunchKernelGGL((final_fwd_kernel<DH, NS, GLA, 1, OUT>), dim3((unsigned)BH, p.S), dim3(T), 0, s, p);
   return rr::check_launch("final-state forward");
 }
 
-template <bool GLA>
+template <bool GLA, int OUT>
 int run(FinalArgs& p, int64_t B, int64_t H, int64_t Dh, int64_t N, void* ws, size_t wsb, hipStream_t s) {
   const int64_t BH = B * H;
   segments(BH, p.nC, Dh, p.S, p.cps);
@@ -523,7 +570,7 @@ int run(FinalArgs& p, int64_t B, int64_t H, int64_t Dh, int64_t N, void* ws, siz
     p.segP = reinterpret_cast<float*>(static_cast<char*>(ws) + (size_t)BH * (p.S - 1) * Dh * std::max<int64_t>(N, 32) * 4);
   }
 #define RR_CASE(D, NN) \
-  if (Dh == D && N == NN) return launch<D, NN, GLA>(p, BH, s)
+  if (Dh == D && N == NN) return launch<D, NN, GLA, OUT>(p, BH, s)
   if constexpr (GLA) {
     RR_CASE(32, 32);
     RR_CASE(64, 64);
@@ -544,25 +591,70 @@ bool sizes_ok(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N) {
          H * std::max(Dh, N) * Q * 4 < (int64_t(1) << 31);
 }
 
-// Which calls run here.  Where seg leaves a checkpoint interval T below 32 the
-// other forward is the VALU engine: every covered size (bf16 prompts of odd
-// length: 2.8x at B1 L40 H8, 43x at B4 L1000 H80 Dh64 N128).  At T = 32 it is
-// the training forward with its checkpoints, which has more parallelism for
-// short prompts (resident / direct kernels, one workgroup per chunk) and less
-// work per chunk at N = 16: this kernel from 17 chunks with N >= 64 (24 with
-// N = 32), where it measured 1.08x (GLA B8 L768 H80 Dh64, 166 -> 154 us) to
-// 2.5x (SSD B4 L2048 H24 Dh64 N128, 193 -> 76 us); below that 0.6x to 1.1x
-// (SSD B3 L512 H12 Dh64 N16 9.7 -> 15.1 us), at N = 16 0.83x to 1.22x.
+// Calls without a gradient: where seg leaves a checkpoint interval T below 32
+// the other forward is the VALU engine, so every covered size runs here (bf16
+// prompts of odd length: 2.8x at B1 L40 H8, 57x at B4 L1000 H80 Dh64 N128); at
+// T = 32 the sizes for which the training forward walks too, and N = 32 from 24
+// chunks (no checkpoints to write: SSD 36 heads Dh 32, 24 chunks 17.2 -> 14.3).
 int64_t query(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg, int dtype, bool gla) {
   if (dtype != RR_BF16 || !sizes_ok(B, L, H, Dh, N) || !covered(Dh, N, gla)) return -1;
   const int64_t nC = (L + Q - 1) / Q;
-  if (rr::chunk_len(L, seg) == Q && !(N >= 64 ? nC > 16 : N == 32 && nC >= 24)) return -1;
+  if (rr::chunk_len(L, seg) == Q && !(rr::walk_preferred(B * H, nC, Dh, N, gla) || (N == 32 && nC >= 24 && B * H >= 24)))
+    return -1;
   int S, cps;
   segments(B * H, nC, Dh, S, cps);
   return (int64_t)ws_bytes(B * H, Dh, N, S);
 }
 
 }  // namespace
+
+namespace rr {
+
+// Measured at T = 32 with checkpoints, the walk against the other forwards
+// (resident, direct, whole-head, scan + chunk kernels), us at (heads, chunks):
+// - from 17 chunks with N >= 64 it never lost (1.0x at SSD B8 L4096 H80 Dh64
+//   N128, 1233 -> 1224, bound by its traffic; 456 -> 215 at GLA 96 heads Dh
+//   128; 1.02x to 2.24x between); with N = 32 it wins from 32 chunks (below,
+//   14.8 -> 17.5 at 36 heads); with N = 16 its chunk costs as much as with 32,
+//   so only where the others leave the GPU idle (up to 256 heads; 233 -> 254
+//   at 640);
+// - fewer than 24 heads: the chunk-parallel kernels (SSD 2 heads, 32 chunks,
+//   Dh 64 N 128: 15.9 against 19.7; at 24 heads, 17 chunks 22.3 against 20.8);
+// - in shorter heads the resident and direct kernels are more parallel
+//   (SSD 36 heads, 16 chunks, Dh 64 N 16: 9.5 against 16.3) except N = 64 from
+//   256 heads (66 -> 44 at 320 heads, 16 chunks) and N = 128, which the
+//   resident kernel does not cover, below 512 heads (123 -> 94) unless GLA's
+//   wide direct mode takes it (BH nC <= 768: 23 against 31).
+bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla) {
+  if (BH < 24 || BH * Q >= (int64_t(1) << 31)) return false;
+  if (nC > 16) return N >= 64 || (nC >= 32 && (N == 32 || BH <= 256));
+  if (N == 128) return BH < 512 && !(gla && BH * nC <= 768);
+  return N == 64 && Dh == 64 && BH >= 256;
+}
+
+size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
+  int S, cps;
+  segments(B * H, nC, Dh, S, cps);
+  return ws_bytes(B * H, Dh, N, S);
+}
+
+int walk_fwd(const ChunkArgs& a, int64_t B, hipStream_t s, bool gla) {
+  FinalArgs p{};
+  p.u = a.u;
+  p.step = a.delta;
+  p.Bm = a.Bm;
+  p.Cm = a.Cm;
+  p.A = a.A;
+  p.h0 = a.h0;
+  p.y = a.y;
+  p.fin = a.ckpt;
+  p.L = a.L; p.H = a.H; p.nC = a.nC;
+  const size_t wsb = walk_ws_bytes(B, a.H, a.nC, a.DH, a.NS);
+  if (gla) return run<true, kCkpt>(p, B, a.H, a.DH, a.NS, a.ws, wsb, s);
+  return run<false, kCkpt>(p, B, a.H, a.DH, a.NS, a.ws, wsb, s);
+}
+
+}  // namespace rr
 
 extern "C" int64_t rr_ssd_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
                                                 int64_t A_stride_n, int dtype) {
@@ -589,7 +681,7 @@ extern "C" int rr_ssd_final_fwd(const void* u, const void* delta, const void* Bm
   p.y = y;
   p.fin = fin;
   p.L = (int)L; p.H = (int)H; p.nC = (int)((L + Q - 1) / Q);
-  return run<false>(p, B, H, Dh, N, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  return run<false, kFinal>(p, B, H, Dh, N, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int64_t rr_gla_final_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t seg, int dtype) {
@@ -613,5 +705,5 @@ extern "C" int rr_gla_final_fwd(const void* q, const void* k, const void* v, con
   p.y = y;
   p.fin = fin;
   p.L = (int)L; p.H = (int)H; p.nC = (int)((L + Q - 1) / Q);
-  return run<true>(p, B, H, Dh, Dh, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  return run<true, kFinal>(p, B, H, Dh, Dh, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }

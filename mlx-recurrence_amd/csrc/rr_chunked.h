@@ -186,7 +186,9 @@ __device__ __forceinline__ int state_off(int d, int n) {
 //           scan: one workgroup per run of R = 2 or 4 consecutive chunks;
 //           the scan stores the adjoint leaving every R-th chunk only, and
 //           the workgroup carries it across the run's inner boundaries.
-enum Mode { kWhole = 0, kPipe = 1, kDirect = 2, kSum = 3, kRes = 4, kPair = 5 };
+//   kWalk   forward only: a head's chunks walked by one workgroup per segment,
+//           waves that own rows of the state (final_fwd.hip).
+enum Mode { kWhole = 0, kPipe = 1, kDirect = 2, kSum = 3, kRes = 4, kPair = 5, kWalk = 6 };
 
 // Per-chunk kernels run on a 1-D grid of chunk_grid(p) workgroups.  The GPU
 // hands workgroups to its 8 XCDs round-robin by linear index; the decode

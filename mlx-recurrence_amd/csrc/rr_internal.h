@@ -90,6 +90,14 @@ int gla2_bwd(const ChunkArgs& p, int64_t B, hipStream_t s);
 bool res_fwd_supported(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
 int res_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 
+// Forward with a head's chunks walked by one workgroup per segment
+// (final_fwd.hip), writing every checkpoint: Dh in {32, 64, 128}, N in
+// {16, 32, 64, 128} (GLA: N = Dh).  p.ws holds walk_ws_bytes bytes (the
+// segments' maps; none for one segment).
+bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla);   // faster than the other modes
+size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
+int walk_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
+
 // Gated DeltaNet forward in chunkwise (WY) form (gdn_chunk.hip): bf16, Dh 64,
 // checkpoint interval 32; the workspace holds every chunk's operand fragments.
 bool gdn_chunk_supported(int dtype, int64_t Dh, int64_t T);

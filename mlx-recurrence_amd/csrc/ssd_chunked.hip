@@ -54,6 +54,7 @@ bool ssd2_supported(int dtype, int64_t L, int64_t seg, int64_t Dh, int64_t N, in
 
 int ssd2_fwd(const ChunkArgs& p, int64_t B, hipStream_t s) {
   if (p.mode == kRes) return res_fwd(p, B, s, false);
+  if (p.mode == chunked::kWalk) return walk_fwd(p, B, s, false);
   switch (p.DH * 1000 + p.NS) {
     case 32016: return chunked::launch_fwd<32, 16, false>(p, B, s);
     case 32032: return chunked::launch_fwd<32, 32, false>(p, B, s);
@@ -868,6 +869,7 @@ int chunked_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N, int pa
   // stays per chunk (measured on MI355X, fwd / bwd µs, whole-head vs per chunk:
   // B96 L512 H12 Dh64 N16 137 / 414 vs 194 / 357 (sum mode); B8 L4096 H80
   // Dh64 N128 2308 / 7457 vs 4025 / 4873 (pipelined)).
+  if (pass == 0 && walk_preferred(B * H, nC, Dh, N, false)) return chunked::kWalk;
   if (B * H >= 512 && pass == 0) return chunked::kWhole;
   if (wide_direct(B, H, nC, Dh, N)) return chunked::kDirect;
   // Short heads: the forward holds all chunks of a head in one workgroup per
@@ -910,6 +912,7 @@ bool adjoint_slots(int mode, int64_t Dh, int64_t N) {
 }  // namespace
 
 size_t ssd2_ws_bytes(int64_t B, int64_t H, int64_t nC, int mode, int64_t Dh, int64_t N, int pass) {
+  if (mode == chunked::kWalk) return walk_ws_bytes(B, H, nC, Dh, N);
   const int64_t R = chunked_run(mode, nC), nR = (nC + R - 1) / R;
   const bool pipe = mode == chunked::kPipe || mode == chunked::kPair;
   int64_t f = pipe ? align64(B * H * nC) : 0;
@@ -925,6 +928,7 @@ void ssd2_carve_ws(ChunkArgs& a, void* ws, int64_t B, int pass) {
   const int64_t nR = (a.nC + a.R - 1) / a.R;
   const bool pipe = a.mode == chunked::kPipe || a.mode == chunked::kPair;
   a.tot = a.ws = a.agg = nullptr;
+  if (a.mode == chunked::kWalk) { a.ws = f; return; }
   if (pipe) { a.tot = f; f += align64(B * a.H * a.nC); }
   if (pass == 1) {
     a.ws = f; f += align64(B * a.H * nR * a.NS);
@@ -945,6 +949,7 @@ int64_t ssd2_ws_extent(int64_t B, int64_t H, int64_t nC, int mode, int64_t Dh, i
     if (region == nullptr) return;
     ext = std::max<int64_t>(ext, reinterpret_cast<const char*>(region + first + count) - base);
   };
+  if (mode == kWalk) return (int64_t)walk_ws_bytes(B, H, nC, Dh, N);   // (its maps fill it)
   const int64_t state = Dh * N, BH = B * H;
   const bool pipe = mode == kPipe || mode == kPair;
   if (pipe && BH < kScanMinHeads) {

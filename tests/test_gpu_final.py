@@ -1,6 +1,7 @@
-"""The forward that keeps no checkpoints (final_fwd.hip: calls without a
-gradient, bf16, one decay rate per head for SSD) against the float64 oracle and
-against the general path, at the edges of its chunks and segments (MI355X only).
+"""The walking forward (final_fwd.hip: bf16, one decay rate per head for SSD; in
+calls without a gradient it keeps no checkpoints) against the float64 oracle
+and against the general path, at the edges of its chunks and segments (MI355X
+only).
 
 Bar: it works to fp32 accuracy (three-term bf16 splits, fp32 accumulation), so
 outputs are held to the fp32 bar, 1e-5 of the largest value."""
@@ -40,9 +41,9 @@ def _gla(B, L, H, Dh, seed):
 # every Dh and N, several segments (1000 and 2040 steps of few heads), T = 32
 SSD = [(1, 1, 2, 32, 16, 1), (2, 31, 1, 64, 128, 31), (1, 33, 3, 128, 32, 11), (2, 40, 5, 32, 64, 8),
        (1, 100, 3, 64, 64, 4), (2, 1000, 3, 64, 16, 8), (1, 2040, 2, 32, 128, 8), (1, 520, 2, 128, 128, 8),
-       (1, 72, 2, 128, 16, 24), (1, 77, 2, 32, 32, 7), (3, 544, 2, 64, 128, 32), (1, 768, 1, 64, 32, 32)]
+       (1, 72, 2, 128, 16, 24), (1, 77, 2, 32, 32, 7), (3, 544, 8, 64, 128, 32), (1, 768, 24, 64, 32, 32)]
 GLA = [(1, 1, 2, 64, 1), (2, 31, 1, 32, 31), (1, 33, 3, 128, 11), (1, 1000, 2, 64, 8), (2, 520, 1, 128, 8),
-       (1, 100, 3, 32, 20), (1, 544, 2, 64, 32)]
+       (1, 100, 3, 32, 20), (1, 544, 24, 64, 32)]
 
 
 @pytest.mark.parametrize("h0", [False, True])
@@ -73,6 +74,44 @@ def test_gla_final(B, L, H, Dh, seg, h0):
     rep = {}
     check("y", y, y_o, TOL[F32], rep)
     check("final", fs, fs_o, TOL[F32], rep)
+    print(rep, flush=True)
+
+
+# training calls whose forward walks (17 chunks: several segments, an odd one
+# last; 64 chunks of more heads: fewer segments), every Dh with its widest N
+WALKS = [("ssd", 1, 544, 24, 64, 64), ("ssd", 2, 544, 12, 64, 128), ("ssd", 1, 576, 24, 32, 128),
+         ("ssd", 1, 544, 24, 128, 128), ("ssd", 1, 1024, 24, 64, 16), ("gla", 1, 544, 24, 64, 64),
+         ("gla", 2, 544, 12, 128, 128), ("gla", 3, 2048, 24, 32, 32), ("ssd", 1, 128, 24, 64, 128)]
+
+
+@pytest.mark.parametrize("kind,B,L,H,Dh,N", WALKS)
+def test_walking_training_forward(kind, B, L, H, Dh, N):
+    """y and the checkpoints (the state after every chunk) of rr_ssd_fwd and
+    rr_gla_fwd where they walk."""
+    print(f"[case] walk {kind} B={B} L={L} H={H} Dh={Dh} N={N}", flush=True)
+    ins, st = _ssd(B, L, H, Dh, N, 3) if kind == "ssd" else _gla(B, L, H, Dh, 3)
+    y = torch.empty((B, L, H, Dh), device=st.device)
+    ckpt = torch.full((B, H, L // 32, Dh, N), float("nan"), device=st.device)
+    if kind == "ssd":
+        ws = _lib.ssd_workspace(B, L, H, Dh, N, 32, 0, BF16, 0, st.device)
+        _lib.ssd_fwd(*ins, 0, st, 32, y, ckpt, ws)
+        ref = [rounded(t) for t in ins]
+        ref[4] = np.repeat(ref[4][:, None], N, axis=1)
+        fwd = orc.ssd_forward
+    else:
+        ws = _lib.gla_workspace(B, L, H, Dh, 32, BF16, 0, st.device)
+        _lib.gla_fwd(*ins, st, 32, y, ckpt, ws)
+        ref = [rounded(t) for t in ins]
+        fwd = orc.gla_forward
+    rep = {}
+    y_o, fs_o = fwd(*ref, rounded(st))
+    check("y", y, y_o, TOL[F32], rep)
+    for c in (0, 1, L // 64, L // 32 - 1):
+        cut = [r[:, :32 * (c + 1)] if r.ndim >= 3 else r for r in ref]
+        _, h = fwd(*cut, rounded(st))
+        got = ckpt[:, :, c] if kind == "ssd" else ckpt[:, :, c].transpose(-1, -2)
+        check(f"ckpt {c}", got, h, TOL[F32], rep)
+    assert not torch.isnan(ckpt).any()
     print(rep, flush=True)
 
 
