@@ -100,10 +100,19 @@ int64_t rr_tile_schedule(int scan, int pass, int64_t B, int64_t L, int64_t D, in
 size_t rr_ssd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N,
                               int64_t seg, int64_t A_stride_n, int dtype, int pass);
 
-/* One past the largest workspace byte that the chunked (MFMA) SSD kernels of
+/* What rr_ssd_bwd needs of that for these arguments: at most
+ * rr_ssd_workspace_bytes(..., pass = 1), which has room for the adjoint of every
+ * chunk or pair of chunks, and far less where the backward walks a head's
+ * chunks with the adjoint in registers (long heads, Dh and N 64 or 128). */
+size_t rr_ssd_bwd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N,
+                                  int64_t seg, int64_t A_stride_n, int dtype);
+
+/* One past the largest workspace byte that the per-chunk (MFMA) SSD kernels of
  * this call write or read: the library walks the grids of the pass's kernels
  * with their own workgroup decode and slot arithmetic.  For tests that the
- * kernels stay inside rr_ssd_workspace_bytes.  No reference counterpart.
+ * kernels stay inside rr_ssd_workspace_bytes.  (For calls whose backward walks
+ * a head's chunks instead it bounds the per-chunk kernels they would take
+ * otherwise.)  No reference counterpart.
  * Returns -1 for invalid arguments or a call that the chunked bf16 kernels do
  * not run (the fp32-MFMA and VALU paths carve fixed regions of the size
  * rr_ssd_workspace_bytes returns). */

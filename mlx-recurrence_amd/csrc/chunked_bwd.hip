@@ -1,5 +1,6 @@
 // chunked_bwd.hip — backward of the chunked scans (rr_chunked.h) with the
-// state blocks owned by columns: GLA (any size) and SSD with N >= 64.
+// state blocks owned by columns, per chunk: GLA and SSD with N >= 64, where
+// walk_bwd.hip does not take them (few chunks in all, Dh or N 32).
 //
 // Per 32-step chunk (reference adjoints ssd.py:203-268, gla.py:184-236 in
 // matrix form), with h_in the state entering the chunk (forward checkpoint),

@@ -44,6 +44,7 @@ constexpr int64_t kGlaWholeBwdMaxChunks = 16;
 
 int gla2_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass) {
   if (pass == 0 && walk_preferred(B * H, nC, Dh, Dh, true)) return chunked::kWalk;
+  if (pass == 1 && walk_bwd_preferred(B * H, nC, Dh, Dh)) return chunked::kWalk;
   if (B * H >= kGlaWholeMinHeads && (pass == 0 || nC <= kGlaWholeBwdMaxChunks)) return chunked::kWhole;
   if (pass == 0 && res_fwd_supported(B, H, nC, Dh, Dh)) return chunked::kRes;   // short heads, resident
   if (Dh * Dh > chunked::kDirectMaxState)   // Dh 128: the wide direct mode (direct_sum_wide) while resident
@@ -55,7 +56,8 @@ int gla2_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass) {
 
 size_t gla2_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass) {
   const int mode = gla2_mode(B, H, nC, Dh, pass);
-  if (mode == chunked::kWalk) return walk_ws_bytes(B, H, nC, Dh, Dh);
+  if (mode == chunked::kWalk)
+    return pass == 0 ? walk_ws_bytes(B, H, nC, Dh, Dh) : walk_bwd_ws_floats(B * H, nC, Dh, Dh) * sizeof(float);
   if (mode == chunked::kDirect && Dh * Dh > chunked::kDirectMaxState)   // wide: the backward's adjoints
     return pass == 1 ? (size_t)align64(B * H * nC * Dh * Dh) * sizeof(float) : 0;
   if (mode == chunked::kDirect || mode == chunked::kWhole || mode == chunked::kRes) return 0;
@@ -67,7 +69,11 @@ size_t gla2_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass) {
 void gla2_carve_ws(ChunkArgs& a, void* ws, int64_t B, int pass) {
   float* f = static_cast<float*>(ws);
   a.ws = a.tot = a.agg = nullptr;
-  if (a.mode == chunked::kWalk) { a.ws = f; return; }
+  if (a.mode == chunked::kWalk) {
+    a.ws = pass == 0 ? f : nullptr;
+    a.agg = pass == 1 ? f : nullptr;
+    return;
+  }
   if (a.mode == chunked::kDirect && a.DH * a.DH > chunked::kDirectMaxState) {   // wide: the backward's adjoints
     a.agg = pass == 1 ? f : nullptr;
     return;
@@ -89,6 +95,9 @@ int gla2_fwd(const ChunkArgs& p, int64_t B, hipStream_t s) {
   }
 }
 
-int gla2_bwd(const ChunkArgs& p, int64_t B, hipStream_t s) { return chunked_bwd_cols(p, B, s, true); }
+int gla2_bwd(const ChunkArgs& p, int64_t B, hipStream_t s) {
+  if (p.mode == chunked::kWalk) return walk_bwd(p, B, s, true);
+  return chunked_bwd_cols(p, B, s, true);
+}
 
 }  // namespace rr

@@ -98,6 +98,18 @@ bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla);   
 size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
 int walk_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 
+// Backward with a head's chunks walked, the adjoint in registers
+// (walk_bwd.hip): Dh and N in {64, 128} (GLA: N = Dh).  SSD leaves one dA partial per
+// segment of walk_bwd_chunks chunks in p.ws; p.agg holds walk_bwd_ws_floats
+// floats (the segments' adjoint maps; none for one segment).
+bool walk_bwd_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N);   // covered, and faster than the other modes
+int walk_bwd_chunks(int64_t BH, int64_t nC, int64_t Dh, int64_t N);
+size_t walk_bwd_ws_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N);
+int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
+// The SSD backward by that kernel and its dA reduction, and its workspace.
+size_t ssd2_walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
+int ssd2_walk_bwd(ChunkArgs& p, void* ws, int64_t B, hipStream_t s);
+
 // Gated DeltaNet forward in chunkwise (WY) form (gdn_chunk.hip): bf16, Dh 64,
 // checkpoint interval 32; the workspace holds every chunk's operand fragments.
 bool gdn_chunk_supported(int dtype, int64_t Dh, int64_t T);

@@ -992,6 +992,21 @@ int64_t ssd2_ws_extent(int64_t B, int64_t H, int64_t nC, int mode, int64_t Dh, i
   return ext;
 }
 
+size_t ssd2_walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
+  const int64_t R = walk_bwd_chunks(B * H, nC, Dh, N), nR = (nC + R - 1) / R;
+  return ((size_t)align64(B * H * nR * N) + walk_bwd_ws_floats(B * H, nC, Dh, N)) * sizeof(float);
+}
+
+int ssd2_walk_bwd(ChunkArgs& p, void* ws, int64_t B, hipStream_t s) {
+  p.mode = chunked::kWalk;
+  p.R = walk_bwd_chunks(B * p.H, p.nC, p.DH, p.NS);
+  const int64_t nR = (p.nC + p.R - 1) / p.R;
+  p.ws = static_cast<float*>(ws);
+  p.agg = p.ws + align64(B * p.H * nR * p.NS);
+  if (int rc = walk_bwd(p, B, s, false)) return rc;
+  return launch_dA(p, B, s);
+}
+
 int ssd2_bwd(const ChunkArgs& p, int64_t B, hipStream_t s) {
   switch (p.DH * 1000 + p.NS) {
     case 32016: return launch_bwd<32, 16>(p, B, s);

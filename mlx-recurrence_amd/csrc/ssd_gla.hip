@@ -996,6 +996,15 @@ extern "C" size_t rr_ssd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_
   return pass == 0 ? q.fwd_bytes : q.bwd_bytes;
 }
 
+extern "C" size_t rr_ssd_bwd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
+                                             int64_t A_stride_n, int dtype) {
+  if (B <= 0 || L <= 0 || H <= 0 || Dh <= 0 || N <= 0 || rr::chunk_len(L, seg) == 0) return 0;
+  if (rr::ssd2_supported(dtype, L, seg, Dh, N, A_stride_n) && rr::ssd2_bwd_supported(Dh, N) &&
+      rr::walk_bwd_preferred(B * H, L / 32, Dh, N))
+    return rr::ssd2_walk_ws_bytes(B, H, L / 32, Dh, N);
+  return rr_ssd_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype, 1);
+}
+
 extern "C" int64_t rr_ssd_workspace_extent(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
                                            int64_t A_stride_n, int dtype, int pass) {
   if (B <= 0 || L <= 0 || H <= 0 || Dh <= 0 || N <= 0 || rr::chunk_len(L, seg) == 0 || (pass != 0 && pass != 1)) {
@@ -1085,8 +1094,10 @@ extern "C" int rr_ssd_bwd(const float* dy, const float* dfinal, const void* u, c
     return rr::fail(RR_EINVAL, "ssd_bwd: dA_stride_n must be 0 or 1");
   if (rr::ssd2_supported(dtype, L, seg, Dh, N, A_stride_n) && rr::ssd2_bwd_supported(Dh, N)) {
     const int nC = (int)(L / 32);
-    const int mode = rr::chunked_mode(B, H, nC, Dh, N, 1);
-    if (!workspace || workspace_bytes < rr::ssd2_ws_bytes(B, H, nC, mode, Dh, N, 1))
+    const bool walk = rr::walk_bwd_preferred(B * H, nC, Dh, N);
+    const int mode = walk ? -1 : rr::chunked_mode(B, H, nC, Dh, N, 1);
+    if (!workspace || workspace_bytes < (walk ? rr::ssd2_walk_ws_bytes(B, H, nC, Dh, N)
+                                              : rr::ssd2_ws_bytes(B, H, nC, mode, Dh, N, 1)))
       return rr::fail(RR_EWORKSPACE, "ssd_bwd: workspace too small");
     rr::ChunkArgs a{};
     a.u = static_cast<const uint16_t*>(u);
@@ -1107,6 +1118,7 @@ extern "C" int rr_ssd_bwd(const float* dy, const float* dfinal, const void* u, c
     a.dA_sn = (int)dA_stride_n;
     a.dh0 = dh0;
     a.B = (int)B; a.L = (int)L; a.H = (int)H; a.DH = (int)Dh; a.NS = (int)N; a.nC = nC;
+    if (walk) return rr::ssd2_walk_bwd(a, workspace, B, static_cast<hipStream_t>(stream));
     a.mode = mode;
     a.R = rr::chunked_run(mode, nC);
     rr::ssd2_carve_ws(a, workspace, B, 1);

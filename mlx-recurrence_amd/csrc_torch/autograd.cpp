@@ -198,7 +198,7 @@ struct SSDFn : public torch::autograd::Function<SSDFn> {
     const at::ScalarType dt = u_.scalar_type();
     const int64_t es = (int64_t)c10::elementSize(dt);
     const int dtc = dtype_code(dt);
-    const size_t wsb = rr_ssd_workspace_bytes(Bsz, L, H, Dh, N, seg, a_sn, dtc, 1);
+    const size_t wsb = rr_ssd_bwd_workspace_bytes(Bsz, L, H, Dh, N, seg, a_sn, dtc);
     const bool heads = ctx->saved_data["a_dim"].toInt() == 1;   // A_neg [H]: its gradient sums dA over n
     Arena ar;   // du, ddelta, dB, dC in the inputs' dtype
     const int64_t odu = ar.reserve(u_.numel() * es), odd = ar.reserve(d_.numel() * es);

@@ -43,6 +43,7 @@ _SIGS = {
     "rr_async_status": (_c_int, []),
     "rr_tile_schedule": (_c_i64, [_c_int, _c_int] + [_c_i64] * 4 + [_c_int] + [_c_ptr] * 3 + [_c_i64]),
     "rr_ssd_workspace_bytes": (_c_size, [_c_i64] * 7 + [_c_int, _c_int]),
+    "rr_ssd_bwd_workspace_bytes": (_c_size, [_c_i64] * 7 + [_c_int]),
     "rr_ssd_workspace_extent": (_c_i64, [_c_i64] * 7 + [_c_int, _c_int]),
     "rr_ssd_fwd": (_c_int, [_c_ptr] * 5 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 4 + [_c_size, _c_ptr]),
     "rr_ssd_bwd": (_c_int, [_c_ptr] * 7 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 7 + [_c_i64]
@@ -264,6 +265,11 @@ def _alloc_ws(n: int, device) -> torch.Tensor | None:
 def ssd_workspace(B, L, H, Dh, N, seg, a_stride_n, dtype, pass_, device) -> torch.Tensor | None:
     n = _ws_bytes("rr_ssd_workspace_bytes", (B, L, H, Dh, N, seg, a_stride_n, DTYPE_CODE[dtype], pass_))
     return _alloc_ws(n, device)
+
+
+def ssd_bwd_workspace(B, L, H, Dh, N, seg, a_stride_n, dtype, device) -> torch.Tensor | None:
+    """The backward's workspace at the size this call needs (ssd_workspace(pass_=1) is at least that)."""
+    return _alloc_ws(_ws_bytes("rr_ssd_bwd_workspace_bytes", (B, L, H, Dh, N, seg, a_stride_n, DTYPE_CODE[dtype])), device)
 
 
 def ssd_fwd(u, delta, Bm, Cm, A, a_stride_n, h0, seg, y, ckpt, ws):

@@ -100,7 +100,7 @@ class _SSDScan(torch.autograd.Function):
         dA = torch.empty((H,) if ctx.a_dim == 1 else (H, N), dtype=torch.float32, device=dev)
         dh0 = torch.empty((Bsz, H, Dh, N), dtype=torch.float32, device=dev) if ctx.needs_input_grad[5] else None
         with _lib.device_guard(dev):
-            ws = _lib.ssd_workspace(Bsz, L, H, Dh, N, ctx.seg, ctx.a_sn, u_.dtype, 1, dev)
+            ws = _lib.ssd_bwd_workspace(Bsz, L, H, Dh, N, ctx.seg, ctx.a_sn, u_.dtype, dev)
             _lib.ssd_bwd(dy, dfinal, u_, d_, B_, C_, A_, ctx.a_sn, h0_, ckpt, ctx.seg, du, dd, dB, dC, dA, dh0, ws)
         return du, dd, dB, dC, dA, dh0, None, None
 

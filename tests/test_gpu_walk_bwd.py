@@ -1,0 +1,63 @@
+"""The walking backward (walk_bwd.hip) against the float64 oracle at the least
+chunk counts that take it, with an initial state and a final-state cotangent:
+one to many segments, an uneven last one, every Dh x N; GLA with gates of either
+sign and resets (MI355X only).  Bars: those of tests/gpu_util.py (bf16
+gradients: storage rounding; fp32 outputs 1e-4)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import mlx_recurrence_amd as mr
+from oracle import recurrence_oracle as orc
+from tests.gpu_util import TOL, check, rounded, to_dev
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+CASES = [  # kind, B, L, H, Dh, N
+    ("ssd", 1, 2944, 12, 64, 64),      # 92 chunks of 12 heads: many segments
+    ("ssd", 2, 1504, 12, 64, 128),     # 47 chunks, an uneven last segment
+    ("ssd", 1, 1504, 24, 128, 64),
+    ("ssd", 5, 128, 56, 64, 128),      # 4 chunks of 280 heads: one segment
+    ("ssd", 3, 64, 184, 128, 128),     # 2 chunks
+    ("gla", 1, 2944, 12, 64, 64),
+    ("gla", 4, 160, 55, 64, 64),
+    ("gla", 1, 1504, 24, 128, 128),
+]
+
+
+@pytest.mark.parametrize("kind,B,L,H,Dh,N", CASES)
+def test_walk_bwd(kind, B, L, H, Dh, N):
+    print(f"[case] walk_bwd {kind} B={B} L={L} H={H} Dh={Dh} N={N}", flush=True)
+    rng = np.random.default_rng(L + N)
+    h0 = to_dev(rng.standard_normal((B, H, Dh, N)), F32, True)
+    W = rng.standard_normal((B, L, H, Dh)).astype(np.float32).astype(np.float64)
+    Wf = rng.standard_normal((B, H, Dh, N)).astype(np.float32).astype(np.float64)
+    if kind == "ssd":
+        xs = [to_dev(rng.standard_normal((B, L, H, Dh)), BF16, True),
+              to_dev(np.abs(rng.standard_normal((B, L, H))) * 0.1 + 0.01, BF16, True),
+              to_dev(rng.standard_normal((B, L, H, N)), BF16, True), to_dev(rng.standard_normal((B, L, H, N)), BF16, True),
+              to_dev(-np.exp(rng.uniform(0, np.log(16), H)), F32, True)]
+        y, fs = mr.ssd_scan_with_state(*xs, initial_state=h0)
+        ref = [rounded(t) for t in xs]
+        ref[4] = np.repeat(ref[4][:, None], N, axis=1)
+        grads = list(orc.ssd_backward(W, *ref, rounded(h0), Wf))
+        grads[4] = grads[4].sum(1)
+        names = ["u", "delta", "B", "C", "A"]
+    else:
+        g = 1 / (1 + np.exp(-(rng.standard_normal((B, L, H)) + 2)))
+        g[:, L // 2] *= -1
+        g[:, 5:7] *= -1
+        g[:, L // 3] = 0
+        xs = [to_dev(rng.standard_normal((B, L, H, Dh)) / np.sqrt(Dh), BF16, True) for _ in range(3)]
+        xs.append(to_dev(g, BF16, True))
+        y, fs = mr.gla_scan_with_state(*xs, initial_state=h0)
+        grads = list(orc.gla_backward(W, *[rounded(t) for t in xs], rounded(h0), Wf))
+        names = ["q", "k", "v", "g"]
+    ((y * to_dev(W, F32)).sum() + (fs * to_dev(Wf, F32)).sum()).backward()
+    rep = {}
+    for name, t, want in zip(names + ["h0"], xs + [h0], grads):
+        check("grad_" + name, t.grad, want, TOL[BF16], rep)
+    print(rep, flush=True)
