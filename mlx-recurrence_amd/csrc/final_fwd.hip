@@ -41,10 +41,12 @@
 // spill 18 and take 178 us.  With checkpoints the traffic: B8 L4096 H80 Dh64
 // N128 1224 us, 4.4 TB/s; B8 L2048 H12 GLA Dh128 448 -> 215 us.
 #include "rr_chunked.h"
+#include "rr_frag.h"
 
 namespace {
 
 using rr::f32x4_t;
+using rr::lds_barrier;
 using rr::u16x4_t;
 using rr::u16x8_t;
 
@@ -77,13 +79,6 @@ __device__ __forceinline__ void split3(const float (&x)[8], u16x8_t& hi, u16x8_t
   hi = __builtin_bit_cast(u16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
   mid = __builtin_bit_cast(u16x8_t, make_uint4(m[0], m[1], m[2], m[3]));
   lo = __builtin_bit_cast(u16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
-}
-
-// Workgroup barrier ordering LDS only: loads and stores to memory stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // LDS images of one chunk.  16-byte units of a row are permuted by row (xor)

@@ -669,7 +669,7 @@ extern "C" int rr_gdn_bwd(const float* dy, const float* dfinal, const void* q, c
     if (chunked) {
       void* packs = static_cast<char*>(workspace) + align256(adj_bytes(B, L, H, Dh, seg));
       if (int rc = rr::gdn_chunk_adjoint(q, k, v, alpha, beta, dy, dfinal, B, L, H, adjck, dh0, packs, s)) return rc;
-      if (int rc = rr::gdn_chunk_grad(dy, q, k, v, alpha, beta, h0, ckpt, adjck, dq, dk, dv, dalpha, dbeta, B, L, H, s))
+      if (int rc = rr::gdn_chunk_grad(dy, q, k, v, alpha, beta, h0, ckpt, adjck, packs, dq, dk, dv, dalpha, dbeta, B, L, H, s))
         return rc;
     } else if (Dh == 64)
       launch_bwd_dh<InT, 64>(T, dy, dfinal, q, k, v, alpha, beta, h0, ckpt, adjck, dq, dk, dv, dalpha, dbeta, dh0, B,

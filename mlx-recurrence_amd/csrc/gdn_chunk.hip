@@ -31,6 +31,7 @@
 // split into bf16 hi + lo halves (three products), bf16 inputs are exact.
 #include "rr_common.h"
 #include "rr_internal.h"
+#include "rr_frag.h"
 #include "rr_mfma.h"
 
 namespace {
@@ -38,6 +39,7 @@ namespace {
 using rr::f32x4_t;
 using rr::u16x4_t;
 using rr::u16x8_t;
+using rr::split_pair;
 
 constexpr int kQ = 32;      // steps per chunk (= checkpoint interval)
 constexpr int kD = 64;      // Dh
@@ -54,15 +56,20 @@ struct alignas(16) ChunkPack {
   float pad[kQ];
 };
 
-// The backward's fragments of a chunk (kernel 1 in its backward mode ->
-// the reverse state pass): the transposed products of the adjoint
-//   dU = P^T dO + Kbar dS_out,
-//   dS_in = gam_31 dS_out + (diag(gam) Q)^T dO - W^T dU.
+// The backward's fragments of a chunk (kernel 1 in its backward mode -> the
+// reverse state pass).  With E = T^T dU, dU = P^T dO + Kbar dS_out, and W = T
+// diag(beta gam) K the adjoint is
+//   E = (P T)^T dO + (T^T Kbar) dS_out,
+//   dS_in = gam_31 dS_out + (diag(gam) Q)^T dO - (diag(beta gam) K)^T E,
+// so neither dU nor W is formed; the reverse pass leaves E for the gradient
+// pass, which needs dU only through it.
 struct alignas(16) BwdPack {
-  uint4 Pt[2][2][64];      // [rb][hi, lo]: P^T[16 rb + m][pi] = P[pi][16 rb + m]
-  uint4 Kb[2][2][2][64];   // [rb][kb][hi, lo]: Kbar[16 rb + m][32 kb + pi]
+  uint4 Pt[2][2][64];      // [rb][hi, lo]: (P T)^T[16 rb + m][pi]
+  uint4 Kb[2][2][2][64];   // [rb][kb][hi, lo]: (T^T Kbar)[16 rb + m][32 kb + pi]
   uint4 Qg[4][2][64];      // [ib][hi, lo]: gam_pi q_pi[16 ib + m]
-  uint4 Wn[4][2][64];      // [ib][hi, lo]: -W[pi][16 ib + m]
+  uint4 Wn[4][2][64];      // [ib][hi, lo]: -beta_pi gam_pi k_pi[16 ib + m]
+  uint4 T[2][2][64];       // [rb][hi, lo]: T[16 rb + m][pi] (gradient pass)
+  float E[kQ][kD];         // written by the reverse pass
   float gend;
   float pad[63];
 };
@@ -221,11 +228,11 @@ __global__ __launch_bounds__(64) void gdn_wy_kernel(const uint16_t* __restrict__
   }
   __syncthreads();
 
-  // W = T diag(beta gam) K, U0 = T diag(beta) V: A operand T rows (k = c),
-  // column factors applied before the split; B operands by transposing reads
+  // forward: W = T diag(beta gam) K, U0 = T diag(beta) V: A operand T rows (k =
+  // c), column factors applied before the split; B operands by transposing reads
   ChunkPack& pk = static_cast<ChunkPack*>(packs)[(int64_t)bh * nC + c];
   BwdPack& bp = static_cast<BwdPack*>(packs)[(int64_t)bh * nC + c];
-  {
+  if constexpr (!BWD) {
     u16x8_t tw[2][2], tu[2][2];   // [rb][hi, lo]
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -253,52 +260,88 @@ __global__ __launch_bounds__(64) void gdn_wy_kernel(const uint16_t* __restrict__
         w = mfma(tw[rb][1], kf, w);
 #pragma unroll
         for (int r = 0; r < 4; ++r) sm.w[16 * rb + 4 * g + r][16 * nb + l15] = w[r];
-        if constexpr (!BWD) {
-          f32x4_t u = {0.f, 0.f, 0.f, 0.f};
-          u = mfma(tu[rb][0], vf, u);
-          u = mfma(tu[rb][1], vf, u);
-          pk.U0[nb][rb][lane] = make_float4(u[0], u[1], u[2], u[3]);   // slice nb, accumulator layout
-        }
+        f32x4_t u = {0.f, 0.f, 0.f, 0.f};
+        u = mfma(tu[rb][0], vf, u);
+        u = mfma(tu[rb][1], vf, u);
+        pk.U0[nb][rb][lane] = make_float4(u[0], u[1], u[2], u[3]);   // slice nb, accumulator layout
       }
     }
   }
   __syncthreads();
 
   if constexpr (BWD) {
-    // packed A operands of the reverse state pass (k in pi order)
-    float gp[8];   // gam_t, t = pi(g, e)
+    // packed A operands of the reverse state pass (k in pi order); the products
+    // are formed transposed, so that their accumulators are those operands
+    u16x8_t th[2], tl[2], fh[2], fl[2];   // T[8 g + e][16 rb + l15], and f_c times it
+    float gp[8], bg[8];   // gam_t, beta_t gam_t at t = pi(g, e)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) gp[e] = sm.gam[pi_k(g, e)];
+    for (int e = 0; e < 8; ++e) {
+      gp[e] = sm.gam[pi_k(g, e)];
+      bg[e] = -sm.beta[pi_k(g, e)] * gp[e];
+    }
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
-      const int row = 16 * rb + l15;
-      float x[8];
+      float x[8], y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = sm.p[pi_k(g, e)][row];
-      split8(x, bp.Pt[rb][0][lane], bp.Pt[rb][1][lane]);
-      const float fr = __expf(sm.lg[kQ - 1] - sm.lg[row]);   // Kbar row factor
+      for (int e = 0; e < 8; ++e) {
+        x[e] = sm.t[8 * g + e][16 * rb + l15];
+        y[e] = x[e] * __expf(sm.lg[kQ - 1] - sm.lg[8 * g + e]);   // Kbar's row factor
+      }
+      rr::bf_split8(x, th[rb], tl[rb]);
+      rr::bf_split8(y, fh[rb], fl[rb]);
+      const float4 t0 = *reinterpret_cast<const float4*>(&sm.t[16 * rb + l15][4 * g]);
+      const float4 t1 = *reinterpret_cast<const float4*>(&sm.t[16 * rb + l15][16 + 4 * g]);
+      const float tv[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
+      split8(tv, bp.T[rb][0][lane], bp.T[rb][1][lane]);
+    }
+    f32x4_t pt[2][2];   // (P T)[16 cb + 4 g + r][16 rb + l15]
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const u16x4_t k0 = *reinterpret_cast<const u16x4_t*>(&sm.k[row][32 * kb + 4 * g]);
-        const u16x4_t k1 = *reinterpret_cast<const u16x4_t*>(&sm.k[row][32 * kb + 16 + 4 * g]);
-        const float y[8] = {fr * rr::bf_val(k0[0]), fr * rr::bf_val(k0[1]), fr * rr::bf_val(k0[2]),
-                            fr * rr::bf_val(k0[3]), fr * rr::bf_val(k1[0]), fr * rr::bf_val(k1[1]),
-                            fr * rr::bf_val(k1[2]), fr * rr::bf_val(k1[3])};
-        split8(y, bp.Kb[rb][kb][0][lane], bp.Kb[rb][kb][1][lane]);
+    for (int cb = 0; cb < 2; ++cb) {
+      const float4 p0 = *reinterpret_cast<const float4*>(&sm.p[16 * cb + l15][8 * g]);
+      const float4 p1 = *reinterpret_cast<const float4*>(&sm.p[16 * cb + l15][8 * g + 4]);
+      const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+      u16x8_t ph, pl;
+      rr::bf_split8(pv, ph, pl);
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+        x = mfma(pl, th[rb], x);
+        x = mfma(ph, tl[rb], x);
+        pt[cb][rb] = mfma(ph, th[rb], x);
       }
     }
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-      const u16x4_t lo = rr::frag4_tr(&sm.q[0][16 * ib], 72, lane);    // q[4 g + e][16 ib + m]
-      const u16x4_t hi = rr::frag4_tr(&sm.q[16][16 * ib], 72, lane);   // q[16 + 4 g + e][..]
-      const float x[8] = {gp[0] * rr::bf_val(lo[0]), gp[1] * rr::bf_val(lo[1]), gp[2] * rr::bf_val(lo[2]),
-                          gp[3] * rr::bf_val(lo[3]), gp[4] * rr::bf_val(hi[0]), gp[5] * rr::bf_val(hi[1]),
-                          gp[6] * rr::bf_val(hi[2]), gp[7] * rr::bf_val(hi[3])};
-      split8(x, bp.Qg[ib][0][lane], bp.Qg[ib][1][lane]);
-      float w[8];
+    for (int rb = 0; rb < 2; ++rb) {
+      const float x[8] = {pt[0][rb][0], pt[0][rb][1], pt[0][rb][2], pt[0][rb][3],
+                          pt[1][rb][0], pt[1][rb][1], pt[1][rb][2], pt[1][rb][3]};
+      split8(x, bp.Pt[rb][0][lane], bp.Pt[rb][1][lane]);
+    }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = -sm.w[pi_k(g, e)][16 * ib + l15];
-      split8(w, bp.Wn[ib][0][lane], bp.Wn[ib][1][lane]);
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        f32x4_t x[2];   // (T^T Kbar)^T[32 kb + 16 q + 4 g + r][16 rb + l15]
+#pragma unroll
+        for (int q2 = 0; q2 < 2; ++q2) {
+          const u16x8_t kf = rr::frag_tr(&sm.k[0][32 * kb + 16 * q2], 72, lane);   // K[8 g + e][i]
+          x[q2] = mfma(kf, fl[rb], f32x4_t{0.f, 0.f, 0.f, 0.f});
+          x[q2] = mfma(kf, fh[rb], x[q2]);
+        }
+        const float y[8] = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
+        split8(y, bp.Kb[rb][kb][0][lane], bp.Kb[rb][kb][1][lane]);
+      }
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) {
+      auto put = [&](uint16_t (*m)[72], const float (&f8)[8], uint4& hi4, uint4& lo4) {
+        const u16x4_t lo = rr::frag4_tr(&m[0][16 * ib], 72, lane);    // m[4 g + e][16 ib + l15]
+        const u16x4_t hi = rr::frag4_tr(&m[16][16 * ib], 72, lane);   // m[16 + 4 g + e][..]
+        const float x[8] = {f8[0] * rr::bf_val(lo[0]), f8[1] * rr::bf_val(lo[1]), f8[2] * rr::bf_val(lo[2]),
+                            f8[3] * rr::bf_val(lo[3]), f8[4] * rr::bf_val(hi[0]), f8[5] * rr::bf_val(hi[1]),
+                            f8[6] * rr::bf_val(hi[2]), f8[7] * rr::bf_val(hi[3])};
+        split8(x, hi4, lo4);
+      };
+      put(sm.q, gp, bp.Qg[ib][0][lane], bp.Qg[ib][1][lane]);
+      put(sm.k, bg, bp.Wn[ib][0][lane], bp.Wn[ib][1][lane]);
     }
     if (lane == 0) bp.gend = sm.gam[kQ - 1];
   } else {
@@ -372,12 +415,6 @@ __device__ __forceinline__ void load_frags(Frags& f, const ChunkPack& pk, int s,
     f.Kb[ib][1] = pk.Kb[ib][1][lane];
   }
   f.gend = pk.gam[kQ - 1];
-}
-
-// Two 16-row accumulator blocks -> bf16 hi / lo B-operand fragments (k = pi).
-__device__ __forceinline__ void split_pair(const f32x4_t& a0, const f32x4_t& a1, u16x8_t& hi, u16x8_t& lo) {
-  const float x[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-  rr::bf_split8(x, hi, lo);
 }
 
 __global__ __launch_bounds__(64) void gdn_state_kernel(const ChunkPack* __restrict__ pack, const float* __restrict__ h0,
@@ -480,7 +517,8 @@ __global__ __launch_bounds__(64) void gdn_state_kernel(const ChunkPack* __restri
 // steps as four 16-row accumulator blocks.  Per chunk it writes dS as the
 // chunk's adjoint checkpoint (before the chunk's own steps: what the
 // gradient pass starts each interval from), then
-//   dU = P^T dO + Kbar dS,   dS <- gam_31 dS + (diag(gam) Q)^T dO - W^T dU.
+//   E = (P T)^T dO + (T^T Kbar) dS (written for the gradient pass),
+//   dS <- gam_31 dS + (diag(gam) Q)^T dO - (diag(beta gam) K)^T E.
 struct BFrags {
   uint4 Pt[2][2], Kb[2][2][2], Qg[4][2], Wn[4][2];
   float gend;
@@ -512,7 +550,7 @@ __device__ __forceinline__ void load_bfrags(BFrags& f, const BwdPack& pk, const 
   for (int e = 0; e < 8; ++e) f.dO[e] = dy[((row0 + pi_k(g, e)) * H + h) * kD + j];
 }
 
-__global__ __launch_bounds__(64) void gdn_rstate_kernel(const BwdPack* __restrict__ pack, const float* __restrict__ dy,
+__global__ __launch_bounds__(64) void gdn_rstate_kernel(BwdPack* __restrict__ pack, const float* __restrict__ dy,
                                                         const float* __restrict__ dfinal, float* __restrict__ adjck,
                                                         float* __restrict__ dh0, int BH, int H, int L, int nC) {
   const int id = blockIdx.x, xcd = id % kXcd, kk = id / kXcd;
@@ -527,7 +565,7 @@ __global__ __launch_bounds__(64) void gdn_rstate_kernel(const BwdPack* __restric
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       S[ib][r] = dfinal != nullptr ? dfinal[((int64_t)bh * kD + 16 * ib + 4 * g + r) * kD + j] : 0.f;
-  const BwdPack* pk = pack + (int64_t)bh * nC;
+  BwdPack* pk = pack + (int64_t)bh * nC;
   auto row0 = [&](int c) { return (int64_t)b * L + (int64_t)c * kQ; };
   auto step = [&](const BFrags& f, int c) {
     float* ac = adjck + ((int64_t)bh * nC + c) * kD * kD;
@@ -540,7 +578,7 @@ __global__ __launch_bounds__(64) void gdn_rstate_kernel(const BwdPack* __restric
     u16x8_t sh[2], sl[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) split_pair(S[2 * kb], S[2 * kb + 1], sh[kb], sl[kb]);
-    // dU = P^T dO + Kbar dS
+    // E = (P T)^T dO + (T^T Kbar) dS
     f32x4_t U[2];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -556,9 +594,13 @@ __global__ __launch_bounds__(64) void gdn_rstate_kernel(const BwdPack* __restric
       }
       U[rb] = a;
     }
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pk[c].E[16 * rb + 4 * g + r][j] = U[rb][r];
     u16x8_t uh, ul;
     split_pair(U[0], U[1], uh, ul);
-    // dS_in = gam_31 dS + (diag(gam) Q)^T dO - W^T dU
+    // dS_in = gam_31 dS + (diag(gam) Q)^T dO - (diag(beta gam) K)^T E
     const float gend = f.gend;
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib) {
@@ -599,428 +641,345 @@ __global__ __launch_bounds__(64) void gdn_rstate_kernel(const BwdPack* __restric
 }
 
 // ------------------------------------------------------------------ kernel 4
-// The gradient pass in chunkwise form: one workgroup (8 waves) per chunk, all
+// The gradient pass in chunkwise form: one workgroup (4 waves) per chunk, all
 // chunks at once, from the forward checkpoint S_in, the adjoint checkpoint
-// dS_out and dO.  With the forward quantities above (recomputed) and
-// dU = P^T dO + Kbar dS_out:
-//   dQ = diag(gam) dO S_in^T + dQK K,   dQK = tril(R) o dP,   dP = dO U^T
-//   dK = dQK^T Q + diag(f) Kbar' + diag(beta gam) T^T dW + (dG + dG^T) K,
-//        Kbar' = U dS_out^T,  f = gam_31 / gam,  dW = -dU S_in^T
-//   dV = diag(beta) T^T dU
-//   dT = dU V^T diag(beta) + dW K^T diag(beta gam),  dA = -T^T dT T^T (strictly lower)
-//   dG = diag(beta) R o dA
-//   dbeta = rows(T^T dU o V) + gam o rows(T^T dW o K) + rows(R o G o dA)
+// dS_out, dO, and the T and E = T^T dU that the adjoint pass left.  With the
+// forward quantities above and
+//   U = T diag(beta) (V - diag(gam) K S_in):
+//   dV = diag(beta) E
+//   dQ = diag(gam) H1 + dQK K,       H1 = dO S_in^T,  dQK = tril(R) o dP,  dP = dO U^T
+//   dK = diag(f) H2 + dQK^T Q + diag(beta gam) H3 + (dG + dG^T) K,
+//        H2 = U dS_out^T,  H3 = -E S_in^T (= T^T dW),  f = gam_31 / gam
+//   dG = diag(beta) R o dA,   dA = -E U^T (strictly lower)
+// (dA = -T^T dT T^T with dT = dU (diag(beta) V)^T + dW (diag(beta gam) K)^T, dW = -dU
+// S_in^T, is -(E U0^T - E S_in^T W^T) = -E (U0 - W S_in)^T: no product with T is left),
+//   dbeta = rows(E o V) + gam o rows(H3 o K) + rows(R o G o dA)
 // and the decays through lg (gam_r = e^lg_r, R = e^(lg_r - lg_c), f):
-//   dlg = rows(E) - cols(E) + gam o (rows(dO o Q S_in) + beta o rows(T^T dW o K))
-//         - f o rows(Kbar' o K) + [r = 31] (gam_31 <dS_out, S_in> + sum f o rows(Kbar' o K)),
-//   E = (QK o dP (lower, diagonal included) + diag(beta) G o dA) o R,
+//   dlg = rows(Em) - cols(Em) + gam o (rows(Q o H1) + beta o rows(H3 o K))
+//         - f o rows(H2 o K) + [r = 31] (gam_31 <dS_out, S_in> + sum f o rows(H2 o K)),
+//   Em = P o dP + diag(beta) G o dA o R,  P = tril(R) o Q K^T,
 //   dalpha_m = (sum_{r >= m} dlg_r) / alpha_m.
-// (Derived from the chunk equations and checked in float64 against the
-// sequential adjoint before this kernel.)  Every product runs on MFMA from
-// fp32 matrices in LDS (bf16 hi / lo terms; bf16 inputs one term), its 16x16
-// output blocks dealt to the eight waves.
-constexpr int kP68 = 68, kP36 = 36;   // LDS row pitches (fp32): 64 + 4, 32 + 4
-constexpr int kGW = 8;                 // waves of a gradient workgroup
-
+//
+// Work split: wave w owns key columns i = 16 w .. 16 w + 15 (dQ, dK, H1 - H3, formed
+// transposed: S_in and dS_out rows straight from memory as A operands, 8-byte
+// stores) and value columns j = 16 w .. (its slice of U, T's product); the masked
+// 32x32 products, three nonzero 16x16 blocks in both orientations, are formed by
+// waves 0-2 and shared as operand fragments.  Four barriers; 50 KB of LDS and
+// 145 registers keep three workgroups on a CU (the kernel before this one: 20
+// dependent phases over fp32 matrices in 141 KB of LDS, one workgroup per CU).
+// B8 L2048 H12: 126 us against 480, B3 L512 H12 14 against 49; bound by the dependent chain of a
+// chunk and its reads (80 KB a chunk, half of them the two checkpoints).
+constexpr int kGradWaves = 4;
 struct alignas(16) GradSm {
-  float k[kQ][kP68], v[kQ][kP68], q[kQ][kP68], dO[kQ][kP68];
-  float sin[kD][kP68], dso[kD][kP68];
-  float u[kQ][kP68], du[kQ][kP68], w[kQ][kP68];   // U (then dK), dU, W (then dW)
-  float dq[kQ][kP68];
-  float A[kQ][kP36], T[kQ][kP36], P[kQ][kP36], G[kQ][kP36];   // P: QK, then dQK; G: G, then dG + dG^T
-  float dR[kQ][kP36], dT[kQ][kP36], X[kQ][kP36];
-  float x16[16][20];
-  float lg[kQ], gam[kQ], beta[kQ], f[kQ], al[kQ];
-  float dotp[kGW];        // per-wave partial sums of <dS_out, S_in>
-  float part[6][kQ][4];   // per-row partial sums of the elementwise reductions, [quantity][row][column block]
+  uint16_t K[kQ * kD], Q[kQ * kD], Oh[kQ * kD], Ol[kQ * kD], Eh[kQ * kD], El[kQ * kD], Uh[kQ * kD], Ul[kQ * kD];
+  uint2 QA[3][2][64], QB[3][2][64];   // dQK blocks: rows r, columns c; rows c, columns r
+  uint2 DG[4][2][64];                 // dG + dG^T, block (16 cb rows, 16 rb columns) at 2 cb + rb
+  float Em[kQ][36];
+  float lg[kQ], gam[kQ], f[kQ], beta[kQ], al[kQ];
+  float p0[kGradWaves][kQ], p1[kGradWaves][kQ], p3[kGradWaves][kQ];   // rows(Q o H1), rows(H2 o K), rows(H3 o K)
+  float p2[kQ], p4[2][kQ];            // rows(E o V), rows(R o G o dA) by column block
+  float dot[kGradWaves];              // <dS_out, S_in>
 };
 
-// Reads op(M)[row][k0 .. k0 + 7] (TR: M[k][row]) times the optional k and
-// row scales into x[8].
-template <bool TR>
-__device__ __forceinline__ void rd8(const float* M, int ld, int row, int k0, const float* ks, float rs, float (&x)[8]) {
-  if constexpr (TR) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = M[(k0 + e) * ld + row];
-  } else {
-    const float4 a = *reinterpret_cast<const float4*>(&M[row * ld + k0]);
-    const float4 b = *reinterpret_cast<const float4*>(&M[row * ld + k0 + 4]);
-    x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] *= (ks != nullptr ? ks[k0 + e] : 1.f) * rs;
-}
-
-// C = op(A) op(B) (M x N, contraction K) from LDS; each 16 x 16 block goes to
-// out(mb, nb, acc) with acc[r] = C[16 mb + 4 (lane / 16) + r][16 nb + lane % 16].
-// A: A[m][k] (TA: A[k][m]); B: B[k][n] (TB: B[n][k]); ka / kb scale the
-// contraction index of A / B, ma the rows of A; AX / BX: bf16-exact operand.
-template <int M, int N, int K, bool TA, bool TB, bool AX, bool BX, typename OUT>
-__device__ __forceinline__ void mm(const float* A, int lda, const float* B, int ldb, OUT out,
-                                   const float* ka = nullptr, const float* ma = nullptr, const float* kb = nullptr) {
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int l15 = lane & 15, g = lane >> 4;
-  constexpr int MB = M / 16, NB = N / 16, KB = K / 32;
-  for (int blk = w; blk < MB * NB; blk += kGW) {
-    const int mbk = blk / NB, nbk = blk % NB;
-    const int ar = 16 * mbk + l15, bc = 16 * nbk + l15;
-    const float rs = ma != nullptr ? ma[ar] : 1.f;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kk = 0; kk < KB; ++kk) {
-      const int k0 = 32 * kk + 8 * g;
-      float a[8], b[8];
-      rd8<TA>(A, lda, ar, k0, ka, rs, a);
-      rd8<!TB>(B, ldb, bc, k0, kb, 1.f, b);   // B[k][n]: column n of rows k0.. = transposed read
-      u16x8_t ah, al, bh, bl;
-      rr::bf_split8(a, ah, al);
-      rr::bf_split8(b, bh, bl);
-      acc = mfma(ah, bh, acc);
-      if constexpr (!BX) acc = mfma(ah, bl, acc);
-      if constexpr (!AX) acc = mfma(al, bh, acc);
-    }
-    out(mbk, nbk, acc);
-  }
-}
-
-__device__ __forceinline__ float bfv(uint16_t x) { return rr::bf_val(x); }
-
-__global__ __launch_bounds__(64 * kGW) void gdn_cgrad_kernel(const float* __restrict__ dy, const uint16_t* __restrict__ q,
-                                                        const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                                        const uint16_t* __restrict__ alpha,
-                                                        const uint16_t* __restrict__ beta, const float* __restrict__ h0,
-                                                        const float* __restrict__ ckpt, const float* __restrict__ adjck,
-                                                        uint16_t* __restrict__ dq, uint16_t* __restrict__ dk,
-                                                        uint16_t* __restrict__ dv, uint16_t* __restrict__ dalpha,
-                                                        uint16_t* __restrict__ dbeta, int BH, int H, int L, int nC) {
+__global__ __launch_bounds__(64 * kGradWaves, 3) void gdn_cgrad_kernel(
+    const float* __restrict__ dy, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, const uint16_t* __restrict__ alpha, const uint16_t* __restrict__ beta,
+    const float* __restrict__ h0, const float* __restrict__ ckpt, const float* __restrict__ adjck,
+    const BwdPack* __restrict__ packs, uint16_t* __restrict__ dq, uint16_t* __restrict__ dk,
+    uint16_t* __restrict__ dv, uint16_t* __restrict__ dalpha, uint16_t* __restrict__ dbeta, int BH, int H, int L,
+    int nC) {
+  constexpr int T = 64 * kGradWaves;
   __shared__ GradSm sm;
-  const int id = blockIdx.x, xcd = id % kXcd, kk = id / kXcd;
-  const int c = kk % nC, bh = (kk / nC) * kXcd + xcd;
+  const int id = blockIdx.x, xcd = id % kXcd, kk0 = id / kXcd;
+  const int c = kk0 % nC, bh = (kk0 / nC) * kXcd + xcd;
   if (bh >= BH) return;
   const int b = bh / H, h = bh % H;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, g = lane >> 4;
   const int64_t row0 = (int64_t)b * L + (int64_t)c * kQ;
-  const int64_t rs = (int64_t)H * kD;   // element stride of a step in [B, L, H, Dh]
-  // ---- loads: the chunk's inputs (fp32 in LDS), dO, S_in, dS_out
+  const uint32_t rs = (uint32_t)H * kD;   // element stride of a step in [B, L, H, Dh]
+  const int64_t base = (row0 * H + h) * kD;
+  const BwdPack& pk = packs[(int64_t)bh * nC + c];
+
+  // ---- every load first, unconditional (a load under a branch makes the
+  // branch's join wait for every load in flight)
+  const uint32_t o16 = (uint32_t)(tid >> 3) * rs + 8 * (tid & 7);   // row tid / 8, 8 elements
+  const u16x8_t kx = rr::ld32<u16x8_t>(k + base, o16), qx = rr::ld32<u16x8_t>(q + base, o16);
+  float4 dx[2], ex[2];
+  uint2 vx[2];
+  float bx[2];
+#pragma unroll
+  for (int z = 0; z < 2; ++z) {   // row i / 16, 4 elements
+    const int i = tid + T * z, t = i >> 4;
+    const uint32_t o = (uint32_t)t * rs + 4 * (i & 15);
+    dx[z] = rr::ld32<float4>(dy + base, o);
+    vx[z] = rr::ld32<uint2>(v + base, o);
+    ex[z] = *reinterpret_cast<const float4*>(&pk.E[t][4 * (i & 15)]);
+    bx[z] = rr::bf_val(beta[(row0 + t) * H + h]);
+  }
+  const int tq = lane & (kQ - 1);
+  const float alv = rr::bf_val(alpha[(row0 + tq) * H + h]), bev = rr::bf_val(beta[(row0 + tq) * H + h]);
+  const float* const ap = adjck + ((int64_t)bh * nC + c) * kD * kD;
+  const bool has_s = c > 0 || h0 != nullptr;
+  // S_in: checkpoint c - 1, else h0, else zero (a valid matrix read and dropped)
+  const auto sp = rr::as_global(c > 0 ? ckpt + ((int64_t)bh * nC + c - 1) * kD * kD
+                                      : (h0 != nullptr ? h0 + (int64_t)bh * kD * kD : ap));
+  // rows i = 16 w + l15 of S_in and dS_out (k = j in pi order), columns j = 16 w + l15 of S_in
+  f32x4_t sr[4], ar[4], sc[4];
+#pragma unroll
+  for (int z = 0; z < 4; ++z) {
+    const uint32_t o = (uint32_t)((16 * w + l15) * kD + 16 * z + 4 * g);
+    sr[z] = rr::ld32<f32x4_t>(sp, o);
+    ar[z] = rr::ld32<f32x4_t>(ap, o);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sc[z][r] = rr::ld32<float>(sp, (uint32_t)((16 * z + 4 * g + r) * kD + 16 * w + l15));
+  }
+  uint16_t vj[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) vj[e] = rr::ld32<uint16_t>(v + base, (uint32_t)pi_k(g, e) * rs + 16 * w + l15);
+  u16x8_t tf[2][2];   // T[16 rb + l15][pi], hi, lo
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) tf[rb][x] = as_u8(pk.T[rb][x][lane]);
+
+  // ---- stage the row images; dV and rows(E o V) straight from registers
   {
-    const uint16_t* kp = k + (row0 * H + h) * kD;
-    const uint16_t* vp = v + (row0 * H + h) * kD;
-    const uint16_t* qp = q + (row0 * H + h) * kD;
-    const float* dp = dy + (row0 * H + h) * kD;
-    // every load first, unconditional (a load under a branch makes the
-    // branch's join wait for every load in flight): the chunk's rows (32 rows
-    // x 8 pieces of 8 elements; threads >= 256 repeat rows 0-31 and drop
-    // them), S_in (checkpoint c - 1, else h0, else zero: a valid matrix read
-    // and dropped), dS_out (adjoint checkpoint c), alpha and beta
-    const int r8 = (tid >> 3) & (kQ - 1), c8 = 8 * (tid & 7);
-    const u16x8_t kx = *reinterpret_cast<const u16x8_t*>(kp + r8 * rs + c8);
-    const u16x8_t vx = *reinterpret_cast<const u16x8_t*>(vp + r8 * rs + c8);
-    const u16x8_t qx = *reinterpret_cast<const u16x8_t*>(qp + r8 * rs + c8);
-    const float4 d0 = *reinterpret_cast<const float4*>(dp + r8 * rs + c8);
-    const float4 d1 = *reinterpret_cast<const float4*>(dp + r8 * rs + c8 + 4);
-    const float* ap = adjck + ((int64_t)bh * nC + c) * kD * kD;
-    const bool has_s = c > 0 || h0 != nullptr;
-    const float* sp = c > 0 ? ckpt + ((int64_t)bh * nC + c - 1) * kD * kD
-                            : (h0 != nullptr ? h0 + (int64_t)bh * kD * kD : ap);
-    float4 sv[2], av[2];
+    auto put16 = [&](uint16_t* img, const u16x8_t& x) {
+      const uint4 u = as_u4(x);
+      *reinterpret_cast<uint2*>(img + rr::piece<kD>(tid >> 3, 2 * (tid & 7))) = make_uint2(u.x, u.y);
+      *reinterpret_cast<uint2*>(img + rr::piece<kD>(tid >> 3, 2 * (tid & 7) + 1)) = make_uint2(u.z, u.w);
+    };
+    put16(sm.K, kx);
+    put16(sm.Q, qx);
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {   // 64 x 64: 1024 float4, two passes
-      const int i = tid + 512 * it, r = i >> 4, c4 = 4 * (i & 15);
-      sv[it] = *reinterpret_cast<const float4*>(sp + r * kD + c4);
-      av[it] = *reinterpret_cast<const float4*>(ap + r * kD + c4);
+    for (int z = 0; z < 2; ++z) {
+      const int i = tid + T * z, t = i >> 4, o = rr::piece<kD>(t, i & 15);
+      u16x4_t hi, lo;
+      rr::bf_split4(f32x4_t{dx[z].x, dx[z].y, dx[z].z, dx[z].w}, hi, lo);
+      *reinterpret_cast<u16x4_t*>(sm.Oh + o) = hi;
+      *reinterpret_cast<u16x4_t*>(sm.Ol + o) = lo;
+      rr::bf_split4(f32x4_t{ex[z].x, ex[z].y, ex[z].z, ex[z].w}, hi, lo);
+      *reinterpret_cast<u16x4_t*>(sm.Eh + o) = hi;
+      *reinterpret_cast<u16x4_t*>(sm.El + o) = lo;
+      const float dv4[4] = {bx[z] * ex[z].x, bx[z] * ex[z].y, bx[z] * ex[z].z, bx[z] * ex[z].w};
+      *reinterpret_cast<uint2*>(reinterpret_cast<char*>(dv + base) + 2 * ((uint32_t)t * rs + 4 * (i & 15))) =
+          rr::pack4(dv4);
+      const float s = rr::row16_sum((ex[z].x * rr::bf4(vx[z], 0) + ex[z].y * rr::bf4(vx[z], 1)) +
+                                    (ex[z].z * rr::bf4(vx[z], 2) + ex[z].w * rr::bf4(vx[z], 3)));
+      if ((i & 15) == 0) sm.p2[t] = s;
     }
-    const int tq = tid & (kQ - 1);
-    const float alv = bfv(alpha[(row0 + tq) * H + h]), bev = bfv(beta[(row0 + tq) * H + h]);
-    if (tid < 256) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        sm.k[r8][c8 + e] = bfv(kx[e]);
-        sm.v[r8][c8 + e] = bfv(vx[e]);
-        sm.q[r8][c8 + e] = bfv(qx[e]);
-      }
-      *reinterpret_cast<float4*>(&sm.dO[r8][c8]) = d0;
-      *reinterpret_cast<float4*>(&sm.dO[r8][c8 + 4]) = d1;
-    }
-    float dot = 0.f;   // <dS_out, S_in>, this thread's share
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int i = tid + 512 * it, r = i >> 4, c4 = 4 * (i & 15);
-      float4 s4 = sv[it];
-      asm volatile("" : "+v"(s4.x), "+v"(s4.y), "+v"(s4.z), "+v"(s4.w));
-      if (!has_s) s4 = make_float4(0.f, 0.f, 0.f, 0.f);   // uniform
-      const float4 a4 = av[it];
-      *reinterpret_cast<float4*>(&sm.sin[r][c4]) = s4;
-      *reinterpret_cast<float4*>(&sm.dso[r][c4]) = a4;
-      dot += (s4.x * a4.x + s4.y * a4.y) + (s4.z * a4.z + s4.w * a4.w);
-    }
-    dot = rr::wave_sum(dot);
-    if (lane == 0) sm.dotp[w] = dot;
-    if (tid < kQ) {
+    if (w == 0) {
       const float al = fmaxf(alv, 1e-30f);   // alpha = 0 taken as 1e-30
-      sm.al[tid] = al;
-      sm.beta[tid] = bev;
-      sm.lg[tid] = __logf(al);   // prefix-summed below
-    }
-  }
-  __syncthreads();
-  if (w == 0) {
-    const float lgv = rr::prefix32_sum(sm.lg[lane & 31]);
-    rr::wave_lds_sync();
-    if (lane < kQ) {
-      sm.lg[lane] = lgv;
-      sm.gam[lane] = __expf(lgv);
-    }
-    rr::wave_lds_sync();
-    if (lane < kQ) sm.f[lane] = __expf(sm.lg[kQ - 1] - lgv);
-  }
-  __syncthreads();
-
-  // ---- G = K K^T, QK = Q K^T; A, P
-  mm<32, 32, 64, false, true, true, true>(&sm.k[0][0], kP68, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sm.G[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-  });
-  mm<32, 32, 64, false, true, true, true>(&sm.q[0][0], kP68, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sm.P[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-  });
-  __syncthreads();
-  for (int i = tid; i < kQ * kQ; i += 64 * kGW) {
-    const int r = i >> 5, cc = i & 31;
-    const float rat = __expf(cc <= r ? sm.lg[r] - sm.lg[cc] : 0.f);
-    sm.A[r][cc] = cc < r ? sm.beta[r] * rat * sm.G[r][cc] : 0.f;
-    sm.dR[r][cc] = cc <= r ? rat : 0.f;   // R on the lower triangle (kept for the decay terms)
-  }
-  __syncthreads();
-  // ---- T = (I + A)^-1 (wave 0; 16 x 16 blocks as in the WY kernel)
-  if (w == 0) {
-    const int hb = 16 * ((lane >> 4) & 1), cl = l15;
-    float tc[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float s0 = r == cl ? 1.f : 0.f, s1 = 0.f;
-#pragma unroll
-      for (int m = 0; m + 1 < r; m += 2) {
-        s0 -= sm.A[hb + r][hb + m] * tc[m];
-        s1 -= sm.A[hb + r][hb + m + 1] * tc[m + 1];
-      }
-      if (r & 1) s0 -= sm.A[hb + r][hb + r - 1] * tc[r - 1];
-      tc[r] = s0 + s1;
-    }
-    if (lane < kQ) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        sm.T[hb + r][hb + cl] = tc[r];
-        sm.T[hb + r][16 - hb + cl] = 0.f;
+      const float lg = rr::prefix32_sum(__logf(al));
+      const float l31 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lg), 31));
+      if (lane < kQ) {
+        sm.al[lane] = al;
+        sm.beta[lane] = bev;
+        sm.lg[lane] = lg;
+        sm.gam[lane] = __expf(lg);
+        sm.f[lane] = __expf(l31 - lg);
       }
     }
-    rr::wave_lds_sync();
-    const int r0 = 4 * g;
-    float xs[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const float tm = sm.T[m][l15];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xs[i] += sm.A[16 + r0 + i][m] * tm;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sm.x16[r0 + i][l15] = xs[i];
-    rr::wave_lds_sync();
-    float ts[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const float xm = sm.x16[m][l15];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ts[i] -= sm.T[16 + r0 + i][16 + m] * xm;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sm.T[16 + r0 + i][l15] = ts[i];
   }
-  // P = tril(R) o QK (each thread its own elements)
-  for (int i = tid; i < kQ * kQ; i += 64 * kGW) {
-    const int r = i >> 5, cc = i & 31;
-    sm.P[r][cc] *= sm.dR[r][cc];
+  if (!has_s) {   // uniform
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+      sr[z] = sc[z] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
   }
-  __syncthreads();
+  float dot = 0.f;
+#pragma unroll
+  for (int z = 0; z < 4; ++z)
+    dot += (sr[z][0] * ar[z][0] + sr[z][1] * ar[z][1]) + (sr[z][2] * ar[z][2] + sr[z][3] * ar[z][3]);
+  dot = rr::wave_sum(dot);
+  if (lane == 0) sm.dot[w] = dot;
+  rr::lds_barrier();
 
-  // ---- W = T diag(beta gam) K; U = T diag(beta) V - W S_in
+  const f32x4_t z4 = {0.f, 0.f, 0.f, 0.f};
+  // ---- U^T[j][r] of this wave's columns j: Y = diag(beta) (V - diag(gam) K S_in), U = T Y
   {
-    float* bgam = &sm.part[5][0][0];   // beta gam per step, 32 floats
-    if (tid < kQ) bgam[tid] = sm.beta[tid] * sm.gam[tid];
-    __syncthreads();
-    mm<32, 64, 32, false, false, false, true>(&sm.T[0][0], kP36, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+    f32x4_t ks[2] = {z4, z4};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sm.w[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-    }, bgam);
-    mm<32, 64, 32, false, false, false, true>(&sm.T[0][0], kP36, &sm.v[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+    for (int kk = 0; kk < 2; ++kk) {
+      u16x8_t sh, sl;
+      split_pair(sc[2 * kk], sc[2 * kk + 1], sh, sl);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sm.u[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-    }, sm.beta);
-    __syncthreads();
-    mm<32, 64, 64, false, false, false, false>(&sm.w[0][0], kP68, &sm.sin[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sm.u[16 * mb + 4 * g + r][16 * nb + l15] -= acc[r];
-    });
-  }
-  // rows(dO o Q S_in) -> part[0]
-  mm<32, 64, 64, false, false, true, false>(&sm.q[0][0], kP68, &sm.sin[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r;
-      const float s = rr::row16_sum(acc[r] * sm.dO[row][16 * nb + l15]);
-      if (l15 == 0) sm.part[0][row][nb] = s;
+      for (int rb = 0; rb < 2; ++rb) {
+        const u16x8_t kf = rr::row_frag<kD>(sm.K, 16 * rb + l15, kk, g);
+        ks[rb] = mfma(kf, sl, ks[rb]);
+        ks[rb] = mfma(kf, sh, ks[rb]);
+      }
     }
-  });
-  __syncthreads();
+    f32x4_t y[2];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const float4 gm = *reinterpret_cast<const float4*>(&sm.gam[16 * rb + 4 * g]);
+      const float4 be = *reinterpret_cast<const float4*>(&sm.beta[16 * rb + 4 * g]);
+      const float gv[4] = {gm.x, gm.y, gm.z, gm.w}, bv[4] = {be.x, be.y, be.z, be.w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[rb][r] = bv[r] * (rr::bf_val(vj[4 * rb + r]) - gv[r] * ks[rb][r]);
+    }
+    u16x8_t yh, yl;
+    split_pair(y[0], y[1], yh, yl);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      f32x4_t u = mfma(yl, tf[rb][0], z4);
+      u = mfma(yh, tf[rb][1], u);
+      u = mfma(yh, tf[rb][0], u);
+      u16x4_t hi, lo;
+      rr::bf_split4(u, hi, lo);
+      const int o = rr::piece<kD>(16 * rb + l15, 4 * w + g);
+      *reinterpret_cast<u16x4_t*>(sm.Uh + o) = hi;
+      *reinterpret_cast<u16x4_t*>(sm.Ul + o) = lo;
+    }
+  }
+  // ---- H1^T, -H3^T: rows i of this wave, columns r
+  f32x4_t h1[2] = {z4, z4}, h3[2] = {z4, z4}, h2[2] = {z4, z4};
+  auto prod = [&](const uint16_t* xh, const uint16_t* xl, int rb, int kk, const u16x8_t& ah, const u16x8_t& al,
+                  f32x4_t acc) {
+    const u16x8_t bh_ = rr::row_frag<kD>(xh, 16 * rb + l15, kk, g), bl = rr::row_frag<kD>(xl, 16 * rb + l15, kk, g);
+    acc = mfma(al, bh_, acc);
+    acc = mfma(ah, bl, acc);
+    return mfma(ah, bh_, acc);
+  };
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    u16x8_t sh, sl;
+    split_pair(sr[2 * kk], sr[2 * kk + 1], sh, sl);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      h1[rb] = prod(sm.Oh, sm.Ol, rb, kk, sh, sl, h1[rb]);
+      h3[rb] = prod(sm.Eh, sm.El, rb, kk, sh, sl, h3[rb]);
+    }
+  }
+  rr::lds_barrier();   // U
 
-  // ---- dU = P^T dO + Kbar dS_out
-  mm<32, 64, 32, true, false, false, false>(&sm.P[0][0], kP36, &sm.dO[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+  // ---- H2^T
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm.du[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-  });
-  __syncthreads();
-  mm<32, 64, 64, false, false, false, false>(&sm.k[0][0], kP68, &sm.dso[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+  for (int kk = 0; kk < 2; ++kk) {
+    u16x8_t ah, al;
+    split_pair(ar[2 * kk], ar[2 * kk + 1], ah, al);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm.du[16 * mb + 4 * g + r][16 * nb + l15] += acc[r];
-  }, nullptr, sm.f);
-  // dQ = diag(gam) dO S_in^T
-  mm<32, 64, 64, false, true, false, false>(&sm.dO[0][0], kP68, &sm.sin[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r;
-      sm.dq[row][16 * nb + l15] = sm.gam[row] * acc[r];
-    }
-  });
-  // dP = dO U^T: dQK = tril(R) o dP into P's place is below (P still read above);
-  // the decay term QK o dP (lower) is formed from G's place after QK is rebuilt
-  __syncthreads();
-  mm<32, 32, 64, false, true, false, false>(&sm.dO[0][0], kP68, &sm.u[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sm.X[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];   // dP
-  });
-  __syncthreads();
-  // E (decay) += QK o dP o R on the lower triangle: QK = P / R there (R > 0);
-  // recomputing QK avoids the division: P holds tril(R) o QK
-  for (int i = tid; i < kQ * kQ; i += 64 * kGW) {
-    const int r = i >> 5, cc = i & 31;
-    const float dp = sm.X[r][cc], R = sm.dR[r][cc];
-    sm.dT[r][cc] = cc <= r ? sm.P[r][cc] * dp : 0.f;   // E_P = (R o QK) o dP = P o dP
-    sm.X[r][cc] = cc <= r ? R * dp : 0.f;              // dQK = tril(R) o dP
+    for (int rb = 0; rb < 2; ++rb) h2[rb] = prod(sm.Uh, sm.Ul, rb, kk, ah, al, h2[rb]);
   }
-  __syncthreads();
-  // dQ += dQK K -> global; dK = dQK^T Q (into U's place after Kbar' below)
-  mm<32, 64, 32, false, false, false, true>(&sm.X[0][0], kP36, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+  // ---- masked products, block w (0: r, c < 16; 1: r >= 16, c < 16; 2: both >= 16)
+  if (w < 3) {
+    const int rr0 = w > 0 ? 16 : 0, cc0 = w == 2 ? 16 : 0;
+    f32x4_t dp = z4, dpt = z4, eu = z4, eut = z4, qk = z4, gk = z4;   // [r][c]; ..t: [c][r]
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      dq[((row0 + row) * H + h) * kD + col] = rr::bf_bits(sm.dq[row][col] + acc[r]);
+    for (int kk = 0; kk < 2; ++kk) {
+      const u16x8_t uh = rr::row_frag<kD>(sm.Uh, cc0 + l15, kk, g), ul = rr::row_frag<kD>(sm.Ul, cc0 + l15, kk, g);
+      const u16x8_t oh = rr::row_frag<kD>(sm.Oh, rr0 + l15, kk, g), ol = rr::row_frag<kD>(sm.Ol, rr0 + l15, kk, g);
+      const u16x8_t eh = rr::row_frag<kD>(sm.Eh, rr0 + l15, kk, g), el = rr::row_frag<kD>(sm.El, rr0 + l15, kk, g);
+      const u16x8_t kc = rr::row_frag<kD>(sm.K, cc0 + l15, kk, g);
+      dp = mfma(ol, uh, dp);
+      dpt = mfma(uh, ol, dpt);
+      eu = mfma(el, uh, eu);
+      eut = mfma(uh, el, eut);
+      qk = mfma(rr::row_frag<kD>(sm.Q, rr0 + l15, kk, g), kc, qk);
+      gk = mfma(rr::row_frag<kD>(sm.K, rr0 + l15, kk, g), kc, gk);
+      dp = mfma(oh, ul, dp);
+      dpt = mfma(ul, oh, dpt);
+      eu = mfma(eh, ul, eu);
+      eut = mfma(ul, eh, eut);
+      dp = mfma(oh, uh, dp);
+      dpt = mfma(uh, oh, dpt);
+      eu = mfma(eh, uh, eu);
+      eut = mfma(uh, eh, eut);
     }
-  });
-  __syncthreads();
-  // Kbar' = U dS_out^T: dK += f o Kbar', rows(Kbar' o K) -> part[1]
-  mm<32, 64, 64, false, true, false, false>(&sm.u[0][0], kP68, &sm.dso[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+    auto put = [&](uint2(*dst)[64], const float (&x)[4]) {
+      u16x4_t hi, lo;
+      rr::bf_split4(f32x4_t{x[0], x[1], x[2], x[3]}, hi, lo);
+      dst[0][lane] = __builtin_bit_cast(uint2, hi);
+      dst[1][lane] = __builtin_bit_cast(uint2, lo);
+    };
+    const bool off = w == 1;   // the off-diagonal block: c < r throughout
+    float qa[4], qb[4], ga[4], gb[4];
+    const float lc = sm.lg[cc0 + l15], lr = sm.lg[rr0 + l15], br = sm.beta[rr0 + l15];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      sm.dq[row][col] = sm.f[row] * acc[r];   // dK partial (dq's place is free after its store)
-      const float s = rr::row16_sum(acc[r] * sm.k[row][col]);
-      if (l15 == 0) sm.part[1][row][nb] = s;
+    for (int e = 0; e < 4; ++e) {
+      {   // rows r = 4 g + e, column c = l15
+        const int r = 4 * g + e;
+        const bool low = off || l15 <= r, strict = off || l15 < r;
+        const float ex_ = __expf(low ? sm.lg[rr0 + r] - lc : 0.f), R = low ? ex_ : 0.f;
+        const float da = strict ? -eu[e] : 0.f, bt = sm.beta[rr0 + r];
+        qa[e] = R * dp[e];
+        ga[e] = bt * R * da;
+        sm.Em[rr0 + r][cc0 + l15] = qk[e] * qa[e] + gk[e] * ga[e];
+        const float s = rr::row16_sum(R * gk[e] * da);
+        if (l15 == 0) sm.p4[w == 2 ? 1 : 0][rr0 + r] = s;
+      }
+      {   // rows c = 4 g + e, column r = l15
+        const int cx = 4 * g + e;
+        const bool low = off || cx <= l15, strict = off || cx < l15;
+        const float ex_ = __expf(low ? lr - sm.lg[cc0 + cx] : 0.f), R = low ? ex_ : 0.f;
+        qb[e] = R * dpt[e];
+        gb[e] = strict ? -br * R * eut[e] : 0.f;
+      }
     }
-  });
-  __syncthreads();
-  mm<32, 64, 32, true, false, false, true>(&sm.X[0][0], kP36, &sm.q[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+    put(sm.QA[w], qa);
+    put(sm.QB[w], qb);
+    if (off) {
+      put(sm.DG[2], ga);   // rows 16-31, columns 0-15
+      put(sm.DG[1], gb);   // rows 0-15, columns 16-31
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm.dq[16 * mb + 4 * g + r][16 * nb + l15] += acc[r];   // dK += dQK^T Q
-  });
-  // dW = -dU S_in^T (into W's place)
-  __syncthreads();
-  mm<32, 64, 64, false, true, false, false>(&sm.du[0][0], kP68, &sm.sin[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sm.w[16 * mb + 4 * g + r][16 * nb + l15] = -acc[r];
-  });
-  // T^T dU: dV = diag(beta) T^T dU -> global, rows(T^T dU o V) -> part[2]
-  mm<32, 64, 32, true, false, false, false>(&sm.T[0][0], kP36, &sm.du[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      dv[((row0 + row) * H + h) * kD + col] = rr::bf_bits(sm.beta[row] * acc[r]);
-      const float s = rr::row16_sum(acc[r] * sm.v[row][col]);
-      if (l15 == 0) sm.part[2][row][nb] = s;
+      for (int e = 0; e < 4; ++e) ga[e] += gb[e];   // strictly lower and upper parts
+      put(sm.DG[w == 0 ? 0 : 3], ga);
     }
-  });
-  // dT = dU V^T diag(beta)
-  mm<32, 32, 64, false, true, false, true>(&sm.du[0][0], kP68, &sm.v[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = 16 * nb + l15;
-      sm.A[16 * mb + 4 * g + r][col] = sm.beta[col] * acc[r];   // A's place holds dT from here
-    }
-  });
-  __syncthreads();
-  // T^T dW: dK += diag(beta gam) T^T dW, rows(T^T dW o K) -> part[3]
-  mm<32, 64, 32, true, false, false, false>(&sm.T[0][0], kP36, &sm.w[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      sm.dq[row][col] += sm.beta[row] * sm.gam[row] * acc[r];
-      const float s = rr::row16_sum(acc[r] * sm.k[row][col]);
-      if (l15 == 0) sm.part[3][row][nb] = s;
-    }
-  });
-  // dT += dW K^T diag(beta gam)
-  mm<32, 32, 64, false, true, false, true>(&sm.w[0][0], kP68, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = 16 * nb + l15;
-      sm.A[16 * mb + 4 * g + r][col] += sm.beta[col] * sm.gam[col] * acc[r];
-    }
-  });
-  __syncthreads();
-  // dA = -T^T (dT T^T), strictly lower: X = dT T^T
-  mm<32, 32, 32, false, true, false, false>(&sm.A[0][0], kP36, &sm.T[0][0], kP36, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sm.X[16 * mb + 4 * g + r][16 * nb + l15] = acc[r];
-  });
-  __syncthreads();
-  mm<32, 32, 32, true, false, false, false>(&sm.T[0][0], kP36, &sm.X[0][0], kP36, [&](int mb, int nb, f32x4_t acc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      const float da = col < row ? -acc[r] : 0.f;
-      const float R = sm.dR[row][col], Gv = sm.G[row][col];
-      // E += diag(beta) G o dA o R; dG = diag(beta) R o dA; rows(R o G o dA) -> part[4]
-      sm.dT[row][col] += sm.beta[row] * Gv * da * R;
-      sm.A[row][col] = sm.beta[row] * R * da;   // dG (dT no longer needed)
-      const float s = rr::row16_sum(R * Gv * da);
-      if (l15 == 0) sm.part[4][row][nb] = s;
-    }
-  });
-  __syncthreads();
-  // dGs = dG + dG^T (into G's place); dK += dGs K -> global
-  for (int i = tid; i < kQ * kQ; i += 64 * kGW) {
-    const int r = i >> 5, cc = i & 31;
-    sm.G[r][cc] = sm.A[r][cc] + sm.A[cc][r];
   }
-  __syncthreads();
-  mm<32, 64, 32, false, false, false, true>(&sm.G[0][0], kP36, &sm.k[0][0], kP68, [&](int mb, int nb, f32x4_t acc) {
+  rr::lds_barrier();   // fragments
+
+  // ---- dQ^T, dK^T of this wave's rows i
+  {
+    const uint2 zz = make_uint2(0, 0);
+    const u16x8_t kt = rr::col_frag<kD>(sm.K, w, l15, g), qt = rr::col_frag<kD>(sm.Q, w, l15, g);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * g + r, col = 16 * nb + l15;
-      dk[((row0 + row) * H + h) * kD + col] = rr::bf_bits(sm.dq[row][col] + acc[r]);
+    for (int rb = 0; rb < 2; ++rb) {
+      f32x4_t aq = z4, ak = z4;
+#pragma unroll
+      for (int x = 1; x >= 0; --x) {   // lo, then hi
+        const u16x8_t qb = rb == 0 ? rr::join(sm.QB[0][x][lane], zz) : rr::join(sm.QB[1][x][lane], sm.QB[2][x][lane]);
+        const u16x8_t qa = rb == 0 ? rr::join(sm.QA[0][x][lane], sm.QA[1][x][lane]) : rr::join(zz, sm.QA[2][x][lane]);
+        const u16x8_t dg = rr::join(sm.DG[rb][x][lane], sm.DG[2 + rb][x][lane]);
+        aq = mfma(kt, qb, aq);
+        ak = mfma(qt, qa, ak);
+        ak = mfma(kt, dg, ak);
+      }
+      const int t = 16 * rb + l15;
+      const float gm = sm.gam[t], ft = sm.f[t], bg = sm.beta[t] * gm;
+      const uint2 k4 = *reinterpret_cast<const uint2*>(sm.K + rr::piece<kD>(t, 4 * w + g));
+      const uint2 q4 = *reinterpret_cast<const uint2*>(sm.Q + rr::piece<kD>(t, 4 * w + g));
+      float dq4[4], dk4[4], s0 = 0.f, s1 = 0.f, s3 = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float kv = rr::bf4(k4, r);
+        s0 += rr::bf4(q4, r) * h1[rb][r];
+        s1 += kv * h2[rb][r];
+        s3 -= kv * h3[rb][r];
+        dq4[r] = gm * h1[rb][r] + aq[r];
+        dk4[r] = ft * h2[rb][r] - bg * h3[rb][r] + ak[r];
+      }
+      const uint32_t o = (uint32_t)t * rs + 16 * w + 4 * g;
+      *reinterpret_cast<uint2*>(reinterpret_cast<char*>(dq + base) + 2 * o) = rr::pack4(dq4);
+      *reinterpret_cast<uint2*>(reinterpret_cast<char*>(dk + base) + 2 * o) = rr::pack4(dk4);
+      s0 = rr::rows4_sum(s0), s1 = rr::rows4_sum(s1), s3 = rr::rows4_sum(s3);
+      if (g == 0) sm.p0[w][t] = s0, sm.p1[w][t] = s1, sm.p3[w][t] = s3;
     }
-  });
+  }
+  rr::lds_barrier();
   // ---- the step scalars (wave 0, lane t < 32): dbeta, dlg -> dalpha
   //
   // dL/dlog(alpha_m) is the suffix sum over r >= m of dlg_r = dL/dlg_r, with
   //   dlg_r = rowE_r - colE_r + gam_r (p0 + beta_r p3)_r - f_r p1_r
   //           (+ gam_31 <dS_out, S_in> + sum_t f_t p1_t at r = 31).
-  // Summed as written it cancels: the entries of E inside the block
+  // Summed as written it cancels: the entries of Em inside the block
   // rows, columns >= m, and the f_r p1_r with r >= m, are O(1) whatever
   // alpha_m, and appear with both signs, while the sum is O(alpha_m), so its
   // rounding divided by a small alpha_m swamps dalpha_m.  The same sum,
-  // regrouped (E is lower triangular):
-  //   sum_{r >= m} dlg_r = sum_{r >= m, c < m} E[r][c] + sum_{r >= m} gam_r (p0 + beta_r p3)_r
+  // regrouped (Em is lower triangular):
+  //   sum_{r >= m} dlg_r = sum_{r >= m, c < m} Em[r][c] + sum_{r >= m} gam_r (p0 + beta_r p3)_r
   //                        + sum_{t < m} f_t p1_t + gam_31 <dS_out, S_in>,
   // where every term carries alpha_m as a factor (R[r][c] = gam_r / gam_c for
   // c < m <= r, gam_r for r >= m, f_t = gam_31 / gam_t for t < m), so it keeps
@@ -1032,7 +991,7 @@ __global__ __launch_bounds__(64 * kGW) void gdn_cgrad_kernel(const float* __rest
 #pragma unroll 4
     for (int rr_ = 0; rr_ < kQ / 2; ++rr_) {
       const int r = 16 * half + rr_;
-      const float4* row = reinterpret_cast<const float4*>(&sm.dT[r][0]);
+      const float4* row = reinterpret_cast<const float4*>(&sm.Em[r][0]);
       float acc = 0.f;
 #pragma unroll
       for (int c4 = 0; c4 < kQ / 4; ++c4) {
@@ -1043,11 +1002,11 @@ __global__ __launch_bounds__(64 * kGW) void gdn_cgrad_kernel(const float* __rest
       blk += r >= t ? acc : 0.f;
     }
     blk += __shfl_xor(blk, 32);
-    auto rows = [&](int qn) { return (sm.part[qn][t][0] + sm.part[qn][t][1]) + (sm.part[qn][t][2] + sm.part[qn][t][3]); };
-    const float p0 = rows(0), p1 = rows(1), p2 = rows(2), p3 = rows(3);
-    const float p4 = (sm.part[4][t][0] + sm.part[4][t][1]);   // 32 columns: two blocks
+    auto rows = [&](const float(*p)[kQ]) { return (p[0][t] + p[1][t]) + (p[2][t] + p[3][t]); };
+    const float p0 = rows(sm.p0), p1 = rows(sm.p1), p3 = rows(sm.p3);
+    const float p4 = sm.p4[0][t] + (t < 16 ? 0.f : sm.p4[1][t]);
     const float gm = sm.gam[t], be = sm.beta[t], ft = sm.f[t];
-    const float dbe = p2 + gm * p3 + p4;
+    const float dbe = sm.p2[t] + gm * p3 + p4;
     // suffix sum over r >= t of gam_r (p0 + beta_r p3)_r; prefix over t' < t of
     // f p1, shifted by one lane first (f_t p1_t itself does not carry alpha_t,
     // so an inclusive prefix minus it would cancel again)
@@ -1059,10 +1018,8 @@ __global__ __launch_bounds__(64 * kGW) void gdn_cgrad_kernel(const float* __rest
       if (t + o < 32) suf += x;
       if (t >= o) pre += y;
     }
-    float dot = 0.f;
-#pragma unroll
-    for (int ww = 0; ww < kGW; ++ww) dot += sm.dotp[ww];
-    suf += blk + pre + sm.gam[kQ - 1] * dot;
+    const float dots = (sm.dot[0] + sm.dot[1]) + (sm.dot[2] + sm.dot[3]);
+    suf += blk + pre + sm.gam[kQ - 1] * dots;
     if (lane < kQ) {
       dalpha[(row0 + t) * H + h] = rr::bf_bits(suf / sm.al[t]);
       dbeta[(row0 + t) * H + h] = rr::bf_bits(dbe);
@@ -1112,7 +1069,7 @@ int gdn_chunk_adjoint(const void* q, const void* k, const void* v, const void* a
                      (int)L, (int)nC);
   if (int rc = check_launch("gdn chunked adjoint (WY)")) return rc;
   hipLaunchKernelGGL(gdn_rstate_kernel, dim3((unsigned)(groups * kXcd * 4)), dim3(64), 0, s,
-                     static_cast<const BwdPack*>(packs), dy, dfinal, adjck, dh0, (int)BH, (int)H, (int)L, (int)nC);
+                     static_cast<BwdPack*>(packs), dy, dfinal, adjck, dh0, (int)BH, (int)H, (int)L, (int)nC);
   return check_launch("gdn chunked adjoint (state)");
 }
 
@@ -1121,13 +1078,13 @@ int gdn_chunk_adjoint(const void* q, const void* k, const void* v, const void* a
 namespace rr {
 
 int gdn_chunk_grad(const float* dy, const void* q, const void* k, const void* v, const void* alpha, const void* beta,
-                   const float* h0, const float* ckpt, const float* adjck, void* dq, void* dk, void* dv, void* dalpha,
-                   void* dbeta, int64_t B, int64_t L, int64_t H, hipStream_t s) {
+                   const float* h0, const float* ckpt, const float* adjck, const void* packs, void* dq, void* dk, void* dv,
+                   void* dalpha, void* dbeta, int64_t B, int64_t L, int64_t H, hipStream_t s) {
   const int64_t BH = B * H, nC = L / kQ, groups = (BH + kXcd - 1) / kXcd;
-  hipLaunchKernelGGL(gdn_cgrad_kernel, dim3((unsigned)(groups * kXcd * nC)), dim3(64 * kGW), 0, s, dy,
+  hipLaunchKernelGGL(gdn_cgrad_kernel, dim3((unsigned)(groups * kXcd * nC)), dim3(64 * kGradWaves), 0, s, dy,
                      static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
                      static_cast<const uint16_t*>(alpha), static_cast<const uint16_t*>(beta), h0, ckpt, adjck,
-                     static_cast<uint16_t*>(dq), static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv),
+                     static_cast<const BwdPack*>(packs), static_cast<uint16_t*>(dq), static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv),
                      static_cast<uint16_t*>(dalpha), static_cast<uint16_t*>(dbeta), (int)BH, (int)H, (int)L, (int)nC);
   return check_launch("gdn chunked gradients");
 }

@@ -123,10 +123,10 @@ int gdn_chunk_adjoint(const void* q, const void* k, const void* v, const void* a
                       const float* dfinal, int64_t B, int64_t L, int64_t H, float* adjck, float* dh0, void* packs,
                       hipStream_t s);
 // The gradient pass in chunkwise form, every chunk at once, from the forward
-// and adjoint checkpoints.
+// and adjoint checkpoints and what the adjoint pass left in its packs.
 int gdn_chunk_grad(const float* dy, const void* q, const void* k, const void* v, const void* alpha, const void* beta,
-                   const float* h0, const float* ckpt, const float* adjck, void* dq, void* dk, void* dv, void* dalpha,
-                   void* dbeta, int64_t B, int64_t L, int64_t H, hipStream_t s);
+                   const float* h0, const float* ckpt, const float* adjck, const void* packs, void* dq, void* dk, void* dv,
+                   void* dalpha, void* dbeta, int64_t B, int64_t L, int64_t H, hipStream_t s);
 
 // ------------------------------------------------------------------ SSD, rate per (head, n)
 // Chunked SSD for A_neg [H, N] (any input dtype) and for fp32 / fp16 inputs
