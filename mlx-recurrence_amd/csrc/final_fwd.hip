@@ -34,12 +34,12 @@
 //
 // What bounds it: without checkpoints the instructions of a chunk (per wave
 // about 500 VALU, a third of them the state's three-term split, beside 50
-// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 107 us,
+// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 99 us,
 // 2.9 TB/s of the 0.31 GB it cannot do without (6.1 ms on the VALU engine,
 // which forms and stores a state every 8 steps there; 132 us with W and the
 // scalars formed by every wave for itself).  Three waves per SIMD (168 VGPRs)
 // spill 18 and take 178 us.  With checkpoints the traffic: B8 L4096 H80 Dh64
-// N128 1224 us, 4.4 TB/s; B8 L2048 H12 GLA Dh128 448 -> 215 us.
+// N128 1224 us, 4.4 TB/s; B8 L2048 H12 GLA Dh128 448 -> 186 us.
 #include "rr_chunked.h"
 #include "rr_frag.h"
 
@@ -331,10 +331,8 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
 
   for (int c = c0; c < c1; ++c) {
     const int buf = (c - c0) & 1;
-    if (c + 1 < c1) {
-      stage(c + 1, buf ^ 1);
-      load(c + 2);
-    }
+    if (c + 1 < c1) stage(c + 1, buf ^ 1);
+    load(c + 2);   // (unconditional: under the branch, the scalar wave's wait for its step input would cover these too)
     lds_barrier();   // this chunk's W, the next one's rows
     if constexpr (!AGG) {
       if (c + 1 < c1) w_blocks(c + 1, buf ^ 1);
