@@ -37,8 +37,10 @@
 // What bounds it: per wave and chunk about 1000 VALU instructions (the splits of
 // h_in and of both copies of lam are a third) beside 116 MFMAs (Dh 64, N 128) on
 // two waves per SIMD, and the traffic of inputs, checkpoints and gradients.
-// SSD B8 L4096 H80 Dh64 N128: 2.0 ms, 3.3 TB/s of 6.7 GB (adjoint scan + pair kernel
-// 2.7 ms, 12.6 GB); GLA B8 L2048 H12 Dh128: 276 + 67 us (348 + 102 + 156 us).
+// SSD B8 L4096 H80 Dh64 N128: 1.74 + 0.23 ms, 3.4 TB/s of 6.7 GB (adjoint scan +
+// pair kernel 2.7 ms, 12.6 GB); GLA B8 L2048 H12 Dh128: 235 + 65 us (348 + 102 +
+// 156 us).  No register may spill: a spilled load waits for its data at once,
+// and a reload for every load in flight (1.88 ms with 4 spills).
 #include "rr_chunked.h"
 #include "rr_frag.h"
 
@@ -214,14 +216,13 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
                           : (p.h0 != nullptr ? p.h0 + (int64_t)bh * DH * NS : p.ckpt);
     const auto hs = rr::as_global(src);
     const int sd = GLA && !ck ? 1 : NS, sn = GLA && !ck ? DH : 1;   // element strides of d and n
-    const float use = c > 0 || p.h0 != nullptr ? 1.f : 0.f;
 #pragma unroll
     for (int cc = 0; cc < CPW; ++cc) {
       const uint32_t o = (uint32_t)((16 * (w * CPW + cc) + l15) * sn + 4 * g * sd);
 #pragma unroll
       for (int db = 0; db < NBD; ++db)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) hin[cc][db][r] = use * rr::ld32<float>(hs + (16 * db + r) * sd, o);
+        for (int r = 0; r < 4; ++r) hin[cc][db][r] = rr::ld32<float>(hs + (16 * db + r) * sd, o);
     }
   };
   auto scalars = [&](int c) {   // one wave
@@ -285,7 +286,6 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
   load_step(c1 - 1);
   constexpr int MF = CPW * NBD + DPW * NBN;   // float4 per thread of a map
   if constexpr (!MAP) {
-    load_h(c1 - 1);
     if (p.dfinal != nullptr) {
       const float* dp = p.dfinal + (int64_t)bh * DH * NS;
 #pragma unroll
@@ -482,6 +482,7 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
 
   if (w == NW - 1) scalars(c1 - 1);
   load_step(c1 - 2);
+  if constexpr (!MAP) load_h(c1 - 1);   // (last, as in the loop: waits for older loads count past it)
   lds_barrier();
 
   for (int c = c1 - 1; c >= c0; --c) {
@@ -505,6 +506,12 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
     f32x4_t gh[MAP ? 1 : CPW][2], ul[MAP ? 1 : CPW][2];   // GH^T[n][t], UL^T[n][s]
     if constexpr (!MAP) {
       if (w < 3) masked(c, w);
+      if (c == 0 && p.h0 == nullptr) {   // a zero start (load_h read the last row it may)
+#pragma unroll
+        for (int cc = 0; cc < CPW; ++cc)
+#pragma unroll
+          for (int db = 0; db < NBD; ++db) hin[cc][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
       // ---- GH, UL of this wave's columns, their row sums, lam o h_in
       float xs[2] = {0.f, 0.f}, ys[2] = {0.f, 0.f}, trp = 0.f;
 #pragma unroll
@@ -626,7 +633,9 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
         }
       }
       __builtin_amdgcn_sched_barrier(0);   // keeps the phases' operands from living at once
-      load(c - 1);   // (here, not before: the registers of GH and UL are free now)
+      // (here, not before: the registers of GH and UL are free now; a spilled
+      // address or step input would make the wave wait for all of these at once)
+      load(c - 1);
       // ---- du of this wave's rows
       uint16_t* const duP = p.du + (row0 * p.H + h) * DH;
 #pragma unroll
