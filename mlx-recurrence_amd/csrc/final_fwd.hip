@@ -34,12 +34,12 @@
 //
 // What bounds it: without checkpoints the instructions of a chunk (per wave
 // about 500 VALU, a third of them the state's three-term split, beside 50
-// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 99 us,
+// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 97 us,
 // 2.9 TB/s of the 0.31 GB it cannot do without (6.1 ms on the VALU engine,
 // which forms and stores a state every 8 steps there; 132 us with W and the
 // scalars formed by every wave for itself).  Three waves per SIMD (168 VGPRs)
 // spill 18 and take 178 us.  With checkpoints the traffic: B8 L4096 H80 Dh64
-// N128 1224 us, 4.4 TB/s; B8 L2048 H12 GLA Dh128 448 -> 186 us.
+// N128 1168 us, 4.6 TB/s; B8 L2048 H12 GLA Dh128 448 -> 195 us.
 #include "rr_chunked.h"
 #include "rr_frag.h"
 
@@ -326,6 +326,21 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
     scalars(min(c0 + 1, p.nC - 1));
   }
   load_step(c0 + 2);
+  // the rows of y of chunk c, from this head's first column: a store past the
+  // last row of V is dropped
+  auto y_rows = [&](int c, int V) {
+    float* yp = p.y + ((rows + (int64_t)c * Q) * p.H + h) * DH;
+    return __builtin_amdgcn_make_buffer_rsrc(yp, 0, (int)((uint32_t)V * rsD * 4u), 0x00027000);
+  };
+  if constexpr (!AGG) {
+    // as many dropped stores as a chunk makes after its loads: the waits for
+    // those loads at the loop's head then count past a chunk's stores (without
+    // them they cover the stores: 99.5 -> 96.6 us at the first size above)
+    const auto none = y_rows(c0, 0);
+#pragma unroll
+    for (int j = 0; j < 8 * DB + (OUT == kCkpt ? DB * (NS / 16) : 0); ++j)
+      __builtin_amdgcn_raw_buffer_store_b32(0u, none, 4 * lane + 256 * j, 0, 0);
+  }
   lds_barrier();
   if constexpr (!AGG) w_blocks(c0, 0);
 
@@ -430,19 +445,13 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
             }
           }
         }
-        const int V = p.L - c * Q;
-        float* yp = p.y + ((rows + (int64_t)c * Q) * p.H + h) * DH + 16 * (w * DB + i);
-        auto put = [&](int tb, int r) {
-          const uint32_t off = (uint32_t)(16 * tb + 4 * g + r) * rsD + l15;
-          *reinterpret_cast<float*>(reinterpret_cast<char*>(yp) + off * 4u) = o[tb][r];
-        };
-        if (V >= Q) {
+        const auto yr = y_rows(c, min(p.L - c * Q, Q));
 #pragma unroll
-          for (int j = 0; j < 8; ++j) put(j >> 2, j & 3);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (16 * (j >> 2) + 4 * g + (j & 3) < V) put(j >> 2, j & 3);
+        for (int j = 0; j < 8; ++j) {
+          const float v = o[j >> 2][j & 3];   // (a copy: a bit cast of a vector's element takes the first one)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr,
+                                                (int)(4u * ((uint32_t)(16 * (j >> 2) + 4 * g + (j & 3)) * rsD + l15)),
+                                                64 * (w * DB + i), 0);
         }
       }
     }
