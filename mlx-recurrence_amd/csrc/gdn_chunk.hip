@@ -389,6 +389,12 @@ __global__ __launch_bounds__(64) void gdn_wy_kernel(const uint16_t* __restrict__
 // through the chunks in order.  Per chunk: U = U0 - W S_in, the output
 // O = diag(gam) Q S_in + P U, then S_out = gam_31 S_in + Kbar^T U, written as
 // the chunk's checkpoint.
+//
+// What bounds it: the latency of a chunk's 28 loads, one chunk ahead (its 24
+// stores and two sets of loads already fill the wave's counter of 63 accesses
+// in flight; three sets, which the compiler loaded late, took 134 us, this 117
+// at B8 L2048 H12, 2.9 TB/s).  A workgroup per head that shares the operands
+// through LDS took 127 us, and a training step at B3 L512 H12 93 us against 80.
 struct Frags {
   uint4 W[2][2][2], Kb[4][2], P[2][2], Qf[2][2];
   float4 U0[2], gam[2];
@@ -415,6 +421,17 @@ __device__ __forceinline__ void load_frags(Frags& f, const ChunkPack& pk, int s,
     f.Kb[ib][1] = pk.Kb[ib][1][lane];
   }
   f.gend = pk.gam[kQ - 1];
+}
+
+// K stores that the hardware drops (to a buffer of no bytes).  Ahead of a loop
+// that waits for its loads by count, they stand for the stores that an iteration
+// makes after those loads; without them the wait, the same for every iteration,
+// covers the last iteration's stores too.
+template <int K>
+__device__ __forceinline__ void dropped_stores(float* p, int lane) {
+  const auto none = __builtin_amdgcn_make_buffer_rsrc(p, 0, 0, 0x00027000);
+#pragma unroll
+  for (int k = 0; k < K; ++k) __builtin_amdgcn_raw_buffer_store_b32(0u, none, 4 * lane + 256 * k, 0, 0);
 }
 
 __global__ __launch_bounds__(64) void gdn_state_kernel(const ChunkPack* __restrict__ pack, const float* __restrict__ h0,
@@ -493,22 +510,21 @@ __global__ __launch_bounds__(64) void gdn_state_kernel(const ChunkPack* __restri
 #pragma unroll
       for (int r = 0; r < 4; ++r) ck[(16 * ib + 4 * g + r) * kD + j] = S[ib][r];
   };
-  // three fragment sets in a ring, loads two chunks ahead (issued whatever
-  // the chunk count, at clamped indices: the waits for a set stay exact)
+  // two fragment sets, loads a chunk ahead (clamped indices).  No branch within
+  // a pair of chunks: the compiler would move the loads behind it
   auto ld = [&](Frags& f, int c) { load_frags(f, pk[min(c, nC - 1)], s, lane); };
-  Frags fa, fb, fc;
+  Frags fa, fb;
   ld(fa, 0);
-  ld(fb, 1);
-  for (int c = 0; c < nC; c += 3) {
-    ld(fc, c + 2);
+  dropped_stores<24>(y, lane);
+  for (int c = 0; c + 1 < nC; c += 2) {
+    ld(fb, c + 1);
+    __builtin_amdgcn_sched_barrier(0);
     step(fa, c);
-    if (c + 1 >= nC) break;
-    ld(fa, c + 3);
+    ld(fa, c + 2);
+    __builtin_amdgcn_sched_barrier(0);
     step(fb, c + 1);
-    if (c + 2 >= nC) break;
-    ld(fb, c + 4);
-    step(fc, c + 2);
   }
+  if (nC & 1) step(fa, nC - 1);
 }
 
 // ------------------------------------------------------------------ kernel 3
@@ -614,24 +630,23 @@ __global__ __launch_bounds__(64) void gdn_rstate_kernel(BwdPack* __restrict__ pa
       S[ib] = a;
     }
   };
-  // three fragment sets in a ring, loads two chunks ahead (clamped indices)
+  // two fragment sets, as in kernel 2
   auto ld = [&](BFrags& f, int c) {
     const int cc = max(c, 0);
     load_bfrags(f, pk[cc], dy, row0(cc), H, h, j, lane);
   };
-  BFrags fa, fb, fc;
+  BFrags fa, fb;
   ld(fa, nC - 1);
-  ld(fb, nC - 2);
-  for (int c = nC - 1; c >= 0; c -= 3) {
-    ld(fc, c - 2);
+  dropped_stores<24>(adjck, lane);
+  for (int c = nC - 1; c > 0; c -= 2) {
+    ld(fb, c - 1);
+    __builtin_amdgcn_sched_barrier(0);
     step(fa, c);
-    if (c - 1 < 0) break;
-    ld(fa, c - 3);
+    ld(fa, c - 2);
+    __builtin_amdgcn_sched_barrier(0);
     step(fb, c - 1);
-    if (c - 2 < 0) break;
-    ld(fb, c - 4);
-    step(fc, c - 2);
   }
+  if (nC & 1) step(fa, 0);
   if (dh0 != nullptr) {
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib)
