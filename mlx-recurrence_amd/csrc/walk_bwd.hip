@@ -34,10 +34,10 @@
 // and its decay), and segment j starts from dfinal carried through the maps
 // of segments S - 1 .. j + 1.
 //
-// What bounds it: per wave and chunk about 1000 VALU instructions (the splits of
-// h_in and of both copies of lam are a third) beside 116 MFMAs (Dh 64, N 128) on
+// What bounds it: per wave and chunk about 1300 VALU instructions (the splits of
+// h_in and of both copies of lam are a fifth) beside 127 MFMAs (Dh 64, N 128) on
 // two waves per SIMD, and the traffic of inputs, checkpoints and gradients.
-// SSD B8 L4096 H80 Dh64 N128: 1.74 + 0.23 ms, 3.4 TB/s of 6.7 GB (adjoint scan +
+// SSD B8 L4096 H80 Dh64 N128: 1.74 + 0.23 ms, 4.0 TB/s of 6.9 GB (adjoint scan +
 // pair kernel 2.7 ms, 12.6 GB); GLA B8 L2048 H12 Dh128: 235 + 65 us (348 + 102 +
 // 156 us).  No register may spill: a spilled load waits for its data at once,
 // and a reload for every load in flight (1.88 ms with 4 spills).
@@ -800,7 +800,7 @@ namespace rr {
 // or pass (forward + backward, us): from 1100 chunks in all.  768 chunks 0.77x
 // (GLA 96 heads Dh 64, 36.5 -> 47.7) to 1.29x; 1152 chunks 1.02x to 1.39x; 1280
 // 1.0x (GLA 320 heads Dh 64, 4 chunks) to 1.6x; 6144 1.36x to 1.6x (GLA B8 L2048 H12
-// Dh128 810 -> 489).  Fewer than 12 heads serialise too long segments (8
+// Dh128 810 -> 450).  Fewer than 12 heads serialise too long segments (8
 // heads, 128 chunks: 0.9x).
 bool walk_bwd_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N) {
   if (BH * Q >= (int64_t(1) << 31)) return false;
