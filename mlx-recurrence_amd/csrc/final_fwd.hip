@@ -588,8 +588,9 @@ int run(FinalArgs& p, int64_t B, int64_t H, int64_t Dh, int64_t N, void* ws, siz
 
 bool sizes_ok(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N) {
   if (B <= 0 || L <= 0 || H <= 0 || Dh <= 0 || N <= 0) return false;
-  // 1-D grid of heads; 32-bit byte offsets within a chunk; int step counts
-  return B <= 0x7fffffff && H <= 0x7fffffff && B * H < (int64_t(1) << 31) && L < (int64_t(1) << 30) &&
+  // what the entry points take at all; a grid of heads; 32-bit byte offsets
+  // within a chunk; int step counts
+  return rr::scan_dims_ok(B, L, H) && B * H < (int64_t(1) << 31) && L < (int64_t(1) << 30) &&
          H * std::max(Dh, N) * Q * 4 < (int64_t(1) << 31);
 }
 
@@ -668,7 +669,7 @@ extern "C" int rr_ssd_final_fwd(const void* u, const void* delta, const void* Bm
                                 int64_t A_stride_n, int dtype, int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N,
                                 int64_t seg, const float* h0, float* y, float* fin, void* workspace,
                                 size_t workspace_bytes, void* stream) {
-  if (int rc = rr::check_segment_shape(L, seg, Dh, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("ssd_final_fwd", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
   if (!u || !delta || !Bm || !Cm || !A_neg || !y || !fin)
     return rr::fail(RR_EINVAL, "ssd_final_fwd: null pointer argument");
   if (rr_ssd_final_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype) < 0)
@@ -694,7 +695,7 @@ extern "C" int64_t rr_gla_final_workspace_bytes(int64_t B, int64_t L, int64_t H,
 extern "C" int rr_gla_final_fwd(const void* q, const void* k, const void* v, const void* gates, int dtype, int64_t B,
                                 int64_t L, int64_t H, int64_t Dh, int64_t seg, const float* h0, float* y, float* fin,
                                 void* workspace, size_t workspace_bytes, void* stream) {
-  if (int rc = rr::check_segment_shape(L, seg, Dh, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("gla_final_fwd", B, L, H, Dh, Dh, seg, dtype, "Dh")) return rc;
   if (!q || !k || !v || !gates || !y || !fin) return rr::fail(RR_EINVAL, "gla_final_fwd: null pointer argument");
   if (rr_gla_final_workspace_bytes(B, L, H, Dh, seg, dtype) < 0)
     return rr::fail(RR_EUNSUPPORTED, "gla_final_fwd: call not covered (rr_gla_final_workspace_bytes is -1)");

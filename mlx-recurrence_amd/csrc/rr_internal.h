@@ -7,6 +7,16 @@
 
 namespace rr {
 
+// Limits of the SSD and GLA entry points, whichever kernels run the call: a call
+// is refused with and without a gradient alike.
+constexpr int64_t kMaxBatchOrHeads = 65535;
+constexpr int64_t kMaxRows = int64_t(1) << 31;   // B * L
+inline bool scan_dims_ok(int64_t B, int64_t L, int64_t H) {
+  return B <= kMaxBatchOrHeads && H <= kMaxBatchOrHeads && B * L <= kMaxRows;
+}
+int check_scan_dims(const char* who, int64_t B, int64_t L, int64_t H, int64_t DL, int64_t NS, int64_t seg, int dtype,
+                    const char* lane_name);
+
 // Arguments of the chunked kernels, named for SSD.  GLA maps onto them as
 // u = v, delta = gates, Bm = k, Cm = q (du = dv, ddelta = dgates, dB = dk,
 // dC = dq); A, A_stride_h and dA are unused there.

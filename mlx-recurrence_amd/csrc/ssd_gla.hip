@@ -856,19 +856,6 @@ Plan make_plan(int64_t B, int64_t L, int64_t H, int64_t DL, int64_t NS, int64_t 
   return q;
 }
 
-int check_dims(const char* who, int64_t B, int64_t L, int64_t H, int64_t DL, int64_t NS,
-               int64_t seg, int dtype, const char* lane_name) {
-  if (B <= 0 || L <= 0 || H <= 0 || DL <= 0 || NS <= 0)
-    return rr::fail(RR_EINVAL, std::string(who) + ": all dimensions must be positive");
-  if (int rc = rr::check_segment_shape(L, seg, DL, lane_name)) return rc;
-  if (!rr::valid_dtype(dtype)) return rr::fail(RR_EINVAL, std::string(who) + ": unsupported dtype");
-  if (B > 65535 || H > 65535)
-    return rr::fail(RR_EUNSUPPORTED, std::string(who) + ": B and H must be <= 65535");
-  if (B * L > ((int64_t)1 << 31) / kFinRows * kFinRows)
-    return rr::fail(RR_EUNSUPPORTED, std::string(who) + ": B*L too large");
-  return RR_OK;
-}
-
 template <typename InT, bool GLA>
 int launch_fwd(Args<InT> a, const Plan& q, int64_t B, void* ws, hipStream_t s, float* y) {
   if (tile_grid(B, a.H, q.groups, q.ND * q.NN) >= ((int64_t)1 << 31))
@@ -986,6 +973,20 @@ int dense_bwd(rr::DenseArgs d, int dtype, const Plan& q, char* ws, const float* 
 
 }  // namespace
 
+namespace rr {
+int check_scan_dims(const char* who, int64_t B, int64_t L, int64_t H, int64_t DL, int64_t NS, int64_t seg, int dtype,
+                    const char* lane_name) {
+  if (B <= 0 || L <= 0 || H <= 0 || DL <= 0 || NS <= 0)
+    return fail(RR_EINVAL, std::string(who) + ": all dimensions must be positive");
+  if (int rc = check_segment_shape(L, seg, DL, lane_name)) return rc;
+  if (!valid_dtype(dtype)) return fail(RR_EINVAL, std::string(who) + ": unsupported dtype");
+  if (B > kMaxBatchOrHeads || H > kMaxBatchOrHeads)
+    return fail(RR_EUNSUPPORTED, std::string(who) + ": B and H must be <= 65535");
+  if (!scan_dims_ok(B, L, H)) return fail(RR_EUNSUPPORTED, std::string(who) + ": B*L too large");
+  return RR_OK;
+}
+}  // namespace rr
+
 // ====================================================================== SSD
 extern "C" size_t rr_ssd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N,
                                          int64_t seg, int64_t A_stride_n, int dtype, int pass) {
@@ -1020,7 +1021,7 @@ extern "C" int rr_ssd_fwd(const void* u, const void* delta, const void* Bm, cons
                           const float* A_neg, int64_t A_stride_n, int dtype, int64_t B, int64_t L, int64_t H,
                           int64_t Dh, int64_t N, int64_t seg, const float* h0, float* y,
                           float* ckpt, void* workspace, size_t workspace_bytes, void* stream) {
-  if (int rc = check_dims("ssd_fwd", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("ssd_fwd", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
   if (N > 256) return rr::fail(RR_EUNSUPPORTED, "ssd_fwd: N > 256 is not supported");
   if (!u || !delta || !Bm || !Cm || !A_neg || !y || !ckpt)
     return rr::fail(RR_EINVAL, "ssd_fwd: null pointer argument");
@@ -1083,7 +1084,7 @@ extern "C" int rr_ssd_bwd(const float* dy, const float* dfinal, const void* u, c
                           const float* h0, const float* ckpt, void* du, void* ddelta, void* dB,
                           void* dC, float* dA_neg, int64_t dA_stride_n, float* dh0, void* workspace,
                           size_t workspace_bytes, void* stream) {
-  if (int rc = check_dims("ssd_bwd", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("ssd_bwd", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
   if (N > 256) return rr::fail(RR_EUNSUPPORTED, "ssd_bwd: N > 256 is not supported");
   if (!dy || !u || !delta || !Bm || !Cm || !A_neg || !ckpt || !du || !ddelta || !dB || !dC ||
       !dA_neg)
@@ -1223,7 +1224,7 @@ extern "C" int rr_ssd_bwd_noalloc(const float* dy, const float* dfinal, const vo
                                   int64_t seg, const float* h0, const float* ckpt, void* du, void* ddelta,
                                   void* dB, void* dC, float* dA_neg, int64_t dA_stride_n, float* dh0,
                                   void* stream) {
-  if (int rc = check_dims("ssd_bwd_noalloc", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("ssd_bwd_noalloc", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
   if (A_stride_n != 0 && A_stride_n != 1)
     return rr::fail(RR_EINVAL, "ssd_bwd_noalloc: A_stride_n must be 0 or 1");
   const size_t need = rr_ssd_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype, 1);
@@ -1282,7 +1283,7 @@ extern "C" int rr_gla_fwd(const void* qp, const void* kp, const void* vp, const 
                           int dtype, int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t seg,
                           const float* h0, float* y, float* ckpt, void* workspace,
                           size_t workspace_bytes, void* stream) {
-  if (int rc = check_dims("gla_fwd", B, L, H, Dh, Dh, seg, dtype, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("gla_fwd", B, L, H, Dh, Dh, seg, dtype, "Dh")) return rc;
   if (!qp || !kp || !vp || !gates || !y || !ckpt)
     return rr::fail(RR_EINVAL, "gla_fwd: null pointer argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1333,7 +1334,7 @@ extern "C" int rr_gla_bwd(const float* dy, const float* dfinal, const void* qp, 
                           int64_t H, int64_t Dh, int64_t seg, const float* h0, const float* ckpt,
                           void* dq, void* dk, void* dv, void* dgates, float* dh0, void* workspace,
                           size_t workspace_bytes, void* stream) {
-  if (int rc = check_dims("gla_bwd", B, L, H, Dh, Dh, seg, dtype, "Dh")) return rc;
+  if (int rc = rr::check_scan_dims("gla_bwd", B, L, H, Dh, Dh, seg, dtype, "Dh")) return rc;
   if (!dy || !qp || !kp || !vp || !gates || !ckpt || !dq || !dk || !dv || !dgates)
     return rr::fail(RR_EINVAL, "gla_bwd: null pointer argument");
   if (rr::gla2_supported(dtype, B, L, H, seg, Dh, 1)) {
