@@ -590,7 +590,7 @@ bool sizes_ok(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N) {
   if (B <= 0 || L <= 0 || H <= 0 || Dh <= 0 || N <= 0) return false;
   // what the entry points take at all; a grid of heads; 32-bit byte offsets
   // within a chunk; int step counts
-  return rr::scan_dims_ok(B, L, H) && B * H < (int64_t(1) << 31) && L < (int64_t(1) << 30) &&
+  return rr::scan_dims_ok(B, L, H) && rr::grid_ok(B * H, 4 * Dh) && L < (int64_t(1) << 30) &&
          H * std::max(Dh, N) * Q * 4 < (int64_t(1) << 31);
 }
 
@@ -629,7 +629,7 @@ namespace rr {
 //   resident kernel does not cover, below 512 heads (123 -> 94) unless GLA's
 //   wide direct mode takes it (BH nC <= 768: 23 against 31).
 bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla) {
-  if (BH < 24 || BH * Q >= (int64_t(1) << 31)) return false;
+  if (BH < 24 || !grid_ok(BH, 4 * Dh)) return false;
   if (nC > 16) return N >= 64 || (nC >= 32 && (N == 32 || BH <= 256));
   if (N == 128) return BH < 512 && !(gla && BH * nC <= 768);
   return N == 64 && Dh == 64 && BH >= 256;

@@ -16,6 +16,9 @@ inline bool scan_dims_ok(int64_t B, int64_t L, int64_t H) {
 }
 int check_scan_dims(const char* who, int64_t B, int64_t L, int64_t H, int64_t DL, int64_t NS, int64_t seg, int dtype,
                     const char* lane_name);
+// A 1-D grid of this many workgroups of `threads` that HIP launches: fewer than
+// 2^32 threads.
+inline bool grid_ok(int64_t workgroups, int64_t threads) { return workgroups < (int64_t(1) << 32) / threads; }
 
 // Arguments of the chunked kernels, named for SSD.  GLA maps onto them as
 // u = v, delta = gates, Bm = k, Cm = q (du = dv, ddelta = dgates, dB = dk,

@@ -803,7 +803,7 @@ namespace rr {
 // Dh128 810 -> 450).  Fewer than 12 heads serialise too long segments (8
 // heads, 128 chunks: 0.9x).
 bool walk_bwd_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N) {
-  if (BH * Q >= (int64_t(1) << 31)) return false;
+  if (!grid_ok(BH, 512)) return false;   // the most threads a workgroup has
   return (Dh == 64 || Dh == 128) && (N == 64 || N == 128) && BH >= 12 && BH * nC >= 1100;
 }
 
