@@ -152,3 +152,58 @@ def test_non_finite_input_stays_causal(bad):
         y, _ = mr.ssd_scan_with_state(*xs, seg=8, initial_state=st)
         assert torch.equal(y[:, :s], clean[:, :s]) and torch.equal(y[:, :, 0], clean[:, :, 0]), k
         assert not torch.isfinite(y[0, s, 1]).all(), k
+
+
+def _same(got, want, tol):
+    """Infinities and NaN where the recurrence has them; the finite values within tol."""
+    got = got.detach().double().cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    assert np.abs(got[ok] - want[ok]).max(initial=0) <= tol * np.abs(want[ok]).max(initial=0)
+
+
+# one and several segments, a whole number of chunks (walking, with and without checkpoints)
+@pytest.mark.parametrize("kind,B,L,H,N,seg,grad", [("ssd", 1, 72, 2, 128, 8, False), ("ssd", 1, 1000, 2, 16, 8, False),
+                                                   ("ssd", 1, 544, 24, 64, 32, False), ("ssd", 1, 544, 24, 64, 32, True),
+                                                   ("gla", 1, 1000, 2, 64, 8, False), ("gla", 1, 544, 24, 64, 32, True)])
+def test_infinities_follow_the_recurrence(kind, B, L, H, N, seg, grad):
+    """One infinite input, or one in the initial state: y and the final state have
+    infinities and NaN exactly where the recurrence has them."""
+    ins, st = _ssd(B, L, H, 64, N, 9) if kind == "ssd" else _gla(B, L, H, 64, 9)
+    fn, ref = ((mr.ssd_scan_with_state, orc.ssd_forward) if kind == "ssd" else
+               (mr.gla_scan_with_state, orc.gla_forward))
+    if kind == "gla":
+        ins[3] = ins[3].abs().clamp(min=0.5)   # no resets: zero times infinity
+    s = L // 2 + 5
+    for k in range(5):   # u, delta, B, C (q, k, v, gates), initial state
+        xs, x0 = [t.clone() for t in ins], st.clone()
+        if k < 4:
+            xs[k][(0, s, 1, 5)[:xs[k].ndim]] = float("inf")
+        else:
+            x0[0, 1, 5, 7] = float("inf")
+        print(f"[case] inf {kind} L={L} N={N} seg={seg} grad={grad} input {k}", flush=True)
+        r = [rounded(t) for t in xs]
+        if kind == "ssd":
+            r[4] = np.repeat(r[4][:, None], N, axis=1)
+        with np.errstate(all="ignore"):
+            y_o, fs_o = ref(*r, rounded(x0))
+        if grad:
+            xs[0].requires_grad_(True)
+        y, fs = fn(*xs, seg=seg, initial_state=x0)
+        _same(y, y_o, TOL[F32])
+        _same(fs, fs_o, TOL[F32])
+
+
+def test_growing_gates_over_an_empty_start():
+    """Gates above 1 whose product over a segment overflows, over steps that add
+    nothing to a zero state: no infinity times zero."""
+    B, L, H, Dh = 1, 1000, 2, 64
+    (q, k, v, g), _ = _gla(B, L, H, Dh, 4)
+    g[:, :640], v[:, :640] = 6.0, 0.0
+    g[:, 640:] = g[:, 640:].abs().clamp(min=0.5)
+    y, fs = mr.gla_scan_with_state(q, k, v, g, seg=8)
+    y_o, fs_o = orc.gla_forward(*[rounded(t) for t in (q, k, v, g)])
+    assert np.isfinite(y_o).all()
+    _same(y, y_o, TOL[F32])
+    _same(fs, fs_o, TOL[F32])
