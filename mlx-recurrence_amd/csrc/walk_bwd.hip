@@ -71,7 +71,7 @@ struct Shape {
 struct WalkArgs {
   rr::ChunkArgs p;
   float4* mapL;    // [B*H][S-1] adjoint maps of segments 1 .. S-1 (both layouts, fragment order)
-  float* mapP;     // [B*H][S-1] their decays
+  float2* mapP;    // [B*H][S-1] their decays, each as two factors (see scaled)
   int S, cps;      // segments, chunks per segment
 };
 
@@ -87,6 +87,14 @@ struct alignas(16) WalkSm {
   float R[2][4][16];            // SSD: blocks of R_t: [0] t < 16 own, [1] t < 16 from rows >= 16, [2] t >= 16 own,
                                 // [3] row sums of the lower left block
 };
+
+// m 2^e as two factors: a segment's decay may overflow (gates above 1) where its
+// product with a small or zero adjoint does not.  The second one is 1 within
+// fp32's range.
+__device__ __forceinline__ float2 scaled(float m, int e) {
+  const int e1 = min(max(e, -100), 100), e2 = min(max(e - e1, -126), 126);
+  return make_float2(ldexpf(m, e1), ldexpf(1.f, e2));
+}
 
 // The decays M[t][s] of 16x16 block blk (0: t, s < 16; 1: t >= 16, s < 16; 2:
 // both >= 16): ROWS_T: t = 4 g + r, s = l15; else s = 4 g + r, t = l15.  Zero for
@@ -281,7 +289,8 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
   for (int dd = 0; dd < DPW; ++dd)
 #pragma unroll
     for (int nb = 0; nb < NBN; ++nb) lr[dd][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float decay = 1.f;   // MAP
+  float decay = 1.f;   // MAP: the segment's decay is decay 2^decay_e
+  int decay_e = 0;
   load(c1 - 1);
   load_step(c1 - 1);
   constexpr int MF = CPW * NBD + DPW * NBN;   // float4 per thread of a map
@@ -305,21 +314,21 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
     }
     const float4* E = q.mapL + (int64_t)bh * (q.S - 1) * (MF * T) + tid;
     for (int j = q.S - 1; j > seg; --j) {
-      const float P = q.mapP[bh * (q.S - 1) + j - 1];
+      const float2 P = q.mapP[bh * (q.S - 1) + j - 1];
       const float4* e = E + (int64_t)(j - 1) * MF * T;
 #pragma unroll
       for (int cc = 0; cc < CPW; ++cc)
 #pragma unroll
         for (int db = 0; db < NBD; ++db) {
           const float4 v = e[(cc * NBD + db) * T];
-          lc[cc][db] = f32x4_t{v.x, v.y, v.z, v.w} + P * lc[cc][db];
+          lc[cc][db] = f32x4_t{v.x, v.y, v.z, v.w} + P.x * (P.y * lc[cc][db]);
         }
 #pragma unroll
       for (int dd = 0; dd < DPW; ++dd)
 #pragma unroll
         for (int nb = 0; nb < NBN; ++nb) {
           const float4 v = e[(CPW * NBD + dd * NBN + nb) * T];
-          lr[dd][nb] = f32x4_t{v.x, v.y, v.z, v.w} + P * lr[dd][nb];
+          lr[dd][nb] = f32x4_t{v.x, v.y, v.z, v.w} + P.x * (P.y * lr[dd][nb]);
         }
     }
   }
@@ -706,7 +715,11 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
         }
       }
     }
-    if constexpr (MAP) decay *= g31;
+    if constexpr (MAP) {
+      decay *= g31;
+      decay_e += __builtin_amdgcn_frexp_expf(decay);
+      decay = __builtin_amdgcn_frexp_mantf(decay);
+    }
     lds_barrier();   // every row image and fragment read
   }
 
@@ -723,7 +736,7 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
       for (int nb = 0; nb < NBN; ++nb)
         E[(CPW * NBD + dd * NBN + nb) * T] =
             make_float4(lr[dd][nb][0], lr[dd][nb][1], lr[dd][nb][2], lr[dd][nb][3]);
-    if (tid == 0) q.mapP[bh * (q.S - 1) + seg - 1] = decay;
+    if (tid == 0) q.mapP[bh * (q.S - 1) + seg - 1] = scaled(decay, decay_e);
   } else {
     if (w == 3) step_grad(c0);
     if constexpr (!GLA) {
@@ -817,7 +830,7 @@ size_t walk_bwd_ws_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N) {
   int S, cps;
   segments(BH, nC, Dh, N, S, cps);
   if (S <= 1) return 0;
-  return (size_t)BH * (S - 1) * (2 * Dh * N + 1);   // both layouts of the map, its decay
+  return (size_t)BH * (S - 1) * (2 * Dh * N + 2);   // both layouts of the map, its decay
 }
 
 int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla) {
@@ -826,7 +839,7 @@ int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla) {
   a.p = p;
   segments(BH, p.nC, p.DH, p.NS, a.S, a.cps);
   a.mapL = reinterpret_cast<float4*>(p.agg);
-  a.mapP = p.agg == nullptr ? nullptr : p.agg + (size_t)BH * (a.S - 1) * 2 * p.DH * p.NS;
+  a.mapP = p.agg == nullptr ? nullptr : reinterpret_cast<float2*>(p.agg + (size_t)BH * (a.S - 1) * 2 * p.DH * p.NS);
   switch (p.DH * 1000 + p.NS) {
     case 64064: return gla ? launch<64, 64, true>(a, BH, s) : launch<64, 64, false>(a, BH, s);
     case 64128: return launch<64, 128, false>(a, BH, s);

@@ -61,3 +61,24 @@ def test_walk_bwd(kind, B, L, H, Dh, N):
     for name, t, want in zip(names + ["h0"], xs + [h0], grads):
         check("grad_" + name, t.grad, want, TOL[BF16], rep)
     print(rep, flush=True)
+
+
+def test_growing_gates_after_the_last_cotangent():
+    """Gates above 1 whose product over a segment overflows, after the last step
+    that the loss sees: the adjoint of a zero cotangent is zero."""
+    B, L, H, Dh = 1, 2944, 12, 64
+    rng = np.random.default_rng(7)
+    x = [rng.standard_normal((B, L, H, Dh)) / 8 for _ in range(3)]
+    g = 1 / (1 + np.exp(-(rng.standard_normal((B, L, H)) + 2)))
+    W = rng.standard_normal((B, L, H, Dh)).astype(np.float32).astype(np.float64)
+    g[:, 600] = 0
+    g[:, 601:], x[1][:, 601:], x[2][:, 600:], W[:, 600:] = 6.0, 0, 0, 0
+    xs = [to_dev(t, BF16, True) for t in (*x, g)]
+    y, _ = mr.gla_scan_with_state(*xs)
+    (y * to_dev(W, F32)).sum().backward()
+    grads = list(orc.gla_backward(W, *[rounded(t) for t in xs], None, None))
+    rep = {}
+    for name, t, want in zip(["q", "k", "v", "g"], xs, grads):
+        assert np.isfinite(want).all()
+        check("grad_" + name, t.grad, want, TOL[BF16], rep)
+    print(rep, flush=True)
