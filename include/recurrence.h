@@ -143,8 +143,8 @@ int rr_ssd_bwd(const float* dy, const float* dfinal, const void* u, const void* 
  * that forbid hipMalloc).  No counterpart in the reference.  The workspace is
  * a 16 MiB static device array of the library (one per device, held until the
  * process ends); the call allocates nothing.  A call whose
- * rr_ssd_workspace_bytes(..., pass = 1) exceeds 16 MiB returns
- * RR_EUNSUPPORTED (config 1 needs 36 KiB).  Every call on one device shares
+ * rr_ssd_bwd_workspace_bytes exceeds 16 MiB returns RR_EUNSUPPORTED (config 1
+ * needs 36 KiB).  Every call on one device shares
  * that array: calls that overlap on one GPU (other streams or threads) race.
  * Arguments and results otherwise as rr_ssd_bwd. */
 int rr_ssd_bwd_noalloc(const float* dy, const float* dfinal, const void* u, const void* delta,

@@ -1227,7 +1227,7 @@ extern "C" int rr_ssd_bwd_noalloc(const float* dy, const float* dfinal, const vo
   if (int rc = rr::check_scan_dims("ssd_bwd_noalloc", B, L, H, Dh, N, seg, dtype, "Dh")) return rc;
   if (A_stride_n != 0 && A_stride_n != 1)
     return rr::fail(RR_EINVAL, "ssd_bwd_noalloc: A_stride_n must be 0 or 1");
-  const size_t need = rr_ssd_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype, 1);
+  const size_t need = rr_ssd_bwd_workspace_bytes(B, L, H, Dh, N, seg, A_stride_n, dtype);
   if (need > kNoAllocScratchBytes)
     return rr::fail(RR_EUNSUPPORTED, "ssd_bwd_noalloc: this call needs " + std::to_string(need) +
                                          " bytes of workspace, more than the library's " +

@@ -5,6 +5,7 @@ import pathlib
 import re
 
 import pytest
+import torch
 
 from mlx_recurrence_amd import _lib
 
@@ -96,6 +97,21 @@ def test_ssd_bwd_noalloc_rejects_beyond_its_scratch(lib):
                                 1, None, None)
     assert rc == _lib.RR_EINVAL and b"L=30" in lib.rr_last_error()
 
+
+def test_ssd_bwd_noalloc_goes_by_what_the_call_needs(lib):
+    """A walking backward needs kilobytes where the per-chunk kernels' size is
+    above the scratch: it is not refused for that size (without a device it ends
+    at the lookup of the scratch), and a refusal names the call's own need."""
+    p = ctypes.c_void_p(16)
+    args = (4, 128, 80, 64, 128, 32)
+    assert lib.rr_ssd_bwd_workspace_bytes(*args, 0, 1) < (1 << 20) < (16 << 20) < lib.rr_ssd_workspace_bytes(*args, 0, 1, 1)
+    if not torch.cuda.is_available():
+        rc = lib.rr_ssd_bwd_noalloc(p, None, p, p, p, p, p, 0, 1, *args, None, p, p, p, p, p, p, 1, None, None)
+        assert rc == _lib.RR_EHIP and b"no current HIP device" in lib.rr_last_error()
+    args = (8, 4096, 80, 64, 128, 32)   # several segments: their maps
+    need = lib.rr_ssd_bwd_workspace_bytes(*args, 0, 1)
+    rc = lib.rr_ssd_bwd_noalloc(p, None, p, p, p, p, p, 0, 1, *args, None, p, p, p, p, p, p, 1, None, None)
+    assert rc == _lib.RR_EUNSUPPORTED and f"needs {need} bytes".encode() in lib.rr_last_error()
 
 def test_gdn_validation(lib):
     """Gated DeltaNet entry points: shape rules and the kernels' Dh / interval

@@ -42,6 +42,8 @@ CALLS = [
     (3, 512, 12, 64, 16, False, torch.bfloat16, 1),
     (1, 256, 4, 64, 16, False, torch.bfloat16, 2),
     (1, 64, 2, 32, 8, True, torch.float32, 3),     # dense A, fp32: the VALU engine
+    (4, 128, 80, 64, 128, False, torch.bfloat16, 4),   # the walking backward, one segment
+    (1, 1504, 24, 128, 64, False, torch.bfloat16, 5),  # several: their maps in the scratch
 ]
 
 
