@@ -8,7 +8,7 @@
 //     Y     = (M o C B^T o w_s) U + diag(gam) C h_in^T
 //     h_end = gam_31 h_in + (diag(m31 o w) U)^T B,
 // with the last chunk's missing steps taken as identity steps (zero rows, no
-// decay).  A workgroup owns a head and walks its chunks; each wave owns 16
+// decay).  A workgroup owns a head and walks its chunks; each wave owns 16 DB
 // rows d of the state for all n and never exchanges anything with the others:
 // the state lives in accumulators as h^T[n][d] (rows n), which are, element
 // for element, the B operand of C h^T, and (C B^T)^T's accumulators (rows s)
@@ -51,6 +51,11 @@ using rr::u16x4_t;
 using rr::u16x8_t;
 
 constexpr int Q = 32;
+
+// 16-row blocks of the state a wave owns.  One: two leave half the waves.  The
+// kernel stays written for any number, since the compiler's schedule of the same
+// code without the loops over blocks is slower (1 to 2 % in prompts of two chunks).
+constexpr int DB = 1;
 
 struct FinalArgs {
   const uint16_t* u;      // [B,L,H,DH] (GLA: v)
@@ -97,7 +102,7 @@ __device__ __forceinline__ int swz_d(int row) {
 
 template <int DH, int NS>
 struct alignas(16) FinalSm {
-  static constexpr int NSP = NS < 32 ? 32 : NS, NW = DH / 16;
+  static constexpr int NSP = NS < 32 ? 32 : NS, NW = DH / (16 * DB);
   uint16_t B[2][Q * NSP], C[2][Q * NSP], U[2][Q * DH];
   uint2 W[2][3][3][64];    // a chunk's W: [16x16 block][hi, mid, lo][lane], see w_block
   float sc[3][4][Q];       // a chunk's step scalars: gam, m31 w, cd (GLA: gates), w
@@ -157,7 +162,6 @@ __device__ __forceinline__ void decays(const float* st, float a, int blk, int l1
 // segP); kFinal y and the final state; kCkpt y and the state after every chunk
 // (L a multiple of 32).
 enum Out { kMap = 0, kFinal = 1, kCkpt = 2 };
-
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
 
 // The steps of chunks c0 .. c1 - 1 one after another, for a wave whose results of
@@ -215,7 +219,7 @@ __device__ __forceinline__ void by_steps(const FinalArgs& p, int bh, int c0, int
 }
 
 template <int DH, int NS, bool GLA, int OUT>
-__global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
+__global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) {
   using S = FinalSm<DH, NS>;
   constexpr int NSP = S::NSP, NW = S::NW, T = 64 * NW, NK = NSP / 32, NBN = NSP / 16;
   constexpr bool AGG = OUT == kMap;
@@ -342,30 +346,37 @@ __global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
     else stage_rows(V, buf, std::false_type{});
   };
 
-  f32x4_t hs[NBN];     // h^T[16 nb + 4 g + r][d = 16 w + l15]
-  float decay = 1.f;   // AGG: the segment's decay
-  float odd_y = 0.f;   // NaN once a value of y was not finite
+  f32x4_t hs[DB][NBN];   // h^T[16 nb + 4 g + r][d = 16 (w DB + i) + l15]
+  float decay = 1.f;     // AGG: the segment's decay
+  float odd = 0.f;       // NaN once a result was not finite
 #pragma unroll
-  for (int nb = 0; nb < NBN; ++nb) hs[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < DB; ++i)
+#pragma unroll
+    for (int nb = 0; nb < NBN; ++nb) hs[i][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   load(c0);
   if constexpr (!AGG) {
     if (p.h0 != nullptr) {
       const float* hp = p.h0 + (int64_t)bh * DH * NS;
 #pragma unroll
-      for (int nb = 0; nb < NS / 16; ++nb)
+      for (int i = 0; i < DB; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          hs[nb][r] = hp[rr::chunked::state_off<GLA, DH, NS>(16 * w + l15, 16 * nb + 4 * g + r)];
+        for (int nb = 0; nb < NS / 16; ++nb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            hs[i][nb][r] = hp[rr::chunked::state_off<GLA, DH, NS>(16 * (w * DB + i) + l15, 16 * nb + 4 * g + r)];
     }
-    const float4* E = p.segE + (int64_t)bh * (p.S - 1) * (NBN * T) + tid;
+    const float4* E = p.segE + (int64_t)bh * (p.S - 1) * (DB * NBN * T) + tid;
 #pragma unroll 2
     for (int j = 0; j < seg; ++j) {
       const float P = p.segP[bh * (p.S - 1) + j];
 #pragma unroll
-      for (int nb = 0; nb < NBN; ++nb) {
-        const float4 e = E[(j * NBN + nb) * T];
-        hs[nb] = f32x4_t{P * hs[nb][0] + e.x, P * hs[nb][1] + e.y, P * hs[nb][2] + e.z, P * hs[nb][3] + e.w};
-      }
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NBN; ++nb) {
+          const float4 e = E[(j * DB * NBN + i * NBN + nb) * T];
+          hs[i][nb] = f32x4_t{P * hs[i][nb][0] + e.x, P * hs[i][nb][1] + e.y, P * hs[i][nb][2] + e.z,
+                              P * hs[i][nb][3] + e.w};
+        }
     }
   }
   load_step(c0);
@@ -389,7 +400,7 @@ __global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
     // them they cover the stores: 99.5 -> 96.6 us at the first size above)
     const auto none = y_rows(c0, 0);
 #pragma unroll
-    for (int j = 0; j < 8 + (OUT == kCkpt ? NS / 16 : 0); ++j)
+    for (int j = 0; j < 8 * DB + (OUT == kCkpt ? DB * (NS / 16) : 0); ++j)
       __builtin_amdgcn_raw_buffer_store_b32(0u, none, 4 * lane + 256 * j, 0, 0);
   }
   lds_barrier();
@@ -409,12 +420,15 @@ __global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
     const float(*sc)[Q] = sm.sc[c % 3];
     const float tot = sc[0][Q - 1];
     // U as B operand: U[pi(g, e)][d]
-    u16x8_t uf;
+    u16x8_t uf[DB];
     {
       const int r0 = 4 * g + (l15 >> 2), q = l15 & 3;
-      const uint16_t* up = Us + r0 * DH + 8 * ((2 * w + (q >> 1)) ^ swz_d<DH>(r0)) + 4 * (q & 1);
-      const u16x4_t lo = rr::tr_read4(up), hi = rr::tr_read4(up + 16 * DH);
-      uf = u16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        const uint16_t* up = Us + r0 * DH + 8 * ((2 * (w * DB + i) + (q >> 1)) ^ swz_d<DH>(r0)) + 4 * (q & 1);
+        const u16x4_t lo = rr::tr_read4(up), hi = rr::tr_read4(up + 16 * DH);
+        uf[i] = u16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
     }
     if constexpr (!AGG) {
       u16x8_t cf[2][NK];   // C[16 tb + l15][32 kk + pi]
@@ -431,86 +445,92 @@ __global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
         wf[0][k] = __builtin_bit_cast(u16x8_t, make_uint4(x0.x, x0.y, 0, 0));
         wf[1][k] = __builtin_bit_cast(u16x8_t, make_uint4(x1.x, x1.y, x2.x, x2.y));
       }
-      f32x4_t ab[2], as[2];   // C h^T: hi terms, mid + lo terms
-      ab[0] = ab[1] = as[0] = as[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < NK; ++kk) {
-        const float x[8] = {hs[2 * kk][0],     hs[2 * kk][1],     hs[2 * kk][2],     hs[2 * kk][3],
-                            hs[2 * kk + 1][0], hs[2 * kk + 1][1], hs[2 * kk + 1][2], hs[2 * kk + 1][3]};
-        u16x8_t hh, hm, hl;
-        split3(x, hh, hm, hl);
+      for (int i = 0; i < DB; ++i) {
+        f32x4_t ab[2], as[2];   // C h^T: hi terms, mid + lo terms
+        ab[0] = ab[1] = as[0] = as[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+          const float x[8] = {hs[i][2 * kk][0],     hs[i][2 * kk][1],     hs[i][2 * kk][2],     hs[i][2 * kk][3],
+                              hs[i][2 * kk + 1][0], hs[i][2 * kk + 1][1], hs[i][2 * kk + 1][2], hs[i][2 * kk + 1][3]};
+          u16x8_t hh, hm, hl;
+          split3(x, hh, hm, hl);
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb) {
+            as[tb] = rr::mfma16(cf[tb][kk], hl, as[tb]);
+            ab[tb] = rr::mfma16(cf[tb][kk], hh, ab[tb]);
+            as[tb] = rr::mfma16(cf[tb][kk], hm, as[tb]);
+          }
+        }
+        // a non-finite u must not reach the steps before it through W's zeros:
+        // such elements leave the product and are added step by step below
+        u16x8_t ui = uf[i];
+        bool inf_u = false;
+        {
+          uint4 x = __builtin_bit_cast(uint4, ui);
+          auto over = [](uint32_t v) { return ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u; };
+          inf_u = (over(x.x) | over(x.y) | over(x.z) | over(x.w)) != 0;
+        }
+        const bool any_odd = __any(inf_u);
+        if (__builtin_expect(any_odd, 0)) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ui[e] = (ui[e] & 0x7f80) == 0x7f80 ? 0 : ui[e];
+        }
+        f32x4_t o[2];
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
-          as[tb] = rr::mfma16(cf[tb][kk], hl, as[tb]);
-          ab[tb] = rr::mfma16(cf[tb][kk], hh, ab[tb]);
-          as[tb] = rr::mfma16(cf[tb][kk], hm, as[tb]);
+          f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          z = rr::mfma16(wf[tb][2], ui, z);
+          z = rr::mfma16(wf[tb][1], ui, z);
+          const float4 gm = *reinterpret_cast<const float4*>(&sc[0][16 * tb + 4 * g]);
+          z = f32x4_t{gm.x * (ab[tb][0] + as[tb][0]) + z[0], gm.y * (ab[tb][1] + as[tb][1]) + z[1],
+                      gm.z * (ab[tb][2] + as[tb][2]) + z[2], gm.w * (ab[tb][3] + as[tb][3]) + z[3]};
+          o[tb] = rr::mfma16(wf[tb][0], ui, z);
         }
-      }
-      // a non-finite u must not reach the steps before it through W's zeros:
-      // such elements leave the product and are added step by step below
-      u16x8_t ui = uf;
-      bool odd = false;
-      {
-        uint4 x = __builtin_bit_cast(uint4, ui);
-        auto over = [](uint32_t v) { return ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u; };
-        odd = (over(x.x) | over(x.y) | over(x.z) | over(x.w)) != 0;
-      }
-      const bool any_odd = __any(odd);
-      if (any_odd) {
+        if (__builtin_expect(any_odd, 0)) {
+          for (int s = 0; s < Q; ++s) {
+            const int src = 16 * ((s >> 2) & 3), e = (s & 3) + 4 * (s >> 4);
+            float us = 0.f, ws0 = 0.f, ws1 = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ui[e] = (ui[e] & 0x7f80) == 0x7f80 ? 0 : ui[e];
-      }
-      f32x4_t o[2];
+            for (int k = 0; k < 8; ++k) {
+              us = k == e ? rr::bf_val(uf[i][k]) : us;
+              ws0 = k == e ? rr::bf_val(wf[0][0][k]) + rr::bf_val(wf[0][1][k]) : ws0;
+              ws1 = k == e ? rr::bf_val(wf[1][0][k]) + rr::bf_val(wf[1][1][k]) : ws1;
+            }
+            us = __shfl(us, src + l15);
+            const bool add = !(fabsf(us) < __builtin_inff());   // the elements left out above
 #pragma unroll
-      for (int tb = 0; tb < 2; ++tb) {
-        f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-        z = rr::mfma16(wf[tb][2], ui, z);
-        z = rr::mfma16(wf[tb][1], ui, z);
-        const float4 gm = *reinterpret_cast<const float4*>(&sc[0][16 * tb + 4 * g]);
-        z = f32x4_t{gm.x * (ab[tb][0] + as[tb][0]) + z[0], gm.y * (ab[tb][1] + as[tb][1]) + z[1],
-                    gm.z * (ab[tb][2] + as[tb][2]) + z[2], gm.w * (ab[tb][3] + as[tb][3]) + z[3]};
-        o[tb] = rr::mfma16(wf[tb][0], ui, z);
-      }
-      if (any_odd) {
-        for (int s = 0; s < Q; ++s) {
-          const int src = 16 * ((s >> 2) & 3), e = (s & 3) + 4 * (s >> 4);
-          float us = 0.f, ws0 = 0.f, ws1 = 0.f;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            us = k == e ? rr::bf_val(uf[k]) : us;
-            ws0 = k == e ? rr::bf_val(wf[0][0][k]) + rr::bf_val(wf[0][1][k]) : ws0;
-            ws1 = k == e ? rr::bf_val(wf[1][0][k]) + rr::bf_val(wf[1][1][k]) : ws1;
-          }
-          us = __shfl(us, src + l15);
-          const bool add = !(fabsf(us) < __builtin_inff());   // the elements left out above
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float v0 = __shfl(ws0, src + 4 * g + r), v1 = __shfl(ws1, src + 4 * g + r);
-            if (add && s <= 4 * g + r) o[0][r] += v0 * us;
-            if (add && s <= 16 + 4 * g + r) o[1][r] += v1 * us;
+            for (int r = 0; r < 4; ++r) {
+              const float v0 = __shfl(ws0, src + 4 * g + r), v1 = __shfl(ws1, src + 4 * g + r);
+              if (add && s <= 4 * g + r) o[0][r] += v0 * us;
+              if (add && s <= 16 + 4 * g + r) o[1][r] += v1 * us;
+            }
           }
         }
-      }
-      const auto yr = y_rows(c, min(p.L - c * Q, Q));
+        const auto yr = y_rows(c, min(p.L - c * Q, Q));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v = o[j >> 2][j & 3];   // (a copy: a bit cast of a vector's element takes the first one)
-        odd_y = fmaf(v, 0.f, odd_y);
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr,
-                                              (int)(4u * ((uint32_t)(16 * (j >> 2) + 4 * g + (j & 3)) * rsD + l15)),
-                                              64 * w, 0);
+        for (int j = 0; j < 8; ++j) {
+          const float v = o[j >> 2][j & 3];   // (a copy: a bit cast of a vector's element takes the first one)
+          odd = fmaf(v, 0.f, odd);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr,
+                                                (int)(4u * ((uint32_t)(16 * (j >> 2) + 4 * g + (j & 3)) * rsD + l15)),
+                                                64 * (w * DB + i), 0);
+        }
       }
     }
     // h^T <- gam_31 h^T + B^T (m31 w o U): B^T transposed reads are the exact A operand
-    u16x8_t us[3];
+    u16x8_t us[DB][3];
     {
       const float4 x0 = *reinterpret_cast<const float4*>(&sc[1][4 * g]);
       const float4 x1 = *reinterpret_cast<const float4*>(&sc[1][16 + 4 * g]);
       const float mw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      float x[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = mw[e] * rr::bf_val(uf[e]);
-      split3(x, us[0], us[1], us[2]);
+      for (int i = 0; i < DB; ++i) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = mw[e] * rr::bf_val(uf[i][e]);
+        split3(x, us[i][0], us[i][1], us[i][2]);
+      }
     }
     {
       const int r0 = 4 * g + (l15 >> 2), f = swz_n<NSP>(r0);
@@ -519,55 +539,67 @@ __global__ __launch_bounds__(4 * DH, 2) void final_fwd_kernel(FinalArgs p) {
         const uint16_t* bp = Bs + r0 * NSP + 8 * ((4 * (nb >> 1) + (l15 & 3)) ^ f) + 4 * (nb & 1);
         const u16x4_t lo = rr::tr_read4(bp), hi = rr::tr_read4(bp + 16 * NSP);
         const u16x8_t bt = u16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-        z = rr::mfma16(bt, us[2], z);
-        z = rr::mfma16(bt, us[1], z);
-        z = rr::mfma16(bt, us[0], z);
-        hs[nb] = f32x4_t{tot * hs[nb][0] + z[0], tot * hs[nb][1] + z[1], tot * hs[nb][2] + z[2],
-                         tot * hs[nb][3] + z[3]};
+#pragma unroll
+        for (int i = 0; i < DB; ++i) {
+          f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          z = rr::mfma16(bt, us[i][2], z);
+          z = rr::mfma16(bt, us[i][1], z);
+          z = rr::mfma16(bt, us[i][0], z);
+          hs[i][nb] = f32x4_t{tot * hs[i][nb][0] + z[0], tot * hs[i][nb][1] + z[1], tot * hs[i][nb][2] + z[2],
+                              tot * hs[i][nb][3] + z[3]};
+        }
       }
     }
     if constexpr (AGG) decay *= tot;
     if constexpr (OUT == kCkpt) {
       float* ck = p.fin + ((int64_t)bh * p.nC + c) * DH * NS;
 #pragma unroll
-      for (int nb = 0; nb < NS / 16; ++nb)
-        *reinterpret_cast<float4*>(ck + (16 * w + l15) * NS + 16 * nb + 4 * g) =
-            make_float4(hs[nb][0], hs[nb][1], hs[nb][2], hs[nb][3]);
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NS / 16; ++nb)
+          *reinterpret_cast<float4*>(ck + (16 * (w * DB + i) + l15) * NS + 16 * nb + 4 * g) =
+              make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
     }
     lds_barrier();
   }
 
   if constexpr (!AGG) {
-    bool odd = odd_y != 0.f;   // (NaN; a state once not finite stays so)
 #pragma unroll
-    for (int nb = 0; nb < NBN; ++nb)
+    for (int i = 0; i < DB; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) odd |= !finite(hs[nb][r]);
-    if (__any(odd)) {
+      for (int nb = 0; nb < NBN; ++nb)   // (a state once not finite stays so)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) odd = fmaf(hs[i][nb][r], 0.f, odd);
+    if (__builtin_expect(__any(odd != 0.f), 0)) {
       __threadfence_block();   // the wave reads its own stores back
-      by_steps<DH, NS, GLA, OUT>(p, bh, c0, c1, 16 * w + l15, g, hs);
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+        by_steps<DH, NS, GLA, OUT>(p, bh, c0, c1, 16 * (w * DB + i) + l15, g, hs[i]);
     }
   }
   if constexpr (AGG) {
-    float4* E = p.segE + ((int64_t)bh * (p.S - 1) + seg) * (NBN * T) + tid;
+    float4* E = p.segE + ((int64_t)bh * (p.S - 1) + seg) * (DB * NBN * T) + tid;
 #pragma unroll
-    for (int nb = 0; nb < NBN; ++nb)
-      E[nb * T] = make_float4(hs[nb][0], hs[nb][1], hs[nb][2], hs[nb][3]);
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NBN; ++nb)
+        E[(i * NBN + nb) * T] = make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
     if (tid == 0) p.segP[bh * (p.S - 1) + seg] = decay;
   } else if (OUT == kFinal && seg == p.S - 1) {
     float* fp = p.fin + (int64_t)bh * DH * NS;
 #pragma unroll
-    for (int nb = 0; nb < NS / 16; ++nb) {
-      const int d = 16 * w + l15, n = 16 * nb + 4 * g;
-      if constexpr (GLA) {
+    for (int i = 0; i < DB; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) fp[(n + r) * DH + d] = hs[nb][r];
-      } else {
-        *reinterpret_cast<float4*>(fp + d * NS + n) =
-            make_float4(hs[nb][0], hs[nb][1], hs[nb][2], hs[nb][3]);
+      for (int nb = 0; nb < NS / 16; ++nb) {
+        const int d = 16 * (w * DB + i) + l15, n = 16 * nb + 4 * g;
+        if constexpr (GLA) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) fp[(n + r) * DH + d] = hs[i][nb][r];
+        } else {
+          *reinterpret_cast<float4*>(fp + d * NS + n) =
+              make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
+        }
       }
-    }
   }
 }
 
