@@ -701,15 +701,26 @@ namespace rr {
 // - fewer than 24 heads: the chunk-parallel kernels (SSD 2 heads, 32 chunks,
 //   Dh 64 N 128: 15.9 against 19.7; at 24 heads, 17 chunks 22.3 against 20.8);
 // - in shorter heads the resident and direct kernels are more parallel
-//   (SSD 36 heads, 16 chunks, Dh 64 N 16: 9.5 against 16.3) except N = 64 from
-//   256 heads (66 -> 44 at 320 heads, 16 chunks) and N = 128, which the
-//   resident kernel does not cover, below 512 heads (123 -> 94) unless GLA's
-//   wide direct mode takes it (BH nC <= 768: 23 against 31).
+//   (SSD 36 heads, 16 chunks, Dh 64 N 16: 9.5 against 16.3) except
+//   N = 64 from 256 heads (66 -> 44 at 320 heads, 16 chunks; 8.8 -> 6.5 at 256
+//   heads, 1 chunk) unless the whole-head kernel, from 512 heads, has but one
+//   or two chunks to carry (1 chunk: 8.3 against 8.8 at 512 heads, 26.6 against
+//   31.6 at 2560; 2 chunks: 17.0 -> 15.9 at 640, 19.3 against 20.7 at 800; 3
+//   chunks: even from 960), and
+//   N = 128, which the resident kernel does not cover, below 512 heads (16
+//   chunks: 123 -> 94; 8: 46 -> 36 at 256 heads; 1: 10.2 -> 6.4 at 24), unless
+//   GLA's wide direct mode takes it (BH nC <= 768: 23 against 31) or Dh is 32
+//   with 4 or 5 chunks of few heads, where a second segment's launch costs more
+//   than the direct or pipelined kernels (4 chunks: 12.5 against 13.9 at 64
+//   heads, 19.2 -> 14.0 at 72; 5: 15.1 against 16.2 at 48, 17.0 -> 16.5 at 56).
 bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla) {
   if (BH < 24 || !grid_ok(BH, 4 * Dh)) return false;
   if (nC > 16) return N >= 64 || (nC >= 32 && (N == 32 || BH <= 256));
-  if (N == 128) return BH < 512 && !(gla && BH * nC <= 768);
-  return N == 64 && Dh == 64 && BH >= 256;
+  if (N == 128) {
+    if (Dh == 32 && ((nC == 4 && BH <= 64) || (nC == 5 && BH <= 48))) return false;
+    return BH < 512 && !(gla && BH * nC <= 768);
+  }
+  return N == 64 && Dh == 64 && BH >= 256 && (nC >= 3 || BH < 256 * (nC + 1));
 }
 
 size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {

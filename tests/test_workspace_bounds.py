@@ -100,3 +100,16 @@ def test_wide_direct_mode_workspace_at_the_published_shape():
     assert int(lib.rr_ssd_workspace_bytes(5, L, H, Dh, N, 32, 0, BF16, 0)) == 0
     assert int(lib.rr_ssd_workspace_bytes(5, L, H, Dh, N, 32, 0, BF16, 1)) == \
         al(5 * H * nC * 4) + al(5 * H * nC * N * 4) + al(5 * H * nC * Dh * N * 4)
+
+
+def test_few_short_heads_of_dh_32_run_the_direct_kernel():
+    """Dh 32, N 128, 4 chunks: one direct kernel (no workspace) up to 64 heads,
+    the walk in two segments (their maps) from there; 5 chunks: the pipelined
+    kernels (per-chunk decays) up to 48 heads."""
+    lib = _lib.load()
+
+    def fwd(H, nC):
+        return int(lib.rr_ssd_workspace_bytes(1, 32 * nC, H, 32, 128, 32, 0, BF16, 0))
+
+    assert fwd(24, 4) == fwd(64, 4) == 0 and fwd(72, 4) > 72 * 32 * 128 * 4
+    assert 0 < fwd(48, 5) < 4096 and fwd(56, 5) > 56 * 32 * 128 * 4
