@@ -110,14 +110,20 @@ size_t rr_ssd_bwd_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t Dh, i
 /* One past the largest workspace byte that the per-chunk (MFMA) SSD kernels of
  * this call write or read: the library walks the grids of the pass's kernels
  * with their own workgroup decode and slot arithmetic.  For tests that the
- * kernels stay inside rr_ssd_workspace_bytes.  (For calls whose backward walks
- * a head's chunks instead it bounds the per-chunk kernels they would take
- * otherwise.)  No reference counterpart.
+ * kernels stay inside rr_ssd_workspace_bytes.  (With pass = 1, for calls whose
+ * backward walks a head's chunks, it bounds the per-chunk kernels they would take
+ * otherwise: rr_ssd_bwd_workspace_extent bounds the walk.)  No reference
+ * counterpart.
  * Returns -1 for invalid arguments or a call that the chunked bf16 kernels do
  * not run (the fp32-MFMA and VALU paths carve fixed regions of the size
  * rr_ssd_workspace_bytes returns). */
 int64_t rr_ssd_workspace_extent(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
                                 int64_t A_stride_n, int dtype, int pass);
+
+/* The same for the kernels that rr_ssd_bwd runs, to hold against
+ * rr_ssd_bwd_workspace_bytes. */
+int64_t rr_ssd_bwd_workspace_extent(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
+                                    int64_t A_stride_n, int dtype);
 
 /* Replaces _ssd_forward_kernel (reference mlx_recurrence/ssd.py:54-135). */
 int rr_ssd_fwd(const void* u, const void* delta, const void* Bm, const void* Cm,

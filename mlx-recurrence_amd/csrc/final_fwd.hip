@@ -365,10 +365,10 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
           for (int r = 0; r < 4; ++r)
             hs[i][nb][r] = hp[rr::chunked::state_off<GLA, DH, NS>(16 * (w * DB + i) + l15, 16 * nb + 4 * g + r)];
     }
-    const float4* E = p.segE + (int64_t)bh * (p.S - 1) * (DB * NBN * T) + tid;
+    const float4* E = p.segE + rr::chunked::map_slot(bh, p.S, 0) * (DB * NBN * T) + tid;
 #pragma unroll 2
     for (int j = 0; j < seg; ++j) {
-      const float P = p.segP[bh * (p.S - 1) + j];
+      const float P = p.segP[rr::chunked::map_slot(bh, p.S, j)];
 #pragma unroll
       for (int i = 0; i < DB; ++i)
 #pragma unroll
@@ -578,13 +578,13 @@ __global__ __launch_bounds__(4 * DH / DB, 2) void final_fwd_kernel(FinalArgs p) 
     }
   }
   if constexpr (AGG) {
-    float4* E = p.segE + ((int64_t)bh * (p.S - 1) + seg) * (DB * NBN * T) + tid;
+    float4* E = p.segE + rr::chunked::map_slot(bh, p.S, seg) * (DB * NBN * T) + tid;
 #pragma unroll
     for (int i = 0; i < DB; ++i)
 #pragma unroll
       for (int nb = 0; nb < NBN; ++nb)
         E[(i * NBN + nb) * T] = make_float4(hs[i][nb][0], hs[i][nb][1], hs[i][nb][2], hs[i][nb][3]);
-    if (tid == 0) p.segP[bh * (p.S - 1) + seg] = decay;
+    if (tid == 0) p.segP[rr::chunked::map_slot(bh, p.S, seg)] = decay;
   } else if (OUT == kFinal && seg == p.S - 1) {
     float* fp = p.fin + (int64_t)bh * DH * NS;
 #pragma unroll
@@ -621,10 +621,11 @@ void segments(int64_t BH, int64_t nC, int64_t Dh, int& S, int& cps) {
   S = (int)((nC + cps - 1) / cps);
 }
 
+// Workspace: the segments' states, then their decays.
+size_t map_bytes(int64_t Dh, int64_t N) { return (size_t)Dh * (size_t)std::max<int64_t>(N, 32) * 4; }
+size_t decay_offset(int64_t BH, int64_t Dh, int64_t N, int S) { return (size_t)BH * (S - 1) * map_bytes(Dh, N); }
 size_t ws_bytes(int64_t BH, int64_t Dh, int64_t N, int S) {
-  if (S <= 1) return 0;
-  const size_t state = (size_t)Dh * (size_t)std::max<int64_t>(N, 32) * 4;
-  return (size_t)BH * (S - 1) * (state + 4) + 256;
+  return S <= 1 ? 0 : decay_offset(BH, Dh, N, S) + (size_t)BH * (S - 1) * 4 + 256;
 }
 
 template <int DH, int NS, bool GLA, int OUT>
@@ -646,7 +647,7 @@ int run(FinalArgs& p, int64_t B, int64_t H, int64_t Dh, int64_t N, void* ws, siz
   if (need > 0) {
     if (ws == nullptr || wsb < need) return rr::fail(RR_EWORKSPACE, "final-state forward: workspace too small");
     p.segE = static_cast<float4*>(ws);
-    p.segP = reinterpret_cast<float*>(static_cast<char*>(ws) + (size_t)BH * (p.S - 1) * Dh * std::max<int64_t>(N, 32) * 4);
+    p.segP = reinterpret_cast<float*>(static_cast<char*>(ws) + decay_offset(BH, Dh, N, p.S));
   }
 #define RR_CASE(D, NN) \
   if (Dh == D && N == NN) return launch<D, NN, GLA, OUT>(p, BH, s)
@@ -727,6 +728,21 @@ size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
   int S, cps;
   segments(B * H, nC, Dh, S, cps);
   return ws_bytes(B * H, Dh, N, S);
+}
+
+int64_t walk_ws_extent(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
+  int S, cps;
+  segments(B * H, nC, Dh, S, cps);
+  const int64_t T = 4 * Dh, frags = std::max<int64_t>(N, 32) / 16;   // threads, float4 a thread keeps of a map
+  const int64_t decays = S > 1 ? (int64_t)decay_offset(B * H, Dh, N, S) : 0;
+  int64_t ext = 0;
+  for (int64_t bh = 0; bh < B * H; ++bh)
+    for (int j = 0; j + 1 < S; ++j) {
+      const int64_t slot = chunked::map_slot(bh, S, j);
+      if ((slot * frags * T + (frags - 1) * T + T) * 16 > decays) return INT64_MAX;   // into the decays
+      ext = std::max(ext, decays + (slot + 1) * 4);
+    }
+  return ext;
 }
 
 int walk_fwd(const ChunkArgs& a, int64_t B, hipStream_t s, bool gla) {

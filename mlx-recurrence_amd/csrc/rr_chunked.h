@@ -190,6 +190,10 @@ __device__ __forceinline__ int state_off(int d, int n) {
 //           waves that own rows of the state (final_fwd.hip).
 enum Mode { kWhole = 0, kPipe = 1, kDirect = 2, kSum = 3, kRes = 4, kPair = 5, kWalk = 6 };
 
+// Slot of map j (0 .. S - 2) of head bh among the segment maps of the walking
+// kernels (one map fewer than segments).
+__host__ __device__ inline int64_t map_slot(int64_t bh, int S, int j) { return bh * (S - 1) + j; }
+
 // Per-chunk kernels run on a 1-D grid of chunk_grid(p) workgroups.  The GPU
 // hands workgroups to its 8 XCDs round-robin by linear index; the decode
 // gives every chunk of a head the same XCD (x = index % 8), so whatever the

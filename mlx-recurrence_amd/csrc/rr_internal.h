@@ -109,6 +109,8 @@ int res_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 // segments' maps; none for one segment).
 bool walk_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N, bool gla);   // faster than the other modes
 size_t walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
+// One past the last workspace byte of its slots, for tests (INT64_MAX: slots overlap).
+int64_t walk_ws_extent(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
 int walk_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 
 // Backward with a head's chunks walked, the adjoint in registers
@@ -118,9 +120,12 @@ int walk_fwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 bool walk_bwd_preferred(int64_t BH, int64_t nC, int64_t Dh, int64_t N);   // covered, and faster than the other modes
 int walk_bwd_chunks(int64_t BH, int64_t nC, int64_t Dh, int64_t N);
 size_t walk_bwd_ws_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N);
+// One past the last float of its slots there, and the segment count, for tests.
+int64_t walk_bwd_extent_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N, int& S);
 int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla);
 // The SSD backward by that kernel and its dA reduction, and its workspace.
 size_t ssd2_walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
+int64_t ssd2_walk_ws_extent(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N);
 int ssd2_walk_bwd(ChunkArgs& p, void* ws, int64_t B, hipStream_t s);
 
 // Gated DeltaNet forward in chunkwise (WY) form (gdn_chunk.hip): bf16, Dh 64,

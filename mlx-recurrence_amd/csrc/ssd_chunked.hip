@@ -949,7 +949,7 @@ int64_t ssd2_ws_extent(int64_t B, int64_t H, int64_t nC, int mode, int64_t Dh, i
     if (region == nullptr) return;
     ext = std::max<int64_t>(ext, reinterpret_cast<const char*>(region + first + count) - base);
   };
-  if (mode == kWalk) return (int64_t)walk_ws_bytes(B, H, nC, Dh, N);   // (its maps fill it)
+  if (mode == kWalk) return walk_ws_extent(B, H, nC, Dh, N);
   const int64_t state = Dh * N, BH = B * H;
   const bool pipe = mode == kPipe || mode == kPair;
   if (pipe && BH < kScanMinHeads) {
@@ -995,6 +995,17 @@ int64_t ssd2_ws_extent(int64_t B, int64_t H, int64_t nC, int mode, int64_t Dh, i
 size_t ssd2_walk_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
   const int64_t R = walk_bwd_chunks(B * H, nC, Dh, N), nR = (nC + R - 1) / R;
   return ((size_t)align64(B * H * nR * N) + walk_bwd_ws_floats(B * H, nC, Dh, N)) * sizeof(float);
+}
+
+int64_t ssd2_walk_ws_extent(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
+  const int64_t R = walk_bwd_chunks(B * H, nC, Dh, N), nR = (nC + R - 1) / R, agg = align64(B * H * nR * N);
+  int S;
+  const int64_t maps = walk_bwd_extent_floats(B * H, nC, Dh, N, S);
+  int64_t partials = 0;   // dA, one per segment
+  for (int64_t bh = 0; bh < B * H; ++bh)
+    for (int seg = 0; seg < S; ++seg) partials = std::max(partials, chunked::dA_slot(bh, S, seg) * N + N);
+  if (partials > agg || maps == INT64_MAX) return INT64_MAX;   // slots overlap
+  return (S > 1 ? agg + maps : partials) * (int64_t)sizeof(float);
 }
 
 int ssd2_walk_bwd(ChunkArgs& p, void* ws, int64_t B, hipStream_t s) {

@@ -1017,6 +1017,15 @@ extern "C" int64_t rr_ssd_workspace_extent(int64_t B, int64_t L, int64_t H, int6
   return rr::ssd2_ws_extent(B, H, nC, rr::chunked_mode(B, H, nC, Dh, N, pass), Dh, N, pass);
 }
 
+extern "C" int64_t rr_ssd_bwd_workspace_extent(int64_t B, int64_t L, int64_t H, int64_t Dh, int64_t N, int64_t seg,
+                                               int64_t A_stride_n, int dtype) {
+  if (B > 0 && L > 0 && H > 0 && Dh > 0 && N > 0 && rr::chunk_len(L, seg) != 0 &&
+      rr::ssd2_supported(dtype, L, seg, Dh, N, A_stride_n) && rr::ssd2_bwd_supported(Dh, N) &&
+      rr::walk_bwd_preferred(B * H, L / 32, Dh, N))
+    return rr::ssd2_walk_ws_extent(B, H, L / 32, Dh, N);
+  return rr_ssd_workspace_extent(B, L, H, Dh, N, seg, A_stride_n, dtype, 1);
+}
+
 extern "C" int rr_ssd_fwd(const void* u, const void* delta, const void* Bm, const void* Cm,
                           const float* A_neg, int64_t A_stride_n, int dtype, int64_t B, int64_t L, int64_t H,
                           int64_t Dh, int64_t N, int64_t seg, const float* h0, float* y,

@@ -312,9 +312,9 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
           for (int r = 0; r < 4; ++r)
             lr[dd][nb][r] = dp[rr::chunked::state_off<GLA, DH, NS>(16 * (w * DPW + dd) + l15, 16 * nb + 4 * g + r)];
     }
-    const float4* E = q.mapL + (int64_t)bh * (q.S - 1) * (MF * T) + tid;
+    const float4* E = q.mapL + rr::chunked::map_slot(bh, q.S, 0) * (MF * T) + tid;
     for (int j = q.S - 1; j > seg; --j) {
-      const float2 P = q.mapP[bh * (q.S - 1) + j - 1];
+      const float2 P = q.mapP[rr::chunked::map_slot(bh, q.S, j - 1)];
       const float4* e = E + (int64_t)(j - 1) * MF * T;
 #pragma unroll
       for (int cc = 0; cc < CPW; ++cc)
@@ -724,7 +724,7 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
   }
 
   if constexpr (MAP) {
-    float4* E = q.mapL + ((int64_t)bh * (q.S - 1) + seg - 1) * (MF * T) + tid;
+    float4* E = q.mapL + rr::chunked::map_slot(bh, q.S, seg - 1) * (MF * T) + tid;
 #pragma unroll
     for (int cc = 0; cc < CPW; ++cc)
 #pragma unroll
@@ -736,7 +736,7 @@ __global__ __launch_bounds__((Shape<DH, NS>::T), 2) void walk_bwd_kernel(WalkArg
       for (int nb = 0; nb < NBN; ++nb)
         E[(CPW * NBD + dd * NBN + nb) * T] =
             make_float4(lr[dd][nb][0], lr[dd][nb][1], lr[dd][nb][2], lr[dd][nb][3]);
-    if (tid == 0) q.mapP[bh * (q.S - 1) + seg - 1] = scaled(decay, decay_e);
+    if (tid == 0) q.mapP[rr::chunked::map_slot(bh, q.S, seg - 1)] = scaled(decay, decay_e);
   } else {
     if (w == 3) step_grad(c0);
     if constexpr (!GLA) {
@@ -794,6 +794,9 @@ void segments(int64_t BH, int64_t nC, int64_t Dh, int64_t N, int& S, int& cps) {
   }
 }
 
+// Workspace floats: both layouts of every map, then the decays (two floats each).
+size_t decay_offset(int64_t BH, int64_t Dh, int64_t N, int S) { return (size_t)BH * (S - 1) * 2 * Dh * N; }
+
 template <int DH, int NS, bool GLA>
 int launch(const WalkArgs& a, int64_t BH, hipStream_t s) {
   constexpr int T = Shape<DH, NS>::T;
@@ -826,11 +829,27 @@ int walk_bwd_chunks(int64_t BH, int64_t nC, int64_t Dh, int64_t N) {
   return cps;
 }
 
+int64_t walk_bwd_extent_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N, int& S) {
+  int cps;
+  segments(BH, nC, Dh, N, S, cps);
+  const int64_t NW = Dh == 128 && N == 128 ? 8 : 4, T = 64 * NW;   // Shape's
+  const int64_t frags = N / 16 / NW * (Dh / 16) + Dh / 16 / NW * (N / 16);
+  const int64_t decays = S > 1 ? (int64_t)decay_offset(BH, Dh, N, S) : 0;
+  int64_t ext = 0;
+  for (int64_t bh = 0; bh < BH; ++bh)
+    for (int seg = 1; seg < S; ++seg) {
+      const int64_t slot = chunked::map_slot(bh, S, seg - 1);
+      if ((slot * frags * T + (frags - 1) * T + T) * 4 > decays) return INT64_MAX;   // into the decays
+      ext = std::max(ext, decays + (slot + 1) * 2);
+    }
+  return ext;
+}
+
 size_t walk_bwd_ws_floats(int64_t BH, int64_t nC, int64_t Dh, int64_t N) {
   int S, cps;
   segments(BH, nC, Dh, N, S, cps);
   if (S <= 1) return 0;
-  return (size_t)BH * (S - 1) * (2 * Dh * N + 2);   // both layouts of the map, its decay
+  return decay_offset(BH, Dh, N, S) + (size_t)BH * (S - 1) * 2;
 }
 
 int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla) {
@@ -839,7 +858,7 @@ int walk_bwd(const ChunkArgs& p, int64_t B, hipStream_t s, bool gla) {
   a.p = p;
   segments(BH, p.nC, p.DH, p.NS, a.S, a.cps);
   a.mapL = reinterpret_cast<float4*>(p.agg);
-  a.mapP = p.agg == nullptr ? nullptr : reinterpret_cast<float2*>(p.agg + (size_t)BH * (a.S - 1) * 2 * p.DH * p.NS);
+  a.mapP = p.agg == nullptr ? nullptr : reinterpret_cast<float2*>(p.agg + decay_offset(BH, p.DH, p.NS, a.S));
   switch (p.DH * 1000 + p.NS) {
     case 64064: return gla ? launch<64, 64, true>(a, BH, s) : launch<64, 64, false>(a, BH, s);
     case 64128: return launch<64, 128, false>(a, BH, s);

@@ -45,6 +45,7 @@ _SIGS = {
     "rr_ssd_workspace_bytes": (_c_size, [_c_i64] * 7 + [_c_int, _c_int]),
     "rr_ssd_bwd_workspace_bytes": (_c_size, [_c_i64] * 7 + [_c_int]),
     "rr_ssd_workspace_extent": (_c_i64, [_c_i64] * 7 + [_c_int, _c_int]),
+    "rr_ssd_bwd_workspace_extent": (_c_i64, [_c_i64] * 7 + [_c_int]),
     "rr_ssd_fwd": (_c_int, [_c_ptr] * 5 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 4 + [_c_size, _c_ptr]),
     "rr_ssd_bwd": (_c_int, [_c_ptr] * 7 + [_c_i64, _c_int] + [_c_i64] * 6 + [_c_ptr] * 7 + [_c_i64]
                    + [_c_ptr] * 2 + [_c_size, _c_ptr]),
@@ -162,6 +163,11 @@ def ssd_workspace_extent(B: int, L: int, H: int, Dh: int, N: int, seg: int, a_st
     pass touch (walked over their grids by the library), or -1 where the call
     runs on the fp32-MFMA or VALU paths (fixed workspace regions)."""
     return int(load().rr_ssd_workspace_extent(B, L, H, Dh, N, seg, a_stride_n, dtype, pass_))
+
+
+def ssd_bwd_workspace_extent(B: int, L: int, H: int, Dh: int, N: int, seg: int, a_stride_n: int, dtype: int) -> int:
+    """The same for the kernels that ssd_bwd runs (a walking backward among them)."""
+    return int(load().rr_ssd_bwd_workspace_extent(B, L, H, Dh, N, seg, a_stride_n, dtype))
 
 
 def _check(rc: int, what: str) -> None:

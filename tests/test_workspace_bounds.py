@@ -2,15 +2,17 @@
 
 The adjoint scan writes one adjoint per run of R chunks of each head into the
 backward workspace, the pipelined and pair chunk kernels read them back, and
-every backward workgroup writes a dA partial there.  A slot computed past the
+every backward workgroup writes a dA partial there; the walking kernels write
+and read one map per segment of a head's chunks.  A slot computed past the
 end of the workspace is an out-of-bounds write on the GPU (the pair mode's
 first run did exactly that: its scan spaced each head's slots nC apart where
 the workspace holds ceil(nC / R)).  These tests ask the library for the
 largest workspace byte its kernels touch (rr_ssd_workspace_extent: the grids
 walked with the kernels' own workgroup decode and slot arithmetic) and check
-it against the size the library asks callers for (rr_ssd_workspace_bytes),
-for BASELINE config 4, ragged even chunk counts in pair mode, and the other
-modes' shapes.
+it against the size the library asks callers for (rr_ssd_workspace_bytes; what
+the backward runs against rr_ssd_bwd_workspace_bytes), for BASELINE config 4,
+ragged even chunk counts in pair mode, the other modes' shapes, and a sweep over
+heads and chunks for the walks.
 """
 import pytest
 
@@ -21,11 +23,11 @@ ALIGN = 256   # every workspace part starts 256-byte aligned
 
 SHAPES = [
     # (B, L, H, Dh, N) at seg 32, bf16, a per-head A (the chunked kernels)
-    (8, 4096, 80, 64, 128),    # pair mode (nC 128)
+    (8, 4096, 80, 64, 128),    # walks both ways (pass 1's size: pair mode, nC 128)
     (4, 64, 80, 64, 128),      # pair mode, nC 2
-    (4, 192, 80, 64, 64),      # pair mode, nC 6
+    (4, 192, 80, 64, 64),      # walks (pass 1's size: pair mode, nC 6)
     (1, 320, 320, 32, 128),    # pair mode, nC 10, Dh 32
-    (5, 1088, 64, 64, 64),     # pair mode, nC 34
+    (5, 1088, 64, 64, 64),     # walks (pass 1's size: pair mode, nC 34)
     (4, 160, 80, 64, 128),     # nC 5 (odd): per-chunk adjoints from the scan
     (2, 1056, 4, 64, 64),      # nC 33, few heads: aggregate + adjoint-pass kernels
     (3, 512, 12, 64, 16),      # sum mode
@@ -35,6 +37,9 @@ SHAPES = [
     (2, 256, 6, 64, 128),      # Dh 64 N 128, short heads: pipelined
     (4, 512, 16, 128, 64),     # Dh 128, 1024 chunk workgroups: per-chunk mode
     (96, 512, 12, 64, 16),     # SSD c1 shape at B 96: per-chunk with the scan
+    (1, 2944, 12, 64, 64),     # walks, many segments
+    (2, 1504, 12, 128, 128),   # walks, an uneven last segment
+    (5, 128, 56, 64, 128),     # the backward walks in one segment
 ]
 
 
@@ -49,6 +54,32 @@ def test_kernels_stay_inside_the_workspace(B, L, H, Dh, N, pass_):
     if pass_ == 1:
         # every part of the backward workspace is used up to its alignment padding
         assert need - ext < ALIGN, (need, ext)
+
+
+@pytest.mark.parametrize("B,L,H,Dh,N", SHAPES)
+def test_the_backward_stays_inside_its_own_workspace(B, L, H, Dh, N):
+    need = int(_lib.load().rr_ssd_bwd_workspace_bytes(B, L, H, Dh, N, 32, 0, BF16))
+    ext = _lib.ssd_bwd_workspace_extent(B, L, H, Dh, N, 32, 0, BF16)
+    assert 0 <= ext <= need < ext + ALIGN, (ext, need)
+
+
+def test_walks_over_heads_and_chunks():
+    """Both walks' slots against what their callers allocate, and the backward's
+    size against rr_ssd_workspace_bytes(pass = 1), its documented bound."""
+    lib = _lib.load()
+    walks = 0
+    for Dh, N in [(32, 16), (32, 128), (64, 16), (64, 64), (64, 128), (128, 64), (128, 128)]:
+        for H in (1, 7, 12, 24, 50, 96, 300, 640, 1500):
+            for nC in (1, 2, 3, 5, 17, 23, 33, 47, 92, 128, 257):
+                a = (1, 32 * nC, H, Dh, N, 32, 0, BF16)
+                assert 0 <= _lib.ssd_workspace_extent(*a, 0) <= lib.rr_ssd_workspace_bytes(*a, 0), a
+                ext, need, most = (lib.rr_ssd_bwd_workspace_extent(*a), lib.rr_ssd_bwd_workspace_bytes(*a),
+                                   lib.rr_ssd_workspace_bytes(*a, 1))
+                assert need <= most, a
+                if ext >= 0:   # (Dh 128 with N 16 runs the fp32-MFMA path)
+                    assert ext <= need, a
+                walks += need != most
+    assert walks > 100
 
 
 def test_pair_mode_bound_detects_the_old_slot_spacing():
