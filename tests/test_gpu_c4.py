@@ -1,9 +1,9 @@
 """GPU parity at BASELINE config 4's full workload (MI355X only).
 
 ssd_scan forward + backward at B=8, L=4096, H=80, Dh=64, N=128, bf16 inputs,
-fp32 state, seg=32: 128 checkpoint intervals per head.  At this shape the
-forward runs the whole-head chunked kernel and the backward the per-head
-adjoint scan (B*H = 640 heads) followed by the column-owned chunk kernel.
+fp32 state, seg=32: 128 checkpoint intervals per head.  At this shape both
+passes walk a head's chunks (final_fwd.hip with checkpoints, walk_bwd.hip in two
+segments per head, the second one's adjoint map first).
 
 The inputs are drawn on the device (config 0's distributions) and rounded to
 bf16 there.  Every (batch, head) is an independent scan, so the float64 oracle

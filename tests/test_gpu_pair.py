@@ -1,15 +1,16 @@
 """The SSD backward in pair mode (MI355X only): many heads with a wide state
-(N >= 64, Dh <= 64, B*H >= 320, an even chunk count) run the per-head adjoint
-scan storing the adjoint leaving every second chunk only, and one workgroup
-per pair of chunks that carries the adjoint across the pair itself.
+(N >= 64, Dh <= 64, B*H >= 320, an even chunk count), where neither the direct
+mode (Dh 32: up to four chunks) nor the walking backward (Dh 64: from 1100
+chunks in all) takes them: the per-head adjoint scan stores the adjoint leaving
+every second chunk only, and one workgroup per pair of chunks carries the
+adjoint across the pair itself.
 
-Shapes: B=4 L=128 H=80 Dh=64 N=128 bf16 (320 heads, 4 chunks per head: two
-pairs), the smallest that takes the mode with more than one pair per head;
-the guard test also at L=64 (one pair per head).
+Shapes, B=4 H=80 bf16: L=192 Dh=32 N=128 and N=64 (320 heads, 6 chunks: three
+pairs), and L=64 Dh=64 N=128 (one pair).
   - Through the C ABI, with guard regions after the workspace (as large as the
     workspace itself) and after every output, filled with a byte pattern:
     nothing may be written past the sizes the library states
-    (rr_ssd_workspace_bytes, the output shapes).
+    (rr_ssd_bwd_workspace_bytes, the output shapes).
   - Through the C ABI: all batch rows of heads 0, 37 and 79 against the
     float64 oracle (oracle/recurrence_oracle.py, reference ssd.py:203-268),
     so dA of those heads is complete, compared per state n (dA_neg [H, N] as
@@ -33,13 +34,15 @@ import mlx_recurrence_amd as mr
 
 pytestmark = pytest.mark.gpu
 
-B, L, H, Dh, N, SEG = 4, 128, 80, 64, 128, 32
+B, H, SEG = 4, 80, 32
+SHAPES = [(192, 32, 128), (64, 64, 128)]   # L, Dh, N
+IDS = ["three_pairs", "one_pair"]
 HEADS = (0, 37, 79)
 PATTERN = 0x5A
 GUARD_OUT = 4096   # bytes past each output
 
 
-def _inputs(seed, L=L):
+def _inputs(seed, L, Dh, N):
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(seed)
     bf = torch.bfloat16
@@ -57,13 +60,13 @@ def _a64(n):
 
 
 def _assert_pair_mode(Bsz, seq, Hh, dh, n_st):
-    """The backward workspace the library asks for at this shape is the pair
-    mode's (per-chunk decays, dA partials and one adjoint per pair of chunks,
-    each part 256-byte aligned), which tells the mode apart from the
-    per-chunk pipelined one (an adjoint per chunk) and the direct one."""
+    """The workspace that the backward of this shape takes is the pair mode's
+    (per-chunk decays, dA partials and one adjoint per pair of chunks, each part
+    256-byte aligned), which tells the mode apart from the per-chunk pipelined
+    one (an adjoint per chunk), the direct one and the walk (no adjoints)."""
     nC = seq // 32
     want = 4 * (_a64(Bsz * Hh * nC) + _a64(Bsz * Hh * (nC // 2) * n_st) + _a64(Bsz * Hh * (nC // 2) * dh * n_st))
-    got = _lib.load().rr_ssd_workspace_bytes(Bsz, seq, Hh, dh, n_st, SEG, 0, _lib.DTYPE_CODE[torch.bfloat16], 1)
+    got = _lib.load().rr_ssd_bwd_workspace_bytes(Bsz, seq, Hh, dh, n_st, SEG, 0, _lib.DTYPE_CODE[torch.bfloat16])
     assert got == want, f"not the pair mode at B={Bsz} L={seq} H={Hh} Dh={dh} N={n_st}: {got} != {want}"
 
 
@@ -75,17 +78,17 @@ def _guarded(shape, dtype, guard_bytes):
     return buf[:n].view(dtype).view(shape), buf[n:]
 
 
-@pytest.mark.parametrize("L", [L, 64], ids=["two_pairs", "one_pair"])
-def test_pair_mode_writes_inside_its_buffers(L):
+@pytest.mark.parametrize("L,Dh,N", SHAPES, ids=IDS)
+def test_pair_mode_writes_inside_its_buffers(L, Dh, N):
     print(f"[case] ssd pair-mode guards B={B} L={L} H={H} Dh={Dh} N={N} bf16", flush=True)
     _assert_pair_mode(B, L, H, Dh, N)
-    u, delta, Bm, Cm, A, dy = _inputs(11, L)
+    u, delta, Bm, Cm, A, dy = _inputs(11, L, Dh, N)
     nC = L // _lib.chunk_len(L, SEG)
     y = torch.empty((B, L, H, Dh), dtype=torch.float32, device=u.device)
     ckpt = torch.empty((B, H, nC, Dh, N), dtype=torch.float32, device=u.device)
     wsf = _lib.ssd_workspace(B, L, H, Dh, N, SEG, 0, u.dtype, 0, u.device)
     _lib.ssd_fwd(u, delta, Bm, Cm, A, 0, None, SEG, y, ckpt, wsf)
-    nws = _lib.load().rr_ssd_workspace_bytes(B, L, H, Dh, N, SEG, 0, _lib.DTYPE_CODE[u.dtype], 1)
+    nws = _lib.load().rr_ssd_bwd_workspace_bytes(B, L, H, Dh, N, SEG, 0, _lib.DTYPE_CODE[u.dtype])
     assert nws > 0
     ws_buf = torch.full((2 * nws,), PATTERN, dtype=torch.uint8, device=u.device)
     ws, ws_guard = ws_buf[:nws], ws_buf[nws:]
@@ -100,14 +103,15 @@ def test_pair_mode_writes_inside_its_buffers(L):
         assert bool(torch.isfinite(o.float()).all()), f"{name} not finite"
 
 
-@pytest.fixture(scope="module")
-def pair_run():
+@pytest.fixture(scope="module", params=SHAPES, ids=IDS)
+def pair_run(request):
     """Forward + backward through the C ABI (so dA_neg comes per state n,
     [H, N], as the kernels form it); returns float64 CPU slices of the
     selected heads."""
+    L, Dh, N = request.param
     print(f"[case] ssd pair-mode parity B={B} L={L} H={H} Dh={Dh} N={N} bf16", flush=True)
     _assert_pair_mode(B, L, H, Dh, N)
-    u, delta, Bm, Cm, A, W = _inputs(12)
+    u, delta, Bm, Cm, A, W = _inputs(12, L, Dh, N)
     nC = L // _lib.chunk_len(L, SEG)
     y = torch.empty((B, L, H, Dh), dtype=torch.float32, device=u.device)
     ckpt = torch.empty((B, H, nC, Dh, N), dtype=torch.float32, device=u.device)
@@ -116,7 +120,7 @@ def pair_run():
     grads = [torch.empty_like(u), torch.empty_like(delta), torch.empty_like(Bm), torch.empty_like(Cm),
              torch.empty((H, N), dtype=torch.float32, device=u.device)]
     _lib.ssd_bwd(W, None, u, delta, Bm, Cm, A, 0, None, ckpt, SEG, *grads, None,
-                 _lib.ssd_workspace(B, L, H, Dh, N, SEG, 0, u.dtype, 1, u.device))
+                 _lib.ssd_bwd_workspace(B, L, H, Dh, N, SEG, 0, u.dtype, u.device))
     torch.cuda.synchronize()
     idx = torch.tensor(HEADS, device=u.device)
 
@@ -133,7 +137,7 @@ def test_pair_mode_parity(pair_run, j):
     r = pair_run
     sl = (slice(None), slice(None), slice(j, j + 1))
     u, dl, Bm, Cm = r["u"][sl], r["delta"][:, :, j:j + 1], r["Bm"][sl], r["Cm"][sl]
-    A = np.repeat(r["A"][j:j + 1, None], N, axis=1)
+    A = np.repeat(r["A"][j:j + 1, None], Bm.shape[-1], axis=1)
     y_o, fs_o = orc.ssd_forward(u, dl, Bm, Cm, A)
     du_o, dd_o, dB_o, dC_o, dA_o, _ = orc.ssd_backward(r["W"][sl], u, dl, Bm, Cm, A)
     errs = {
@@ -150,12 +154,12 @@ def test_pair_mode_parity(pair_run, j):
 
 
 def test_pair_mode_initial_state_and_final_cotangent():
-    """N = 64, three pairs per head (L = 192: more than the four chunks of the
-    direct mode), with an initial state and a loss on the final state: the
+    """Dh = 32, N = 64, three pairs per head (L = 192: more than the four chunks
+    of the direct mode), with an initial state and a loss on the final state: the
     entering state of the first chunk, the final-state cotangent through the
     adjoint scan and dh0 (through the public API; heads 0 and 79 against
     the oracle)."""
-    n_st, seq = 64, 192
+    Dh, n_st, seq = 32, 64, 192
     print(f"[case] ssd pair-mode h0 + dfinal B={B} L={seq} H={H} Dh={Dh} N={n_st} bf16", flush=True)
     _assert_pair_mode(B, seq, H, Dh, n_st)
     dev = torch.device("cuda:0")

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import mlx_recurrence_amd as mr
+from mlx_recurrence_amd import _lib
 from oracle import recurrence_oracle as orc
 from tests.gpu_util import TOL, check, rounded, to_dev
 
@@ -82,3 +83,50 @@ def test_growing_gates_after_the_last_cotangent():
         assert np.isfinite(want).all()
         check("grad_" + name, t.grad, want, TOL[BF16], rep)
     print(rep, flush=True)
+
+
+@pytest.mark.parametrize("kind,B,L,H,Dh,N", [("ssd", 5, 128, 56, 64, 128), ("ssd", 1, 2944, 12, 64, 64),
+                                             ("ssd", 1, 1504, 24, 128, 128), ("gla", 1, 1504, 24, 128, 128)])
+def test_walks_write_inside_their_buffers(kind, B, L, H, Dh, N):
+    """Forward and backward with workspaces of exactly the stated size and outputs
+    of exactly their shapes, each followed by a byte pattern that must stay: one
+    segment (no maps) and several."""
+    print(f"[case] walk guards {kind} B={B} L={L} H={H} Dh={Dh} N={N}", flush=True)
+    rng = np.random.default_rng(5)
+    guard, keep = 1 << 20, []
+
+    def buf(shape, dtype):
+        n = int(np.prod(shape)) * torch.empty(0, dtype=dtype).element_size()
+        b = torch.full((n + guard,), 0x5A, dtype=torch.uint8, device="cuda")
+        keep.append(b[n:])
+        return b[:n].view(dtype).view(shape)
+
+    def ws(n):
+        assert n % 4 == 0
+        return buf((n,), torch.uint8) if n else None
+
+    lib, dt = _lib.load(), _lib.DTYPE_CODE[BF16]
+    dy = to_dev(rng.standard_normal((B, L, H, Dh)), F32)
+    st, df = (to_dev(rng.standard_normal((B, H, Dh, N)), F32) for _ in range(2))
+    y, ckpt, dh0 = buf((B, L, H, Dh), F32), buf((B, H, L // 32, Dh, N), F32), buf((B, H, Dh, N), F32)
+    if kind == "ssd":
+        size = (B, L, H, Dh, N, 32, 0, dt)
+        need = lib.rr_ssd_bwd_workspace_bytes(*size)
+        assert need < lib.rr_ssd_workspace_bytes(*size, 1)   # the backward walks
+        xs = [to_dev(rng.standard_normal((B, L, H, Dh)), BF16), to_dev(np.abs(rng.standard_normal((B, L, H))) * 0.1, BF16),
+              to_dev(rng.standard_normal((B, L, H, N)), BF16), to_dev(rng.standard_normal((B, L, H, N)), BF16),
+              to_dev(-np.exp(rng.uniform(0, 2, H)), F32)]
+        grads = [buf(x.shape, BF16) for x in xs[:4]] + [buf((H, N), F32)]
+        _lib.ssd_fwd(*xs, 0, st, 32, y, ckpt, ws(lib.rr_ssd_workspace_bytes(*size, 0)))
+        _lib.ssd_bwd(dy, df, *xs, 0, st, ckpt, 32, *grads, dh0, ws(need))
+    else:
+        size = (B, L, H, Dh, 32, dt)
+        xs = [to_dev(rng.standard_normal((B, L, H, Dh)) / 8, BF16) for _ in range(3)]
+        xs.append(to_dev(1 / (1 + np.exp(-(rng.standard_normal((B, L, H)) + 2))), BF16))
+        grads = [buf(x.shape, BF16) for x in xs]
+        _lib.gla_fwd(*xs, st, 32, y, ckpt, ws(lib.rr_gla_workspace_bytes(*size, 0)))
+        _lib.gla_bwd(dy, df, *xs, st, ckpt, 32, *grads, dh0, ws(lib.rr_gla_workspace_bytes(*size, 1)))
+    torch.cuda.synchronize()
+    assert all(bool((g == 0x5A).all()) for g in keep)
+    for t in (y, ckpt, dh0, *grads):
+        assert bool(torch.isfinite(t.float()).all())
