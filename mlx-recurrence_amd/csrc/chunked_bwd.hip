@@ -982,7 +982,8 @@ int launch(const rr::ChunkArgs& p, int64_t B, hipStream_t s) {
     if (int rc = rr::chunked::launch_scan<DH, NS, GLA>(p, B, s, true)) return rc;
     hipLaunchKernelGGL((col_bwd_kernel<DH, NS, kPipe, GLA>), rr::chunked::chunk_grid(p), dim3(256), 0, s, p);
   } else if (p.mode == rr::chunked::kPair) {
-    if constexpr (GLA || DH > 64) {   // (the host picks it for SSD with Dh <= 64 only)
+    if constexpr (GLA || DH > 64 || (DH == 64 && NS == 64)) {   // (the host picks it for SSD with Dh <= 64 only;
+                                                                // Dh 64 N 64 walks there)
       return rr::fail(RR_EUNSUPPORTED, "chunked backward: no pair mode for this state");
     } else {
       if (p.R < 2 || p.nC % p.R != 0) return rr::fail(RR_EINVAL, "chunked backward: runs of R > 1 chunks dividing nC");

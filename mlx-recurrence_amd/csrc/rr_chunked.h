@@ -704,6 +704,12 @@ __global__ __launch_bounds__(256) void scan_kernel(ChunkArgs p) {
 // serial walks would leave most CUs idle (measured at B3 H12 nC16: 14.7 µs
 // against 9.5 µs), the aggregate kernel and the per-element state pass.
 constexpr int64_t kScanMinHeads = 320;
+// States whose per-head scans the host's modes reach: with that many heads wider
+// ones walk or run in the direct, resident and whole-head modes.
+template <int DH, int NS, bool GLA>
+constexpr bool kHasFwdScan = NS <= 32 || (DH == 128 && NS == 64 && !GLA);
+template <int DH, int NS>
+constexpr bool kHasBwdScan = !(DH == 64 && NS == 64);
 template <int DH, int NS, bool GLA>
 int launch_scan(const ChunkArgs& p, int64_t B, hipStream_t s, bool bwd) {
   const int kind = bwd ? 1 : 0;
@@ -714,9 +720,16 @@ int launch_scan(const ChunkArgs& p, int64_t B, hipStream_t s, bool bwd) {
     hipLaunchKernelGGL((pass_kernel<DH, NS, GLA>), dim3(DH * NS / 256, p.H, (unsigned)B), dim3(256), 0, s, p, kind);
     return check_launch(bwd ? "chunked backward adjoint pass" : "chunked forward state pass");
   }
-  if (bwd) hipLaunchKernelGGL((scan_kernel<DH, NS, GLA, true>), dim3(p.H, (unsigned)B), dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((scan_kernel<DH, NS, GLA, false>), dim3(p.H, (unsigned)B), dim3(256), 0, s, p);
-  return check_launch(bwd ? "chunked backward adjoint scan" : "chunked forward state scan");
+  if (bwd) {
+    if constexpr (kHasBwdScan<DH, NS>) {
+      hipLaunchKernelGGL((scan_kernel<DH, NS, GLA, true>), dim3(p.H, (unsigned)B), dim3(256), 0, s, p);
+      return check_launch("chunked backward adjoint scan");
+    }
+  } else if constexpr (kHasFwdScan<DH, NS, GLA>) {
+    hipLaunchKernelGGL((scan_kernel<DH, NS, GLA, false>), dim3(p.H, (unsigned)B), dim3(256), 0, s, p);
+    return check_launch("chunked forward state scan");
+  }
+  return fail(RR_EUNSUPPORTED, "chunked scan: no per-head scan for this state");
 }
 
 // ------------------------------------------------------------------ direct mode
