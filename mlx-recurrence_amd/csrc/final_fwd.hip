@@ -29,8 +29,8 @@
 // maps of segments 0 .. j - 1.
 //
 // W is formed once per chunk: its three nonzero 16x16 blocks are dealt to the
-// waves, which also take turns at the step scalars, a chunk ahead, so a chunk
-// has two barriers (LDS only: loads and stores stay in flight across them).
+// waves, a chunk ahead, and the last wave forms the step scalars two ahead, so a
+// chunk has two barriers (LDS only: loads and stores stay in flight across them).
 //
 // What bounds it: without checkpoints the instructions of a chunk (per wave
 // about 500 VALU, a third of them the state's three-term split, beside 50

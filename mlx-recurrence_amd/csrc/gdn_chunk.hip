@@ -450,7 +450,7 @@ __global__ __launch_bounds__(64) void gdn_state_kernel(const ChunkPack* __restri
     for (int r = 0; r < 4; ++r)
       S[ib][r] = h0 != nullptr ? h0[((int64_t)bh * kD + 16 * ib + 4 * g + r) * kD + j] : 0.f;
   const ChunkPack* pk = pack + (int64_t)bh * nC;
-  // one chunk; its fragments were loaded two chunks ahead
+  // one chunk; its fragments were loaded a chunk ahead
   auto step = [&](const Frags& f, int c) {
     // the state as B operands of its two 32-row k blocks
     u16x8_t sh[2], sl[2];

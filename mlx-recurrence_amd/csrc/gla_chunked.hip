@@ -2,8 +2,9 @@
 //
 // GLA (reference gla.py:78-100) is the chunked recurrence of rr_chunked.h with
 // u = v, B = k, C = q, d = j (value index), n = i (key index), per-step decay
-// g_t and input weight 1.  The forward runs the shared kernels of
-// rr_chunked.h; the backward is the column-owned kernel of chunked_bwd.hip.
+// g_t and input weight 1.  The forward runs the walk of final_fwd.hip or the
+// shared kernels of rr_chunked.h, the backward the walk of walk_bwd.hip or the
+// column-owned kernel of chunked_bwd.hip.
 // This file holds the host-side mode choice and workspace layout.
 #include "rr_chunked.h"
 
@@ -34,11 +35,13 @@ bool gla2_supported(int dtype, int64_t B, int64_t L, int64_t H, int64_t seg, int
 // kernels it saves).
 constexpr int64_t kGlaDirectMaxChunks = 4;
 constexpr int64_t kGlaDirectMaxWorkgroups = 3 * 256;
-// With enough heads to fill the GPU, whole heads: the forward always (the
-// state in registers from chunk to chunk: no aggregates, no state pass, no
-// checkpoint re-read; B96 L512 H12: 238 -> 175 us), the backward for short
-// heads (the adjoint carried likewise, no adjoint scan or workspace: 383 ->
-// 365 us; long heads serialise too many chunks per workgroup).
+// With enough heads to fill the GPU and no walk (one or two chunks, Dh 32, Dh 128
+// with up to 16), whole heads: the forward always (the state in registers from
+// chunk to chunk: no aggregates, no state pass, no checkpoint re-read), the
+// backward for short heads (the adjoint carried likewise, no adjoint scan or
+// workspace; long heads serialise too many chunks per workgroup).  Measured
+// against the pipelined kernels at B96 L512 H12 Dh 64, which both passes walk
+// now: 238 -> 175 and 383 -> 365 us.
 constexpr int64_t kGlaWholeMinHeads = 512;
 constexpr int64_t kGlaWholeBwdMaxChunks = 16;
 

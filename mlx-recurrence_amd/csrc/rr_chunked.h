@@ -185,9 +185,10 @@ __device__ __forceinline__ int state_off(int d, int n) {
 //   kPair   backward of the column-owned kernel with the per-head adjoint
 //           scan: one workgroup per run of R = 2 or 4 consecutive chunks;
 //           the scan stores the adjoint leaving every R-th chunk only, and
-//           the workgroup carries it across the run's inner boundaries.
-//   kWalk   forward only: a head's chunks walked by one workgroup per segment,
-//           waves that own rows of the state (final_fwd.hip).
+//           the workgroup carries it across the run's inner boundaries;
+//   kWalk   a head's chunks walked by one workgroup per segment: forward with
+//           waves that own rows of the state (final_fwd.hip), backward with the
+//           adjoint in registers (walk_bwd.hip).
 enum Mode { kWhole = 0, kPipe = 1, kDirect = 2, kSum = 3, kRes = 4, kPair = 5, kWalk = 6 };
 
 // Slot of map j (0 .. S - 2) of head bh among the segment maps of the walking
@@ -1553,9 +1554,9 @@ __global__ __launch_bounds__(256, (kFwdWgs<DH, NS, MODE, GLA>)) void fwd_kernel(
   // whole head with a 64-column state: the next chunk's loads are issued as
   // soon as this chunk's are staged (the first before the loop; the last
   // chunk repeats itself, so the count of loads in flight is the same every
-  // time).  Measured on one box: GLA B96 L512 H12 forward 161 -> 152 us; SSD
-  // config 4 (N = 128) 1110 -> 1127 us, so not there; N = 16 (SSD B96)
-  // 95 -> 108 us.
+  // time).  Measured: GLA B96 L512 H12 forward 161 -> 152 us; N = 128 (SSD B8
+  // L4096 H80) 1110 -> 1127 us, so not there (both walk now, see
+  // walk_preferred); N = 16 (SSD B96) 95 -> 108 us.
   constexpr bool PREF = MODE == kWhole && NS == 64;
   if constexpr (PREF) issue(cbeg, tid);
   for (int c = cbeg; c < cend; ++c) {

@@ -51,10 +51,12 @@ struct ChunkArgs {
   int mode;                // rr::chunked::Mode (rr_chunked.h)
 };
 
-// Mode of the SSD chunked kernels for pass 0 (forward) or 1 (backward), B*H
-// heads of nC chunks of a Dh x N state: a whole head per workgroup for the
-// forward when the heads alone fill the GPU (and for either pass when a 1-D
-// per-chunk grid would exceed 2^31 workgroups); else one workgroup per chunk,
+// Mode of the SSD chunked kernels for pass 0 (forward) or 1 (backward; where it
+// does not walk, see walk_bwd_preferred), B*H heads of nC chunks of a Dh x N
+// state: the walk of a head's chunks for the forward where walk_preferred says
+// so; a whole head per workgroup for the forward when the heads alone fill the
+// GPU (and for either pass when a 1-D per-chunk grid would exceed 2^31
+// workgroups); the resident forward for short heads; else one workgroup per chunk,
 // with the entering states formed directly (nC <= 4 with Dh * N <= 64 * 64;
 // nC <= 16 with Dh 128, N 64 and at most 768 chunk workgroups), from the chunk
 // aggregates (nC <= 16, N <= 32) or by the pipelined aggregate and state-pass
@@ -84,14 +86,14 @@ int ssd2_bwd(const ChunkArgs& p, int64_t B, hipStream_t s);
 // ------------------------------------------------------------------ GLA
 // True when the chunked GLA kernels cover this call (pass 0 forward, 1
 // backward): bf16 inputs, checkpoint interval 32, Dh in {32, 64, 128}, and a
-// 1-D grid of one workgroup per
-// chunk below 2^31 (direct or pipelined modes; whole heads run with
-// B * H >= 512: the forward always, the backward up to 16 chunks).
+// 1-D grid of one workgroup per chunk below 2^31 (direct or pipelined modes;
+// where neither pass walks, whole heads run with B * H >= 512: the forward
+// always, the backward up to 16 chunks).
 bool gla2_supported(int dtype, int64_t B, int64_t L, int64_t H, int64_t seg, int64_t Dh, int pass);
 int gla2_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass);
 // Workspace of the pipelined mode: chunk decays [B,H,nC] (both passes) and
-// the backward chunk adjoints [B,H,nC,Dh,Dh] (pass 1); none in the direct and
-// whole-head modes.
+// the backward chunk adjoints [B,H,nC,Dh,Dh] (pass 1); of the walks their
+// segment maps; none in the direct and whole-head modes.
 size_t gla2_ws_bytes(int64_t B, int64_t H, int64_t nC, int64_t Dh, int pass);
 void gla2_carve_ws(ChunkArgs& a, void* ws, int64_t B, int pass);
 int gla2_fwd(const ChunkArgs& p, int64_t B, hipStream_t s);

@@ -865,10 +865,10 @@ bool wide_direct(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N) {
 int chunked_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N, int pass) {
   const int64_t grid = nC * ((B * H + chunked::kXcds - 1) / chunked::kXcds * chunked::kXcds);
   if (grid >= ((int64_t)1 << 31)) return chunked::kWhole;   // beyond a 1-D per-chunk grid
-  // Enough heads to fill the GPU: the forward runs whole heads; the backward
-  // stays per chunk (measured on MI355X, fwd / bwd µs, whole-head vs per chunk:
-  // B96 L512 H12 Dh64 N16 137 / 414 vs 194 / 357 (sum mode); B8 L4096 H80
-  // Dh64 N128 2308 / 7457 vs 4025 / 4873 (pipelined)).
+  // Enough heads to fill the GPU: the forward runs whole heads where it does not
+  // walk; the backward stays per chunk (measured on MI355X, fwd / bwd µs,
+  // whole-head vs per chunk: B96 L512 H12 Dh64 N16 137 / 414 vs 194 / 357 (sum
+  // mode)).
   if (pass == 0 && walk_preferred(B * H, nC, Dh, N, false)) return chunked::kWalk;
   if (B * H >= 512 && pass == 0) return chunked::kWhole;
   if (wide_direct(B, H, nC, Dh, N)) return chunked::kDirect;
@@ -883,10 +883,11 @@ int chunked_mode(int64_t B, int64_t H, int64_t nC, int64_t Dh, int64_t N, int pa
   if (nC <= chunked::kDirectMaxChunks && N <= 32 && B * H * nC <= kDirectMaxWorkgroups) return chunked::kSum;
   if (nC <= kDirectMaxChunksWide && Dh * N <= chunked::kDirectMaxState) return chunked::kDirect;
   // Wide states (the column-owned backward) with the per-head adjoint scan:
-  // a workgroup per pair of chunks, half the adjoints through memory
-  // (measured at config 4: runs of 2 3.98 ms against 4.45 ms per chunk; runs
-  // of 4 3.92 ms, but the carried adjoint's rounding then reaches 8e-6 of dA
-  // where pairs keep 6e-6, so pairs)
+  // a workgroup per pair of chunks, half the adjoints through memory.  Reached
+  // with Dh 32, and with Dh 64 N 128 at two chunks: the rest walks, the shape
+  // this was measured at (B8 L4096 H80 Dh64 N128) among it: runs of 2 3.98 ms
+  // against 4.45 ms per chunk; runs of 4 3.92 ms, but the carried adjoint's
+  // rounding then reaches 8e-6 of dA where pairs keep 6e-6, so pairs
   if (pass == 1 && N >= 64 && Dh <= 64 && nC % 2 == 0 && B * H >= chunked::kScanMinHeads)
     return chunked::kPair;
   return chunked::kPipe;
