@@ -144,3 +144,25 @@ def test_few_short_heads_of_dh_32_run_the_direct_kernel():
 
     assert fwd(24, 4) == fwd(64, 4) == 0 and fwd(72, 4) > 72 * 32 * 128 * 4
     assert 0 < fwd(48, 5) < 4096 and fwd(56, 5) > 56 * 32 * 128 * 4
+
+
+def test_states_without_a_per_head_scan_never_take_it():
+    """From 320 heads the pipelined and pair modes run per-head scans, which are
+    not built for the states that walk there (or run direct, resident or whole
+    heads): their workspace is never that of those modes."""
+    lib = _lib.load()
+
+    def al(n):
+        return (n + 63) // 64 * 64 * 4
+
+    for H in [*range(320, 560), 640, 767, 768, 1024, 4099, 65535]:
+        for nC in [*range(1, 36), 64, 129]:
+            for Dh, N in [(32, 64), (64, 64), (32, 128), (64, 128), (128, 128)]:
+                assert lib.rr_ssd_workspace_bytes(1, 32 * nC, H, Dh, N, 32, 0, BF16, 0) != al(H * nC), (H, nC, Dh, N)
+            for Dh in (64, 128):
+                assert lib.rr_gla_workspace_bytes(1, 32 * nC, H, Dh, 32, BF16, 0) != al(H * nC), (H, nC, Dh)
+            own = lib.rr_ssd_bwd_workspace_bytes(1, 32 * nC, H, 64, 64, 32, 0, BF16)
+            for runs in {nC, nC // 2}:
+                assert own != al(H * nC) + al(H * runs * 64) + al(H * runs * 64 * 64), (H, nC)
+            gla = lib.rr_gla_workspace_bytes(1, 32 * nC, H, 64, 32, BF16, 1)
+            assert gla != al(H * nC) + al(H * nC * 64 * 64), (H, nC)
