@@ -82,6 +82,7 @@ _SIGS = {
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGS)
+ABI_VERSION = 13   # RR_ABI_VERSION of the header these signatures are from
 
 _lib = None
 
@@ -97,6 +98,9 @@ def load() -> ctypes.CDLL:
             "`python mlx-recurrence_amd/build.py` (hipcc, gfx950)"
         )
     lib = ctypes.CDLL(os.fspath(LIB_PATH))
+    if lib.rr_abi_version() != ABI_VERSION:
+        raise RuntimeError(f"{LIB_PATH} has ABI version {lib.rr_abi_version()}, this package needs {ABI_VERSION}; "
+                           "rebuild it with `python mlx-recurrence_amd/build.py`")
     for name, (res, args) in _SIGS.items():
         fn = getattr(lib, name)
         fn.restype = res

@@ -34,7 +34,19 @@ def test_exports_every_declared_symbol(lib):
 
 
 def test_abi_version(lib):
-    assert lib.rr_abi_version() == 12
+    assert lib.rr_abi_version() == _lib.ABI_VERSION == 13
+
+
+def test_a_library_of_another_abi_is_refused(lib, monkeypatch):
+    class Older:
+        @staticmethod
+        def rr_abi_version():
+            return 12
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib.ctypes, "CDLL", lambda path: Older())
+    with pytest.raises(RuntimeError, match="ABI version 12, this package needs 13"):
+        _lib.load()
 
 
 @pytest.mark.parametrize("L,seg,T", [(512, 32, 32), (96, 16, 16), (128, 64, 32), (96, 48, 16),
