@@ -22,8 +22,8 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # (bench workload maker, config); the chunked SSD/GLA modes: direct (c1, c2),
-    # whole head (B96 forward), pipelined (B96 backward, c4-like N = 128 with the
-    # per-head adjoint scan); the tiled RG-LRU / rotLRU passes (config 3)
+    # whole head and pipelined with the per-head adjoint scan (SSD B96), walking
+    # both ways (GLA B96, c4-like N = 128); the tiled RG-LRU / rotLRU passes (config 3)
     ("ssd", dict(B=3, L=512, H=12, Dh=64, N=16, seg=32)),
     ("gla", dict(B=3, L=512, H=12, Dh=64, seg=32)),
     ("ssd", dict(B=96, L=512, H=12, Dh=64, N=16, seg=32)),

@@ -354,7 +354,8 @@ SSD_CASES = [
     (2, 320, 2, 32, 64, 32, BF16, "cfg", True, True, 32),    # pipelined (10 chunks)
     (1, 192, 3, 64, 128, 32, BF16, "cfg", False, True, 33),  # pipelined
     (1, 64, 512, 32, 64, 32, BF16, "cfg", True, True, 34),   # whole head
-    (2, 96, 256, 64, 128, 32, BF16, "cfg", True, True, 35),  # whole head, config 4's tile
+    (2, 96, 256, 64, 128, 32, BF16, "cfg", True, True, 35),  # whole-head forward, walking backward, config 4's tile
+    (1, 32, 512, 64, 64, 32, BF16, "cfg", True, True, 81),   # whole-head forward, direct backward
     # Dh = 128 (column-owned backward, two du row blocks per wave)
     (3, 512, 12, 128, 64, 32, BF16, "cfg", True, True, 40),   # the reference's production shape: wide direct mode
     # wide direct mode (Dh 128, N 64, short heads): block-owned sums over the
@@ -367,8 +368,10 @@ SSD_CASES = [
     (4, 512, 12, 128, 64, 32, BF16, "cfg", True, True, 79),   # 768 chunk workgroups: the wide direct mode's largest
     (5, 512, 12, 128, 64, 32, BF16, "cfg", False, True, 80),  # 960: pipelined
     (1, 160, 3, 128, 128, 32, BF16, "cfg", True, True, 41),   # N = 128, pipelined
-    (2, 192, 160, 128, 64, 32, BF16, "cfg", False, True, 42), # B*H >= 320: per-head adjoint scan
+    (2, 192, 160, 128, 64, 32, BF16, "cfg", False, True, 42), # resident forward, walking backward
     # pipelined with B*H >= 320: the per-head state / adjoint scan kernel
+    # (39: resident forward; pairs of chunks in the backward)
+    (2, 96, 160, 128, 64, 32, BF16, "cfg", False, True, 82),
     (1, 640, 320, 32, 16, 32, BF16, "cfg", True, True, 38),
     (2, 320, 160, 32, 64, 32, BF16, "cfg", True, True, 39),
     # VALU engine (fp32 / fp16 inputs, dense A_neg [H, N], T < 32) past one
@@ -518,7 +521,8 @@ GLA_CASES = [
     (1, 480, 2, 64, 32, BF16, "zeros", True, True, 33),     # direct mode, 15 chunks, zero gates
     (5, 512, 12, 64, 32, BF16, "cfg", False, True, 34),     # 960 workgroups: pipelined
     (4, 512, 12, 64, 32, BF16, "cfg", True, False, 35),     # 768 workgroups: direct, the largest
-    (1, 160, 512, 64, 32, BF16, "signed", True, True, 36),  # B*H >= 512: whole-head forward
+    (1, 160, 512, 64, 32, BF16, "signed", True, True, 36),  # walking forward and backward, one segment
+    (1, 32, 512, 64, 32, BF16, "signed", True, True, 46),   # B*H >= 512, one chunk: whole head
     (2, 64, 256, 32, 32, BF16, "zeros", True, True, 37),    # whole-head forward, Dh = 32
     (1, 32, 512, 128, 32, BF16, "cfg", True, True, 38),     # whole-head forward and backward, Dh = 128
     (1, 64, 512, 128, 32, BF16, "zeros", True, True, 40),   # whole head, Dh = 128, 2 chunks, zero gates

@@ -28,7 +28,8 @@ SHAPES = [
     (4, 192, 80, 64, 64),      # walks (pass 1's size: pair mode, nC 6)
     (1, 320, 320, 32, 128),    # pair mode, nC 10, Dh 32
     (5, 1088, 64, 64, 64),     # walks (pass 1's size: pair mode, nC 34)
-    (4, 160, 80, 64, 128),     # nC 5 (odd): per-chunk adjoints from the scan
+    (4, 160, 80, 64, 128),     # walks (pass 1's size: nC 5, per-chunk adjoints from the scan)
+    (4, 96, 80, 64, 128),      # nC 3 (odd): per-chunk adjoints from the scan
     (2, 1056, 4, 64, 64),      # nC 33, few heads: aggregate + adjoint-pass kernels
     (3, 512, 12, 64, 16),      # sum mode
     (3, 512, 12, 64, 64),      # per-chunk mode, wide state, few heads
