@@ -34,12 +34,12 @@
 //
 // What bounds it: without checkpoints the instructions of a chunk (per wave
 // about 500 VALU, a third of them the state's three-term split, beside 50
-// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 97 us,
-// 2.9 TB/s of the 0.31 GB it cannot do without (6.1 ms on the VALU engine,
+// MFMAs at N = 128) on two waves per SIMD; B4 L1000 H80 Dh64 N128 takes 95 us,
+// 3.2 TB/s of the 0.31 GB it cannot do without (6.1 ms on the VALU engine,
 // which forms and stores a state every 8 steps there; 132 us with W and the
 // scalars formed by every wave for itself).  Three waves per SIMD (168 VGPRs)
 // spill 18 and take 178 us.  With checkpoints the traffic: B8 L4096 H80 Dh64
-// N128 1168 us, 4.6 TB/s; B8 L2048 H12 GLA Dh128 448 -> 195 us.
+// N128 1114 us, 4.6 TB/s of the 5.1 GB counted; B8 L2048 H12 GLA Dh128 448 -> 195 us.
 #include "rr_chunked.h"
 #include "rr_frag.h"
 

@@ -37,10 +37,10 @@
 // What bounds it: per wave and chunk about 1300 VALU instructions (the splits of
 // h_in and of both copies of lam are a fifth) beside 127 MFMAs (Dh 64, N 128) on
 // two waves per SIMD, and the traffic of inputs, checkpoints and gradients.
-// SSD B8 L4096 H80 Dh64 N128: 1.74 + 0.23 ms, 4.0 TB/s of 6.9 GB (adjoint scan +
-// pair kernel 2.7 ms, 12.6 GB); GLA B8 L2048 H12 Dh128: 235 + 65 us (348 + 102 +
-// 156 us).  No register may spill: a spilled load waits for its data at once,
-// and a reload for every load in flight (1.88 ms with 4 spills).
+// SSD B8 L4096 H80 Dh64 N128: 1.60 + 0.19 ms, the walk 4.3 TB/s of 6.9 GB (adjoint
+// scan + pair kernel 2.7 ms, 12.6 GB); GLA B8 L2048 H12 Dh128: 254 + 69 us profiled
+// (348 + 102 + 156 us).  No register may spill: a spilled load waits for its data at
+// once, and a reload for every load in flight (8 % more with 4 spills).
 #include "rr_chunked.h"
 #include "rr_frag.h"
 
