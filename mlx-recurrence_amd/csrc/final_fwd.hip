@@ -89,6 +89,8 @@ __device__ __forceinline__ void split3(const float (&x)[8], u16x8_t& hi, u16x8_t
 // LDS images of one chunk.  16-byte units of a row are permuted by row (xor)
 // so that both the row fragments (16 rows, one unit) and the transposing reads
 // (4 rows x 4 units) of a 16-lane group hit distinct banks.
+// (B and C: the images of rr_frag.h, written out here; through its helpers the
+// kernel measured 0 to 1 % slower.)
 template <int NSP>
 __device__ __forceinline__ int swz_n(int row) {
   return NSP == 128 ? ((row & 3) << 2) | ((row >> 2) & 3)
